@@ -75,386 +75,167 @@ enum GemmOut : uint32_t {
   GO_TAG = 2,    // T[b][o] = tag(gen[b], scale[b] * y)  (tagged logits)
 };
 
-// Complete binary tree over 16 values in index order.
-__device__ __forceinline__ f4v tree16(const f4v* a) {
-  f4v p[8], q[4];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) p[k] = a[2 * k] + a[2 * k + 1];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) q[k] = p[2 * k] + p[2 * k + 1];
-  return (q[0] + q[1]) + (q[2] + q[3]);
+// 16 bytes at a byte offset from a wave-uniform base.
+__device__ __forceinline__ float4 ldg4_at(const float* base, uint32_t byte_off) {
+  const v4f x = *(const AS_GLOBAL v4f*)((const AS_GLOBAL char*)(uintptr_t)base + byte_off);
+  return make_float4(x.x, x.y, x.z, x.w);
 }
 
-// Chunks of operands in flight through LDS, and the LDS a launch needs.
-// Four-tile tasks take a CU's LDS alone; smaller ones fit two workgroups
-// per CU with three stages.
-__host__ __device__ constexpr uint32_t gemm_stages(uint32_t tn) { return tn == 4 ? 4 : 3; }
-__host__ __device__ constexpr uint32_t gemm_lds_bytes(uint32_t tn) {
-  return gemm_stages(tn) * (4 + tn) * PANEL_TILE * 4;
+// The order of a launch's tasks, rows (row groups) x cols (column groups):
+// the dispatcher deals workgroups to the XCDs in turn, so workgroup b runs
+// task b / NXCD of a contiguous run of XCD b % NXCD, and the runs go through
+// bands of `band` column groups, row group by row group. What an XCD has in
+// flight is then a block of a few row groups by a band: a weight tile is
+// fetched into its L2 once per band, not once per column group (8B shape,
+// 28672 x 4096 by 500 rows: 1,368 us with the rows fastest, 1,013 so).
+struct TaskXY {
+  uint32_t x, y;
+};
+__device__ __forceinline__ TaskXY gemm_task(uint32_t b, uint32_t n, uint32_t rows, uint32_t cols,
+                                            uint32_t band) {
+  const uint32_t k = b % NXCD, t = k * (n / NXCD) + min(k, n % NXCD) + b / NXCD;
+  const uint32_t c0 = t / (rows * band) * band, w = min(band, cols - c0), r = t - rows * c0;
+  return {r / w, c0 + r % w};
 }
-constexpr uint32_t GEMM_WAVES = 8;
 
-// Y[b][o] = W[o] . X[b] for o < M, b < B, K columns. A task (x, y) covers
-// row tiles 4x .. 4x+3 and column tiles cbase + y*TN .. cbase + y*TN+TN-1.
-// Eight waves, two per SIMD, so one wave's MFMAs run while the other waits
-// for its operands: wave w owns row tile 4x + w%4 and column tiles
-// (w/4)*TN/2 .. of the task (TN = 1: the waves w < 4 only), all 16
-// segments of each of its outputs in its own accumulators, reduced with
-// tree16 at the end. A chunk's operands (the four row tiles and the TN
-// column tiles, 4 KB each) are copied into LDS by the waves together (16
-// bytes per lane straight from memory into LDS), gemm_stages(TN) - 1 chunks
-// ahead of their use, so each tile is read from memory once per workgroup.
-// The kernel is persistent: workgroup k takes tasks k, k + gridDim.x, ...,
-// and the copies run ahead across task boundaries. PARTIAL: K may end
-// inside a chunk.
-template <int TN, uint32_t OUT, bool PARTIAL>
-__global__ __launch_bounds__(512) void k_gemm(const float* __restrict__ Wp, uint32_t M, uint32_t K,
-                                              const float* __restrict__ Xp, uint32_t B,
-                                              float* __restrict__ Y, uint32_t ldy,
-                                              const float* __restrict__ scale,
-                                              const uint32_t* __restrict__ gen, uint32_t cbase,
-                                              uint32_t ncols, float* __restrict__ P) {
-  extern __shared__ float4 gsm[];  // [stages][4 + TN tiles][4 quarters][64 lanes]
-  constexpr uint32_t GEMM_STAGES = gemm_stages(TN);
-  constexpr uint32_t NT = 4 + TN;                    // tiles per stage
-  constexpr uint32_t WN = TN >= 2 ? TN / 2 : 1;      // column tiles per wave
-  constexpr uint32_t NQ = 4 * NT;                    // 1 KB copies per stage
-  // The wave index is uniform: scalar registers and branches for it.
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-  const uint32_t rt = wave % 4, half = wave / 4;
-  const bool mfma_wave = TN >= 2 || half == 0;
-  const uint32_t nld = (NQ - wave + GEMM_WAVES - 1) / GEMM_WAVES;  // this wave's copies per stage
-  const uint32_t gdx = gridDim.x;  // kept in a register (a reload would wait for every LDS read)
+// Y[b][o] = W[o] . X[b] for o < M, b < B, K columns. A task is TR row tiles
+// by TC column tiles; its four waves take a quarter of the segments each
+// (wave q: segments 4q .. 4q+3, quarter q of every panel tile, 1 KB
+// contiguous), so every operand byte is used by one wave only: it goes from
+// memory straight into that wave's registers, D chunks ahead of its use, and
+// the main loop has neither LDS nor barriers. Each wave forms its quarter's
+// subtree of tree16, ((s_4q + s_4q+1) + (s_4q+2 + s_4q+3)); the four meet in
+// LDS as (t_0 + t_1) + (t_2 + t_3) -- the complete tree over the 16 segments
+// -- and the output is written from there.
+//
+// Bound: the matrix cores for wide batches (two 4x2 workgroups per CU, one
+// wave of each per SIMD), memory for narrow ones. Measured against the
+// operands shared through LDS (one workgroup of eight waves, a barrier per
+// chunk), us before -> now: 3072 x 576 by 2048 rows 86 -> 75 (97 TFLOP/s),
+// 576 x 1536 by 2048 59 -> 38, 576 x 1536 by 301 35 -> 9.2, 28672 x 4096 by
+// 500 1,338 -> 1,013 (116 TFLOP/s), 128256 x 4096 by 1 row 1,042 -> 342
+// (6.1 TB/s of weights). Workgroups that take several tasks and load ahead
+// across them measured the same or slower.
+constexpr uint32_t GEMM_BAND = 32;  // column tiles of a band
+__host__ __device__ constexpr int gemm_depth(int tr, int tc) { return tr * tc >= 8 ? 2 : tr * tc >= 4 ? 3 : 4; }
+template <int TR, int TC, uint32_t OUT, bool PARTIAL>
+__global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, uint32_t M, uint32_t K,
+                                                 const float* __restrict__ Xp, uint32_t B,
+                                                 float* __restrict__ Y, uint32_t ldy,
+                                                 const float* __restrict__ scale,
+                                                 const uint32_t* __restrict__ gen,
+                                                 float* __restrict__ P) {
+  constexpr int D = gemm_depth(TR, TC), NT = TR * TC;
+  __shared__ float4 sub[4 * NT * WAVE];  // [quarter][tile][lane]
+  // The wave index is uniform: scalar registers for it and the tile bases.
+  const uint32_t q = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const uint32_t nch = panel_chunks(K), nrt = (M + 15) / 16, nct = (B + 15) / 16;
-  const uint32_t nrg = (nrt + 3) / 4, ngy = (ncols + TN - 1) / TN, ntask = nrg * ngy;
-  const uint32_t mine = blockIdx.x < ntask ? (ntask - blockIdx.x + gdx - 1) / gdx : 0;
-  const uint32_t total = mine * nch;  // chunks of this workgroup's tasks, in order
-  const uint32_t lds0 = (uint32_t)(uintptr_t)gsm;
-  // The copies run ahead of the MFMAs through the workgroup's chunks in
-  // order: chunk ci of task ct is next. A wave's copies of a stage are
-  // entries wave, wave + 8, ... of the stage's (tile, quarter) list; cb[j]
-  // is the tile of its copy j in task ct (tiles past the last one load a
-  // real tile, never used, so a wave issues the same number of copies for
-  // every chunk). Only a new task divides.
-  constexpr uint32_t MAXJ = (NQ + GEMM_WAVES - 1) / GEMM_WAVES;
-  uint32_t ct = blockIdx.x, ci = 0;
-  const float* cb[MAXJ];
-  auto set_task = [&]() {
-    const uint32_t x = ct % nrg, C0 = cbase + (ct / nrg) * TN;
+  const TaskXY task = gemm_task(blockIdx.x, gridDim.x, (nrt + TR - 1) / TR, (nct + TC - 1) / TC, GEMM_BAND / TC);
+  // Tiles past the last one load a real tile, never used.
+  const float *wa[TR], *xb[TC];
 #pragma unroll
-    for (uint32_t j = 0; j < MAXJ; ++j) {
-      const uint32_t tile = (wave + GEMM_WAVES * j) / 4;
-      cb[j] = tile < 4 ? Wp + (size_t)min(4 * x + tile, nrt - 1) * nch * PANEL_TILE
-                       : Xp + (size_t)min(C0 + tile - 4, nct - 1) * nch * PANEL_TILE;
-    }
+  for (int r = 0; r < TR; ++r)
+    wa[r] = Wp + (size_t)min(TR * task.x + r, nrt - 1) * nch * PANEL_TILE + q * 256;
+#pragma unroll
+  for (int c = 0; c < TC; ++c)
+    xb[c] = Xp + (size_t)min(TC * task.y + c, nct - 1) * nch * PANEL_TILE + q * 256;
+  f4v acc[TR][TC][4];
+#pragma unroll
+  for (int r = 0; r < TR; ++r)
+#pragma unroll
+    for (int c = 0; c < TC; ++c)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[r][c][u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 a[D][TR], b[D][TC];
+  const uint32_t last = (nch - 1) * (PANEL_TILE * 4) + lane * 16;
+  uint32_t off = lane * 16;
+  auto load = [&](int d) {  // the next chunk (past the last one: that one again, never used)
+#pragma unroll
+    for (int r = 0; r < TR; ++r) a[d][r] = ldg4_at(wa[r], off);
+#pragma unroll
+    for (int c = 0; c < TC; ++c) b[d][c] = ldg4_at(xb[c], off);
+    off = min(off + PANEL_TILE * 4, last);
   };
-  set_task();
-  // The next chunk into stage st.
-  auto issue = [&](uint32_t st) {
-    const uint32_t sb = lds0 + st * NT * PANEL_TILE * 4;
+  auto mfma = [&](int d, int u) {
 #pragma unroll
-    for (uint32_t j = 0; j < MAXJ; ++j) {
-      const uint32_t f = wave + GEMM_WAVES * j;
-      if (f < NQ) dma16(cb[j] + (size_t)ci * PANEL_TILE + (f % 4) * 256 + lane * 4, sb + f * 1024);
-    }
-    if (++ci == nch) {
-      ci = 0;
-      ct += gdx;
-      set_task();
-    }
+    for (int r = 0; r < TR; ++r)
+#pragma unroll
+      for (int c = 0; c < TC; ++c)
+        acc[r][c][u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[d][r].x)[u], (&b[d][c].x)[u],
+                                                            acc[r][c][u], 0, 0, 0);
   };
-  for (uint32_t g = 0; g + 1 < GEMM_STAGES && g < total; ++g) issue(g);
-  for (uint32_t k = 0; k < mine; ++k) {
-    f4v acc[WN][16];
 #pragma unroll
-    for (int t = 0; t < (int)WN; ++t)
+  for (int d = 0; d < D; ++d) load(d);
+  const uint32_t nfull = K / 64;
+  uint32_t i = 0;
+  for (; i + D <= nfull; i += D) {
 #pragma unroll
-      for (int s = 0; s < 16; ++s) acc[t][s] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-    // Chunk i of this task from its stage, once it has landed: chunk g has
-    // landed once at most the later chunks' copies are in flight; the
-    // barrier makes that true of every wave, and every wave is then done
-    // with chunk g - 1's stage, which the next request overwrites.
-    auto operands = [&](uint32_t i, float4 (&a)[4], float4 (&b)[WN][4]) {
-      const uint32_t g = k * nch + i;
-      stage_wait(min(GEMM_STAGES - 2, total - 1 - g) * nld);
-      __syncthreads();
-      if (g + GEMM_STAGES - 1 < total) issue((g + GEMM_STAGES - 1) % GEMM_STAGES);
-      const float4* sa = gsm + (g % GEMM_STAGES) * NT * 256;
+    for (int d = 0; d < D; ++d) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) a[q] = sa[(rt * 4 + q) * 64 + lane];
-#pragma unroll
-      for (int t = 0; t < (int)WN; ++t)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) b[t][q] = sa[((4 + half * WN + t) * 4 + q) * 64 + lane];
-    };
-    const uint32_t nfull = K / 64;
-    for (uint32_t i = 0; i < nfull; ++i) {
-      float4 a[4], b[WN][4];
-      operands(i, a, b);
-      if (!mfma_wave) continue;
-#pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        const float av = (&a[s / 4].x)[s % 4];
-#pragma unroll
-        for (int t = 0; t < (int)WN; ++t)
-          acc[t][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, (&b[t][s / 4].x)[s % 4], acc[t][s],
-                                                           0, 0, 0);
-      }
+      for (int u = 0; u < 4; ++u) mfma(d, u);
+      load(d);
     }
-    if (PARTIAL && nfull < nch) {
+  }
+#pragma unroll
+  for (int d = 0; d < D; ++d) {
+    if (i + d < nfull) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) mfma(d, u);
+    } else if (PARTIAL && i + d < nch) {
       // A last, partial chunk: the segments past K are left alone (their
       // zero padding would still turn a -0 sum into +0).
-      float4 a[4], b[WN][4];
-      operands(nfull, a, b);
-      const uint32_t ns = (K - 64 * nfull) / 4;
 #pragma unroll
-      for (int s = 0; s < 16; ++s) {
-        if ((uint32_t)s < ns && mfma_wave) {
-          const float av = (&a[s / 4].x)[s % 4];
-#pragma unroll
-          for (int t = 0; t < (int)WN; ++t)
-            acc[t][s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, (&b[t][s / 4].x)[s % 4],
-                                                             acc[t][s], 0, 0, 0);
-        }
-      }
-    }
-    // The task's outputs, one tile at a time.
-    const uint32_t tk = blockIdx.x + gdx * k;
-    const uint32_t T = 4 * (tk % nrg) + rt, C0 = cbase + (tk / nrg) * TN + half * WN;
-#pragma unroll
-    for (int t = 0; t < (int)WN; ++t) {
-      __builtin_amdgcn_sched_barrier(0);
-      const f4v r = tree16(acc[t]);
-      const uint32_t b = (C0 + t) * 16 + lane % 16;
-      const uint32_t o = T * 16 + 4 * (lane / 16);
-      if (!mfma_wave || T >= nrt || C0 + t >= cbase + ncols || b >= B) continue;
-      const size_t at = (size_t)b * ldy + o;
-      const uint32_t nchp = panel_chunks(M);  // the residual's panel: K = M
-      if (OUT != GO_TAG && o + 4 <= M && (at & 3) == 0) {
-        float4* y4 = reinterpret_cast<float4*>(Y + at);
-        float4 v = make_float4(r[0], r[1], r[2], r[3]);
-        if (OUT == GO_RESID) {
-          const float4 old = *y4;
-          v = make_float4(old.x + r[0], old.y + r[1], old.z + r[2], old.w + r[3]);
-          P[panel_at(b, o, nchp)] = v.x;
-          P[panel_at(b, o + 1, nchp)] = v.y;
-          P[panel_at(b, o + 2, nchp)] = v.z;
-          P[panel_at(b, o + 3, nchp)] = v.w;
-        }
-        *y4 = v;
-        continue;
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (o + j >= M) continue;
-        if (OUT == GO_PLAIN) {
-          Y[at + j] = r[j];
-        } else if (OUT == GO_RESID) {
-          const float v = Y[at + j] + r[j];
-          Y[at + j] = v;
-          P[panel_at(b, o + j, nchp)] = v;
-        } else {
-          const float v = scale[b] * r[j];
-          reinterpret_cast<u64*>(Y)[at + j] = ((u64)gen[b] << 32) | (u64)__float_as_uint(v);
-        }
-      }
+      for (int u = 0; u < 4; ++u)
+        if (64 * nfull + 4 * (4 * q + u) < K) mfma(d, u);
     }
   }
-}
-
-// The same product for narrow batches (at most four column tiles, B <= 64):
-// a task is one row tile with every column tile, so there are enough tasks
-// to stream the weights through every CU. Wave w computes column tile w % 4
-// over segments 8h .. 8h+7 (h = w / 4) and forms their subtree; the two
-// halves meet in LDS as (s0..s7) + (s8..s15) -- the same tree16.
-constexpr uint32_t GEMMN_STAGES = 3;  // two workgroups per CU
-__host__ __device__ constexpr uint32_t gemm_n_lds_bytes() {
-  return GEMMN_STAGES * 5 * PANEL_TILE * 4 + 4 * 64 * 16;
-}
-template <uint32_t OUT, bool PARTIAL>
-__global__ __launch_bounds__(512) void k_gemm_n(const float* __restrict__ Wp, uint32_t M,
-                                                uint32_t K, const float* __restrict__ Xp,
-                                                uint32_t B, float* __restrict__ Y, uint32_t ldy,
-                                                const float* __restrict__ scale,
-                                                const uint32_t* __restrict__ gen,
-                                                float* __restrict__ P) {
-  extern __shared__ float4 gsm[];  // [stages][5 tiles][4 quarters][64 lanes], then [4][64] f4v
-  constexpr uint32_t NT = 5, NQ = 4 * NT;
-  f4v* half_sum = reinterpret_cast<f4v*>(gsm + GEMMN_STAGES * NT * 256);
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-  const uint32_t gdx = gridDim.x;  // kept in a register (a reload would wait for every LDS read)
-  const uint32_t ct = wave % 4, h = wave / 4;
-  const uint32_t nch = panel_chunks(K), nrt = (M + 15) / 16, nct = (B + 15) / 16;
-  const uint32_t nld = (NQ - wave + GEMM_WAVES - 1) / GEMM_WAVES;
-  const uint32_t mine = blockIdx.x < nrt ? (nrt - blockIdx.x + gdx - 1) / gdx : 0;
-  const uint32_t total = mine * nch;
-  const uint32_t lds0 = (uint32_t)(uintptr_t)gsm;
-  auto issue = [&](uint32_t g, uint32_t st) {
-    const uint32_t T = blockIdx.x + gdx * (g / nch), i = g % nch;
-    const uint32_t sb = lds0 + st * NT * PANEL_TILE * 4;
 #pragma unroll
-    for (uint32_t f = wave; f < NQ; f += GEMM_WAVES) {
-      const uint32_t tile = f / 4, q = f % 4;
-      const float* src = tile == 0 ? Wp + ((size_t)T * nch + i) * PANEL_TILE
-                                   : Xp + ((size_t)min(tile - 1, nct - 1) * nch + i) * PANEL_TILE;
-      dma16(src + q * 256 + lane * 4, sb + f * 1024);
+  for (int r = 0; r < TR; ++r)
+#pragma unroll
+    for (int c = 0; c < TC; ++c) {
+      const f4v t = (acc[r][c][0] + acc[r][c][1]) + (acc[r][c][2] + acc[r][c][3]);
+      sub[(q * NT + r * TC + c) * WAVE + lane] = make_float4(t[0], t[1], t[2], t[3]);
     }
-  };
-  for (uint32_t g = 0; g + 1 < GEMMN_STAGES && g < total; ++g) issue(g, g);
-  for (uint32_t k = 0; k < mine; ++k) {
-    f4v acc[8];
+  __syncthreads();
 #pragma unroll
-    for (int s = 0; s < 8; ++s) acc[s] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t i = 0; i < nch; ++i) {
-      const uint32_t g = k * nch + i;
-      stage_wait(min(GEMMN_STAGES - 2, total - 1 - g) * nld);
-      __syncthreads();
-      if (g + GEMMN_STAGES - 1 < total)
-        issue(g + GEMMN_STAGES - 1, (g + GEMMN_STAGES - 1) % GEMMN_STAGES);
-      const float4* sa = gsm + (g % GEMMN_STAGES) * NT * 256;
-      float4 a[2], b[2];
+  for (int t0 = 0; t0 < NT; t0 += 4) {
+    const uint32_t t = t0 + q;  // this wave's tile
+    if (t >= NT) break;
+    const uint32_t T = TR * task.x + t / TC, bc = (TC * task.y + t % TC) * 16 + lane % 16;
+    const uint32_t o = T * 16 + 4 * (lane / 16);
+    if (T >= nrt || bc >= B) continue;
+    float4 s[4];
 #pragma unroll
-      for (int qq = 0; qq < 2; ++qq) {
-        a[qq] = sa[(2 * h + qq) * 64 + lane];
-        b[qq] = sa[((1 + ct) * 4 + 2 * h + qq) * 64 + lane];
+    for (uint32_t k = 0; k < 4; ++k) s[k] = sub[(k * NT + t) * WAVE + lane];
+    const float v[4] = {(s[0].x + s[1].x) + (s[2].x + s[3].x), (s[0].y + s[1].y) + (s[2].y + s[3].y),
+                        (s[0].z + s[1].z) + (s[2].z + s[3].z), (s[0].w + s[1].w) + (s[2].w + s[3].w)};
+    const size_t at = (size_t)bc * ldy + o;
+    const uint32_t nchp = panel_chunks(M);  // the residual's panel: K = M
+    if (OUT != GO_TAG && o + 4 <= M && (at & 3) == 0) {
+      float4* y4 = reinterpret_cast<float4*>(Y + at);
+      float4 w = make_float4(v[0], v[1], v[2], v[3]);
+      if (OUT == GO_RESID) {
+        const float4 old = *y4;
+        w = make_float4(old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]);
+        P[panel_at(bc, o, nchp)] = w.x;
+        P[panel_at(bc, o + 1, nchp)] = w.y;
+        P[panel_at(bc, o + 2, nchp)] = w.z;
+        P[panel_at(bc, o + 3, nchp)] = w.w;
       }
-#pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        // A last, partial chunk: the segments past K are left alone (their
-        // zero padding would still turn a -0 sum into +0).
-        if (PARTIAL && 64 * i + 4 * (8 * h + s) >= K) continue;
-        acc[s] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[s / 4].x)[s % 4], (&b[s / 4].x)[s % 4],
-                                                      acc[s], 0, 0, 0);
-      }
+      *y4 = w;
+      continue;
     }
-    // Subtree of this wave's eight segments; the upper half hands its own to
-    // the lower half through LDS.
-    f4v p4[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) p4[u] = acc[2 * u] + acc[2 * u + 1];
-    const f4v t8 = (p4[0] + p4[1]) + (p4[2] + p4[3]);
-    if (h == 1) half_sum[ct * 64 + lane] = t8;
-    __syncthreads();
-    const uint32_t T = blockIdx.x + gdx * k;
-    if (h == 0 && ct < nct) {
-      const f4v r = t8 + half_sum[ct * 64 + lane];
-      const uint32_t b = ct * 16 + lane % 16;
-      const uint32_t o = T * 16 + 4 * (lane / 16);
-      if (b < B) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (o + j >= M) continue;
-          const size_t at = (size_t)b * ldy + o + j;
-          if (OUT == GO_PLAIN) {
-            Y[at] = r[j];
-          } else if (OUT == GO_RESID) {
-            const float v = Y[at] + r[j];
-            Y[at] = v;
-            P[panel_at(b, o + j, panel_chunks(M))] = v;
-          } else {
-            const float v = scale[b] * r[j];
-            reinterpret_cast<u64*>(Y)[at] = ((u64)gen[b] << 32) | (u64)__float_as_uint(v);
-          }
-        }
-      }
-    }
-    // half_sum is rewritten by the next task only after this barrier.
-    __syncthreads();
-  }
-}
-
-// Narrow batches (B <= 64) with few row groups: the segments split four
-// ways. Quarter q of tree16 is ((s_4q + s_4q+1) + (s_4q+2 + s_4q+3)), a
-// subtree of its own, and it needs only quarter q of every chunk (one
-// contiguous 1 KB block per tile and chunk in the panel layout), so a task
-// is (pair of row tiles, quarter q, four column tiles): it reads a quarter
-// of the rows' weights and of four column tiles' panel, and writes its
-// subtree to plane q of Q ([4][B][M]); k_gemm_qcomb forms (t_0 + t_1) +
-// (t_2 + t_3), the same tree16, and applies OUT. With all four column tiles
-// of B <= 64 in one task, each weight quarter is read by one task only.
-// Eight waves: wave w owns row tile w % 2 and column tile w / 2. A chunk's
-// six 1 KB blocks (two row tiles, four column tiles) take one copy each
-// from waves 0..5; a stage holds GEMMQ_CPB chunks (one barrier per stage),
-// GEMMQ_STAGES - 1 stages ahead.
-constexpr uint32_t GEMMQ_CPB = 8, GEMMQ_STAGES = 3;
-__host__ __device__ constexpr uint32_t gemm_q_lds_bytes() {
-  return GEMMQ_STAGES * GEMMQ_CPB * 6 * 1024;
-}
-template <bool PARTIAL>
-__global__ __launch_bounds__(512) void k_gemm_q(const float* __restrict__ Wp, uint32_t M, uint32_t K,
-                                                const float* __restrict__ Xp, uint32_t B,
-                                                float* __restrict__ Q) {
-  extern __shared__ float4 gsm[];  // [stages][GEMMQ_CPB chunks][6 blocks][64 lanes]
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-  const uint32_t gdx = gridDim.x;  // kept in a register (a reload would wait for every LDS read)
-  const uint32_t rt = wave % 2, ct = wave / 2;
-  const uint32_t nch = panel_chunks(K), nrt = (M + 15) / 16, nct = (B + 15) / 16;
-  const uint32_t nsc = (nch + GEMMQ_CPB - 1) / GEMMQ_CPB;  // stages of chunks per task
-  const uint32_t nrg = (nrt + 1) / 2, ncg = (nct + 3) / 4, ntask = 4 * nrg * ncg;
-  const uint32_t mine = blockIdx.x < ntask ? (ntask - blockIdx.x + gdx - 1) / gdx : 0;
-  const uint32_t total = mine * nsc;
-  const uint32_t nld = wave < 6 ? GEMMQ_CPB : 0u;  // copies per stage
-  const uint32_t lds0 = (uint32_t)(uintptr_t)gsm;
-  // Task t = (x * 4 + q) * ncg + cg. Stage g's chunks into LDS stage st:
-  // block `wave` of each is row tile 2x + wave (waves 0, 1) or column tile
-  // 4cg + wave - 2, quarter q. Tiles and chunks past the last load a real
-  // one (never used), so every copying wave issues GEMMQ_CPB per stage.
-  auto issue = [&](uint32_t g, uint32_t st) {
-    const uint32_t t = blockIdx.x + gdx * (g / nsc), i0 = (g % nsc) * GEMMQ_CPB;
-    const uint32_t cg = t % ncg, xq = t / ncg, x = xq / 4, q = xq % 4;
-    if (wave >= 6) return;
-    const float* src = wave < 2 ? Wp + (size_t)min(2 * x + wave, nrt - 1) * nch * PANEL_TILE
-                                : Xp + (size_t)min(4 * cg + wave - 2, nct - 1) * nch * PANEL_TILE;
-#pragma unroll
-    for (uint32_t c = 0; c < GEMMQ_CPB; ++c)
-      dma16(src + (size_t)min(i0 + c, nch - 1) * PANEL_TILE + q * 256 + lane * 4,
-            lds0 + ((st * GEMMQ_CPB + c) * 6 + wave) * 1024);
-  };
-  for (uint32_t g = 0; g + 1 < GEMMQ_STAGES && g < total; ++g) issue(g, g);
-  for (uint32_t k = 0; k < mine; ++k) {
-    const uint32_t t = blockIdx.x + gdx * k;
-    const uint32_t cg = t % ncg, xq = t / ncg, x = xq / 4, q = xq % 4;
-    f4v acc[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) acc[u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-    for (uint32_t j = 0; j < nsc; ++j) {
-      const uint32_t g = k * nsc + j;
-      // Stage g has landed once at most the later stages' copies are in
-      // flight; after the barrier every wave is done with stage g - 1's
-      // LDS, which the next request overwrites.
-      stage_wait(min(GEMMQ_STAGES - 2, total - 1 - g) * nld);
-      __syncthreads();
-      if (g + GEMMQ_STAGES - 1 < total) issue(g + GEMMQ_STAGES - 1, (g + GEMMQ_STAGES - 1) % GEMMQ_STAGES);
-      const float4* sa = gsm + (g % GEMMQ_STAGES) * GEMMQ_CPB * 6 * 64;
-      float4 a[GEMMQ_CPB], b[GEMMQ_CPB];
-#pragma unroll
-      for (uint32_t c = 0; c < GEMMQ_CPB; ++c) {
-        a[c] = sa[(c * 6 + rt) * 64 + lane];
-        b[c] = sa[(c * 6 + 2 + ct) * 64 + lane];
-      }
-#pragma unroll
-      for (uint32_t c = 0; c < GEMMQ_CPB; ++c) {
-        const uint32_t i = j * GEMMQ_CPB + c;
-        if (i >= nch) break;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          // A last, partial chunk: the segments past K are left alone.
-          if (PARTIAL && 64 * i + 4 * (4 * q + u) >= K) continue;
-          acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&a[c].x)[u], (&b[c].x)[u], acc[u], 0, 0, 0);
-        }
-      }
-    }
-    const uint32_t T = 2 * x + rt, o = T * 16 + 4 * (lane / 16);
-    const f4v r = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-    const uint32_t bc = (4 * cg + ct) * 16 + lane % 16;
-    if (T < nrt && bc < B) {
-      float* dst = Q + ((size_t)q * B + bc) * M + o;
-      if (o + 4 <= M && (((size_t)q * B + bc) * M + o) % 4 == 0) {
-        *reinterpret_cast<float4*>(dst) = make_float4(r[0], r[1], r[2], r[3]);
+    for (int j = 0; j < 4; ++j) {
+      if (o + j >= M) continue;
+      if (OUT == GO_PLAIN) {
+        Y[at + j] = v[j];
+      } else if (OUT == GO_RESID) {
+        const float w = Y[at + j] + v[j];
+        Y[at + j] = w;
+        P[panel_at(bc, o + j, nchp)] = w;
       } else {
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj)
-          if (o + jj < M) dst[jj] = r[jj];
+        reinterpret_cast<u64*>(Y)[at + j] = ((u64)gen[bc] << 32) | (u64)__float_as_uint(scale[bc] * v[j]);
       }
     }
   }
@@ -474,56 +255,6 @@ __device__ __forceinline__ float rms_row_inv(const float* __restrict__ x, uint32
   }
   ss = wave_sum(ss);
   return 1.0f / sqrtf(ss / (float)n + eps);
-}
-
-// The residual output of k_gemm_q (x += tree16 of the four subtrees, and
-// its panel) for one row per workgroup, then the row's 1/rms (k_b_rms's
-// order) for the next matrix product's normalisation: one launch instead of
-// two.
-__global__ __launch_bounds__(256) void k_gemm_qcomb_rms(const float* __restrict__ Q, uint32_t M,
-                                                        uint32_t B, float* __restrict__ Y,
-                                                        uint32_t ldy, float* __restrict__ P,
-                                                        float eps, float* __restrict__ inv) {
-  const uint32_t b = blockIdx.x;
-  const size_t plane = (size_t)B * M;
-  for (uint32_t o = threadIdx.x; o < M; o += blockDim.x) {
-    const size_t e = (size_t)b * M + o;
-    const float r = (Q[e] + Q[plane + e]) + (Q[2 * plane + e] + Q[3 * plane + e]);
-    const size_t at = (size_t)b * ldy + o;
-    const float v = Y[at] + r;
-    Y[at] = v;
-    P[panel_at(b, o, panel_chunks(M))] = v;
-  }
-  // The row's new values, written by the whole workgroup, are visible to it
-  // after the barrier.
-  __syncthreads();
-  if (threadIdx.x < WAVE) {
-    const float r = rms_row_inv(Y + (size_t)b * ldy, M, eps, threadIdx.x);
-    if (threadIdx.x == 0) inv[b] = r;
-  }
-}
-
-// The four quarter subtrees of k_gemm_q into tree16 and the output: thread
-// (b, o) for o < M, b < B.
-template <uint32_t OUT>
-__global__ void k_gemm_qcomb(const float* __restrict__ Q, uint32_t M, uint32_t B,
-                             float* __restrict__ Y, uint32_t ldy, const float* __restrict__ scale,
-                             const uint32_t* __restrict__ gen, float* __restrict__ P) {
-  const uint32_t o = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
-  if (o >= M || b >= B) return;
-  const size_t plane = (size_t)B * M, e = (size_t)b * M + o;
-  const float r = (Q[e] + Q[plane + e]) + (Q[2 * plane + e] + Q[3 * plane + e]);
-  const size_t at = (size_t)b * ldy + o;
-  if (OUT == GO_PLAIN) {
-    Y[at] = r;
-  } else if (OUT == GO_RESID) {
-    const float v = Y[at] + r;
-    Y[at] = v;
-    P[panel_at(b, o, panel_chunks(M))] = v;
-  } else {
-    const float v = scale[b] * r;
-    reinterpret_cast<u64*>(Y)[at] = ((u64)gen[b] << 32) | (u64)__float_as_uint(v);
-  }
 }
 
 // ------------------------------------------------------------- rows
@@ -562,13 +293,11 @@ __global__ __launch_bounds__(256) void k_b_rms(const float* __restrict__ X, uint
 
 // QKV epilogue of the one-token path (phase_qkv) for pair i of head block
 // hb of batch row b: the product's rows r0 = hb * hd + i and r1 = r0 + half
-// (from Y, or combined from k_gemm_q's four subtree planes QS ([4][nb]
-// [qkv_rows]) as k_gemm_qcomb would), scaled by the row's 1/rms, biased,
-// and rotated (q and k heads) -- phase_qkv's expressions.
+// (from Y), scaled by the row's 1/rms, biased, and rotated (q and k heads)
+// -- phase_qkv's expressions.
 __device__ __forceinline__ float2 qkv_epi_pair(const Args& a, uint32_t l, uint32_t pos, uint32_t b,
                                                uint32_t hb, uint32_t i, const float* __restrict__ Y,
-                                               uint32_t ldy, const float* __restrict__ QS,
-                                               uint32_t nb, float iv) {
+                                               uint32_t ldy, float iv) {
   const Dims& d = a.d;
   const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
   float4 e = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
@@ -582,15 +311,7 @@ __device__ __forceinline__ float2 qkv_epi_pair(const Args& a, uint32_t l, uint32
     e.z = bias[r0];
     e.w = bias[r0 + d.half];
   }
-  float y0, y1;
-  if (QS) {
-    const size_t plane = (size_t)nb * d.qkv_rows, e0 = (size_t)b * d.qkv_rows + r0, e1 = e0 + d.half;
-    y0 = (QS[e0] + QS[plane + e0]) + (QS[2 * plane + e0] + QS[3 * plane + e0]);
-    y1 = (QS[e1] + QS[plane + e1]) + (QS[2 * plane + e1] + QS[3 * plane + e1]);
-  } else {
-    y0 = Y[(size_t)b * ldy + r0];
-    y1 = Y[(size_t)b * ldy + r1];
-  }
+  float y0 = Y[(size_t)b * ldy + r0], y1 = Y[(size_t)b * ldy + r1];
   y0 = y0 * iv + e.z;
   y1 = y1 * iv + e.w;
   float a0 = y0, a1 = y1;
@@ -616,8 +337,7 @@ __device__ __forceinline__ void qkv_epi_cache(const Dims& d, const BRow& r, uint
 // k, v into the row's cache at its position.
 __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict__ rows, uint32_t l,
                             const float* __restrict__ Y, uint32_t ldy, const float* __restrict__ inv,
-                            u64* __restrict__ qkvt, uint32_t ldq, const float* __restrict__ QS,
-                            uint32_t nb) {
+                            u64* __restrict__ qkvt, uint32_t ldq) {
   const Dims& d = ap->d;
   const uint32_t b = blockIdx.y;
   const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -625,7 +345,7 @@ __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict_
   const BRow r = rows[b];
   const uint32_t hb = p / d.half, i = p - hb * d.half;
   const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
-  const float2 v = qkv_epi_pair(*ap, l, r.pos, b, hb, i, Y, ldy, QS, nb, inv[b]);
+  const float2 v = qkv_epi_pair(*ap, l, r.pos, b, hb, i, Y, ldy, inv[b]);
   const u64 g = (u64)gen_of(d, r.tick, l, PH_QKV) << 32;
   qkvt[(size_t)b * ldq + r0] = g | __float_as_uint(v.x);
   qkvt[(size_t)b * ldq + r1] = g | __float_as_uint(v.y);
@@ -690,8 +410,7 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_b_attn_f(
     const Args* __restrict__ rargs, const BRow* __restrict__ rows,
     const uint32_t* __restrict__ items, uint32_t l, const float* __restrict__ Y, uint32_t ldy,
-    const float* __restrict__ QS, uint32_t nb, const float* __restrict__ inv,
-    uint32_t* __restrict__ cnt, float* __restrict__ attp) {
+    const float* __restrict__ inv, uint32_t* __restrict__ cnt, float* __restrict__ attp) {
   const uint32_t e = items[blockIdx.x], b = e >> 16, x = e & 0xffffu;
   const Args& a = rargs[b];
   const Lds s = lds_init_attn();
@@ -703,7 +422,7 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
     for (uint32_t u = threadIdx.x; u < (d.group + 2) * d.half; u += blockDim.x) {
       const uint32_t j = u / d.half, i = u - j * d.half;
       const uint32_t hb = j < d.group ? gg * d.group + j : (j == d.group ? d.nh + gg : d.nh + d.nkv + gg);
-      const float2 v = qkv_epi_pair(a, l, r.pos, b, hb, i, Y, ldy, QS, nb, iv);
+      const float2 v = qkv_epi_pair(a, l, r.pos, b, hb, i, Y, ldy, iv);
       float* dst = j < d.group ? qs + j * d.hd : (j == d.group ? kn : vn);
       lds_st(dst + i, v.x);
       lds_st(dst + i + d.half, v.y);

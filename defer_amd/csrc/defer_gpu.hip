@@ -805,38 +805,6 @@ extern "C" int defer_gpu_model_create(const defer_gpu_config* cfg, const float* 
 
   rc = apply_layout(m, std::min<uint32_t>(m->ncu, min_items));
   if (rc) return cleanup(rc);
-  {
-    const void* gk[] = {
-        (const void*)k_gemm<1, GO_PLAIN, false>, (const void*)k_gemm<1, GO_RESID, false>,
-        (const void*)k_gemm<1, GO_TAG, false>,   (const void*)k_gemm<2, GO_PLAIN, false>,
-        (const void*)k_gemm<2, GO_RESID, false>, (const void*)k_gemm<2, GO_TAG, false>,
-        (const void*)k_gemm<4, GO_PLAIN, false>, (const void*)k_gemm<4, GO_RESID, false>,
-        (const void*)k_gemm<4, GO_TAG, false>,   (const void*)k_gemm<1, GO_PLAIN, true>,
-        (const void*)k_gemm<1, GO_RESID, true>,  (const void*)k_gemm<1, GO_TAG, true>,
-        (const void*)k_gemm<2, GO_PLAIN, true>,  (const void*)k_gemm<2, GO_RESID, true>,
-        (const void*)k_gemm<2, GO_TAG, true>,    (const void*)k_gemm<4, GO_PLAIN, true>,
-        (const void*)k_gemm<4, GO_RESID, true>,  (const void*)k_gemm<4, GO_TAG, true>};
-    const int tn[] = {1, 1, 1, 2, 2, 2, 4, 4, 4, 1, 1, 1, 2, 2, 2, 4, 4, 4};
-    for (int i = 0; i < 18; ++i) {
-      e = hipFuncSetAttribute(gk[i], hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)gemm_lds_bytes(tn[i]));
-      if (e != hipSuccess)
-        return cleanup(fail(DEFER_GPU_E_HIP, "LDS attribute (GEMM): %s", hipGetErrorString(e)));
-    }
-    const void* gn[] = {(const void*)k_gemm_n<GO_PLAIN, false>, (const void*)k_gemm_n<GO_RESID, false>,
-                        (const void*)k_gemm_n<GO_TAG, false>,   (const void*)k_gemm_n<GO_PLAIN, true>,
-                        (const void*)k_gemm_n<GO_RESID, true>,  (const void*)k_gemm_n<GO_TAG, true>};
-    for (const void* kf : gn) {
-      e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_n_lds_bytes());
-      if (e != hipSuccess)
-        return cleanup(fail(DEFER_GPU_E_HIP, "LDS attribute (narrow GEMM): %s", hipGetErrorString(e)));
-    }
-    for (const void* kf : {(const void*)k_gemm_q<false>, (const void*)k_gemm_q<true>}) {
-      e = hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)gemm_q_lds_bytes());
-      if (e != hipSuccess)
-        return cleanup(fail(DEFER_GPU_E_HIP, "LDS attribute (quarter GEMM): %s", hipGetErrorString(e)));
-    }
-  }
   e = hipFuncSetAttribute((const void*)k_b_attn_tile, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)attn_tile_lds(MAX_GROUP));
   if (e != hipSuccess)
@@ -1799,7 +1767,6 @@ struct BatchWs {
   // the other GEMM inputs (attention output, activation, final-norm rows).
   float *X = nullptr, *Y = nullptr, *INV = nullptr, *XP = nullptr, *XQ = nullptr;
   float* LINV = nullptr;
-  float* QS = nullptr;  // quarter-split GEMM subtrees [4][B][M], B <= 64, M <= batch_ldy
   u64 *QKVT = nullptr, *PART = nullptr, *LOGT = nullptr, *VMAX = nullptr, *VARG = nullptr,
       *VSUM = nullptr, *VP = nullptr;
   BRow* drows = nullptr;
@@ -1815,7 +1782,7 @@ struct BatchWs {
 
 static void batch_ws_release(BatchWs* w) {
   if (!w) return;
-  void* ps[] = {w->X, w->Y, w->INV, w->XP, w->XQ, w->LINV, w->QS, w->QKVT, w->PART,
+  void* ps[] = {w->X, w->Y, w->INV, w->XP, w->XQ, w->LINV, w->QKVT, w->PART,
                 w->LOGT, w->VMAX, w->VARG, w->VSUM, w->VP, w->drows, w->rargs, w->largs, w->sel,
                 w->lgen, w->stick, w->swords, w->sout, w->items, w->tiles, w->CNT, w->sets, w->st};
   for (void* p : ps) (void)hipFree(p);
@@ -1842,7 +1809,6 @@ static int ensure_ws(defer_gpu_model* m, uint32_t rows, uint32_t lm) {
   const uint32_t kmax = std::max({d.h, d.q, d.ff});
   HIP_TRY(counted_malloc(&w.X, (size_t)R * d.h * sizeof(float)));
   HIP_TRY(counted_malloc(&w.Y, (size_t)R * batch_ldy(d) * sizeof(float)));
-  HIP_TRY(counted_malloc(&w.QS, (size_t)4 * std::min(R, 64u) * batch_ldy(d) * sizeof(float)));
   HIP_TRY(counted_malloc(&w.INV, (size_t)R * sizeof(float)));
   HIP_TRY(counted_malloc(&w.XP, panel_floats(R, d.h) * sizeof(float)));
   HIP_TRY(counted_malloc(&w.QKVT, (size_t)R * d.qkv_rows * sizeof(u64)));
@@ -1924,96 +1890,50 @@ static int ensure_panels(defer_gpu_model* m) {
   return DEFER_GPU_OK;
 }
 
-template <int TN, uint32_t OUT>
-static void launch_gemm_tn(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
-                           uint32_t B, float* Y, uint32_t ldy, const float* scale,
-                           const uint32_t* gen, uint32_t cbase, uint32_t ncols, uint32_t ncu,
-                           float* P) {
-  const uint32_t nrg = (M + 63) / 64, ntask = nrg * ((ncols + TN - 1) / TN);
-  // One workgroup per CU (two for smaller tasks, whose LDS and registers allow it).
-  const uint32_t grid = std::min(ntask, (TN == 4 ? 1 : 2) * ncu);
-  const uint32_t threads = GEMM_WAVES * WAVE;
-  if (K % 64 == 0)
-    k_gemm<TN, OUT, false><<<grid, threads, gemm_lds_bytes(TN), s>>>(Wp, M, K, Xp, B, Y, ldy, scale,
-                                                                      gen, cbase, ncols, P);
-  else
-    k_gemm<TN, OUT, true><<<grid, threads, gemm_lds_bytes(TN), s>>>(Wp, M, K, Xp, B, Y, ldy, scale,
-                                                                     gen, cbase, ncols, P);
+template <int TR, int TC, uint32_t OUT, bool PARTIAL = false>
+static void launch_gemm_tile(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
+                             uint32_t B, float* Y, uint32_t ldy, const float* scale,
+                             const uint32_t* gen, float* P) {
+  const uint32_t n = ((M + 16 * TR - 1) / (16 * TR)) * ((B + 16 * TC - 1) / (16 * TC));
+  k_gemm<TR, TC, OUT, PARTIAL><<<n, 256, 0, s>>>(Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
 }
-// One workgroup per CU runs at a time (registers and LDS), so a grid whose
-// last round would hold only a few workgroups is split: whole rounds of
-// four-column-tile workgroups, then the remaining column tiles one per
-// workgroup (a quarter of the work each), which finish in a fraction of a
-// round. Every output is computed the same way either way.
+// The task shape of a product: the one whose busiest CU has the least work,
+// counted as tasks per CU (rounded up) x tiles per task x the cost of a tile
+// in that shape -- 1.06, 1.15 and 1.3 of a 4x2 task's, as smaller tasks load
+// more operand bytes per tile (wide products, all CUs full: 97 TFLOP/s at
+// 4x2, 93, 86 and 76 for 3072 x 576 by 2048 rows). E.g. 576 x 1536: 2048
+// rows 44.2 us at 4x2 (2.25 tasks per CU), 38.4 at 2x2; 301 rows 15.0, 10.0,
+// and 9.2 at 1x1. Every output is computed the same way in every shape.
+// A K that ends inside a chunk takes the 1x1 tasks.
 template <uint32_t OUT>
-static bool launch_gemm_out(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
+static void launch_gemm_out(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
                             uint32_t B, float* Y, uint32_t ldy, const float* scale,
-                            const uint32_t* gen, uint32_t ncu, float* P, float* QS, size_t qs_floats,
-                            float* inv_out, float eps, bool leave_planes) {
-  // Returns whether the rows' 1/rms (inv_out) was written as well (GO_RESID),
-  // or whether the product was left as QS's four subtree planes and Y not
-  // written (GO_PLAIN with leave_planes).
-  const uint32_t nct = (B + 15) / 16, nrg = (M + 63) / 64;
-  // Narrow batches: four full column tiles and a row group per CU take the
-  // four-tile tasks below; fewer row groups split the segments four ways
-  // (the subtrees in QS, then combined); otherwise one row tile per task.
-  if (nct <= 4 && !(nct == 4 && nrg >= ncu) && QS && nrg < ncu && (size_t)4 * B * M <= qs_floats) {
-    const uint32_t per_cu = gemm_q_lds_bytes() <= 80 * 1024 ? 2 : 1;
-    const uint32_t grid = std::min(4 * ((M + 31) / 32) * ((nct + 3) / 4), per_cu * ncu);
-    if (K % 64 == 0)
-      k_gemm_q<false><<<grid, GEMM_WAVES * WAVE, gemm_q_lds_bytes(), s>>>(Wp, M, K, Xp, B, QS);
-    else
-      k_gemm_q<true><<<grid, GEMM_WAVES * WAVE, gemm_q_lds_bytes(), s>>>(Wp, M, K, Xp, B, QS);
-    if (OUT == GO_RESID && inv_out) {
-      k_gemm_qcomb_rms<<<B, 256, 0, s>>>(QS, M, B, Y, ldy, P, eps, inv_out);
-      return true;
-    }
-    if (OUT == GO_PLAIN && leave_planes) return true;
-    k_gemm_qcomb<OUT><<<dim3((M + 255) / 256, B), 256, 0, s>>>(QS, M, B, Y, ldy, scale, gen, P);
-    return false;
+                            const uint32_t* gen, uint32_t ncu, float* P) {
+  if (K % 64 != 0)
+    return launch_gemm_tile<1, 1, OUT, true>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+  auto cost = [&](uint32_t tr, uint32_t tc, float per_tile) {
+    const uint32_t n = ((M + 16 * tr - 1) / (16 * tr)) * ((B + 16 * tc - 1) / (16 * tc));
+    return (float)((n + ncu - 1) / ncu * tr * tc) * per_tile;
+  };
+  const float c[4] = {cost(4, 2, 1.0f), cost(2, 2, 1.06f), cost(2, 1, 1.15f), cost(1, 1, 1.3f)};
+  switch (std::min_element(c, c + 4) - c) {
+    case 0: return launch_gemm_tile<4, 2, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+    case 1: return launch_gemm_tile<2, 2, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+    case 2: return launch_gemm_tile<2, 1, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+    default: return launch_gemm_tile<1, 1, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
   }
-
-  if (nct <= 4 && !(nct == 4 && nrg >= ncu)) {  // narrow: one row tile per task
-    const uint32_t grid = std::min((M + 15) / 16, 2 * ncu), threads = GEMM_WAVES * WAVE;
-    if (K % 64 == 0)
-      k_gemm_n<OUT, false><<<grid, threads, gemm_n_lds_bytes(), s>>>(Wp, M, K, Xp, B, Y, ldy, scale,
-                                                                     gen, P);
-    else
-      k_gemm_n<OUT, true><<<grid, threads, gemm_n_lds_bytes(), s>>>(Wp, M, K, Xp, B, Y, ldy, scale,
-                                                                    gen, P);
-    return false;
-  }
-  const uint32_t w4 = nrg * ((nct + 3) / 4), rounds = w4 / ncu, rest = w4 % ncu;
-  if (rounds >= 1 && rest > 0 && rest * 4 <= ncu) {
-    const uint32_t y4 = rounds * ncu / nrg;  // column groups of 4 in the whole rounds
-    if (y4 >= 1 && 4 * y4 < nct) {
-      launch_gemm_tn<4, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, 0, 4 * y4, ncu, P);
-      launch_gemm_tn<1, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, 4 * y4, nct - 4 * y4, ncu, P);
-      return false;
-    }
-  }
-  launch_gemm_tn<4, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, 0, nct, ncu, P);
-  return false;
 }
 // P: GO_RESID's panel of the updated rows (K = M).
-// QS / qs_floats: scratch for the quarter-split narrow GEMM (null: not used).
-// inv_out (GO_RESID, ldy = M): the updated rows' 1/rms (k_b_rms's order) as
-// well; returns whether this launch wrote it (else the caller runs k_b_rms).
-// leave_planes (GO_PLAIN): the quarter-split product may stay as QS's
-// subtree planes for the consumer to combine; returns whether it did.
-static bool launch_gemm(hipStream_t s, uint32_t ncu, uint32_t out, const float* Wp, uint32_t M,
+static void launch_gemm(hipStream_t s, uint32_t ncu, uint32_t out, const float* Wp, uint32_t M,
                         uint32_t K, const float* Xp, uint32_t B, float* Y, uint32_t ldy,
                         const float* scale = nullptr, const uint32_t* gen = nullptr,
-                        float* P = nullptr, float* QS = nullptr, size_t qs_floats = 0,
-                        float* inv_out = nullptr, float eps = 0.0f, bool leave_planes = false) {
+                        float* P = nullptr) {
   if (out == GO_PLAIN)
-    return launch_gemm_out<GO_PLAIN>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P, QS,
-                                     qs_floats, nullptr, eps, leave_planes);
-  if (out == GO_RESID)
-    return launch_gemm_out<GO_RESID>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P, QS,
-                                     qs_floats, inv_out, eps, false);
-  return launch_gemm_out<GO_TAG>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P, QS, qs_floats,
-                                 nullptr, eps, false);
+    launch_gemm_out<GO_PLAIN>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
+  else if (out == GO_RESID)
+    launch_gemm_out<GO_RESID>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
+  else
+    launch_gemm_out<GO_TAG>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
 }
 
 // Timing of one launch (profiling on): events recorded around it on the
@@ -2161,25 +2081,20 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   }
   if (!deferred) k_begin<<<1, 1, 0, s>>>(w.st);
   const uint32_t ldy = batch_ldy(d);
-  const size_t qs_n = (size_t)4 * std::min(w.rows, 64u) * ldy;
   k_b_embed<<<n, 256, 0, s>>>(w.drows, dtok, m->embed, d.h, w.X, w.XP);
-  // Each layer's residual products also leave the rows' 1/rms for the next
-  // product (GO_RESID with inv_out); the embedding rows need their own.
   k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   for (uint32_t l = 0; l < d.L; ++l) {
-    bool planes;
     {
       ProfSpan ps(m, 0, 2.0 * d.qkv_rows * d.h * n);
-      planes = launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_qkv[l], d.qkv_rows, d.h, w.XP, n, w.Y, ldy,
-                           nullptr, nullptr, nullptr, w.QS, qs_n, nullptr, 0.0f, true);
+      launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_qkv[l], d.qkv_rows, d.h, w.XP, n, w.Y, ldy);
     }
     if (fused) {
       ProfSpan ps(m, 1, attn_flop);
       k_b_attn_f<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(
-          w.rargs, w.drows, w.items, l, w.Y, ldy, planes ? w.QS : nullptr, n, w.INV, w.CNT, w.XQ);
+          w.rargs, w.drows, w.items, l, w.Y, ldy, w.INV, w.CNT, w.XQ);
     } else {
       k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
-          w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows, planes ? w.QS : nullptr, n);
+          w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
       {
         ProfSpan ps(m, 1, attn_flop);
         if (tiled)
@@ -2192,32 +2107,30 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       k_b_comb<<<dim3(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK), 256, 0, s>>>(
           d, w.drows, w.PART, part_words(d), w.XQ);
     }
-    bool inv_done;
     {
       ProfSpan ps(m, 0, 2.0 * d.h * d.q * n);
-      inv_done = launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_o[l], d.h, d.q, w.XQ, n, w.X, d.h, nullptr,
-                             nullptr, w.XP, w.QS, qs_n, w.INV, d.eps);
+      launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_o[l], d.h, d.q, w.XQ, n, w.X, d.h, nullptr, nullptr,
+                  w.XP);
     }
-    if (!inv_done) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
+    k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
     {
       ProfSpan ps(m, 0, 2.0 * 2 * d.ff * d.h * n);
-      launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_gu[l], 2 * d.ff, d.h, w.XP, n, w.Y, ldy, nullptr,
-                  nullptr, nullptr, w.QS, qs_n);
+      launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_gu[l], 2 * d.ff, d.h, w.XP, n, w.Y, ldy);
     }
     k_b_act<<<dim3((d.ff + 255) / 256, n), 256, 0, s>>>(w.Y, ldy, w.INV, d.ff, d.act, w.XQ);
     {
       ProfSpan ps(m, 0, 2.0 * d.h * d.ff * n);
-      inv_done = launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_d[l], d.h, d.ff, w.XQ, n, w.X, d.h, nullptr,
-                             nullptr, w.XP, w.QS, qs_n, w.INV, d.eps);
+      launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_d[l], d.h, d.ff, w.XQ, n, w.X, d.h, nullptr, nullptr,
+                  w.XP);
     }
-    if (!inv_done && l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
+    if (l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   }
   if (nl) {
     k_b_final<<<nl, 64, 0, s>>>(w.X, w.sel, d.h, m->norm, d.eps, w.XQ, w.LINV);
     {
       ProfSpan ps(m, 0, 2.0 * d.V * d.h * nl);
       launch_gemm(s, m->gemm_ncu, GO_TAG, m->p_lm, d.V, d.h, w.XQ, nl, reinterpret_cast<float*>(w.LOGT), d.V,
-                  w.LINV, w.lgen, nullptr, w.QS, qs_n);
+                  w.LINV, w.lgen);
     }
     k_b_chunkmax<<<dim3((d.nvc + 4 * CM_CPW - 1) / (4 * CM_CPW), nl), 256, 0, s>>>(d, w.LOGT, w.lgen, w.VMAX,
                                                                                    w.VARG, nl);
