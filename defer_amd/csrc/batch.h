@@ -333,8 +333,10 @@ __device__ __forceinline__ void qkv_epi_cache(const Dims& d, const BRow& r, uint
   row[i + d.half] = v.y;
 }
 
-// QKV epilogue per (row, pair): q/k/v words tagged for the attention items;
-// k, v into the row's cache at its position.
+// QKV epilogue per (row, pair): k, v into the row's cache at its position;
+// for the attention, q/k/v words tagged, or (TILED: it reads k and v from the
+// cache) the queries alone as floats [row][q].
+template <bool TILED>
 __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict__ rows, uint32_t l,
                             const float* __restrict__ Y, uint32_t ldy, const float* __restrict__ inv,
                             u64* __restrict__ qkvt, uint32_t ldq) {
@@ -346,10 +348,17 @@ __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict_
   const uint32_t hb = p / d.half, i = p - hb * d.half;
   const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
   const float2 v = qkv_epi_pair(*ap, l, r.pos, b, hb, i, Y, ldy, inv[b]);
+  if (hb >= d.nh) qkv_epi_cache(d, r, l, hb, i, v);
+  if (TILED) {
+    if (hb >= d.nh) return;
+    float* qf = reinterpret_cast<float*>(qkvt) + (size_t)b * d.q;
+    qf[r0] = v.x;
+    qf[r1] = v.y;
+    return;
+  }
   const u64 g = (u64)gen_of(d, r.tick, l, PH_QKV) << 32;
   qkvt[(size_t)b * ldq + r0] = g | __float_as_uint(v.x);
   qkvt[(size_t)b * ldq + r1] = g | __float_as_uint(v.y);
-  if (hb >= d.nh) qkv_epi_cache(d, r, l, hb, i, v);
 }
 
 // LDS of the batched kernels that run one-token functions: no weight
@@ -469,252 +478,286 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 //
 // Rows of one cache at consecutive positions (a prefill or a replay) share
 // their K/V rows, so their attention runs as tiles: a workgroup takes 16
-// consecutive query positions (aligned to 16), one chunk of 128 key
-// positions and one kv head, stages the chunk's K and V rows in LDS once, and
-// computes every query's chunk partials (m, l, acc) in the order phase_attn
-// uses (head_dim 64, chunk 128, positions < 2048), with MFMA chains where
-// phase_attn has fma chains:
-//  * score(q, t): 4 chains over 16 elements each (the lanes of a position),
-//    then ((c0 + c1) + (c2 + c3)) * scale;
+// consecutive query positions (aligned to 16), one chunk of key positions
+// (attn_chunk: 128 * NB) and nj query heads of one kv head, and computes
+// every query's chunk partials (m, l, acc) in the order phase_attn uses, with
+// MFMA chains where phase_attn has fma chains:
+//  * score(q, t): HD / 16 chains of 16 elements (the lanes of a position),
+//    then their tree, times scale;
 //  * softmax: phase_attn's sums -- lane slot L = 0..63 adds positions L,
-//    L + 64 from +0, then the wave tree over the 64 slots -- with 16 lanes
-//    per (query, head), lane s holding slots s + 16v, so a wave takes four
-//    (query, head) rows at once;
-//  * value[d]: 16 position groups (attention wave w, group pl: positions
-//    4w + pl + 16k, k ascending), each a chain, then per w the tree over its
-//    four groups and the sum w = 0..3 in order, from +0.
-// Positions past a query's own (t > pos) carry probability +0 and zero V
-// rows, which leave an accumulator unchanged (a chain started at +0 never
-// holds -0). The scores reuse the LDS of K and Q once every wave is done
-// with them, so with three query heads per kv head two workgroups fit a CU.
+//    L + 64, ... from +0, then the wave tree over the 64 slots -- with 16
+//    lanes per (query, head), lane s holding slots s + 16v, so a wave takes
+//    four (query, head) rows at once;
+//  * value[d]: NCW * PV position groups (attention wave w, group pl:
+//    positions PV*w + pl + NCW*PV*k, k ascending), each a chain, then per w
+//    the tree over its PV groups and the sum w = 0..3 in order, from +0.
+// Positions past a query's own (t > pos) carry probability +0, and V rows
+// past the tile's last position are zeros: both leave an accumulator
+// unchanged (a chain started at +0 never holds -0).
+//
+// K and V rows go from memory (L2: the tiles of a chunk run on one XCD)
+// straight into the registers of the one wave that uses them -- wave w takes
+// every fourth key tile for the scores and phase_attn's wave-w position
+// groups for the values -- so LDS holds only the query operands, the scores
+// and one head's partial sums per wave. A lane loads four consecutive
+// elements of a K row and the wave transposes them into MFMA operands with
+// lane swaps. Staging K and V in LDS instead (64 KB per task, two workgroups
+// per CU, half the clocks in LDS stores and loads) took 100 us per layer for
+// 2048 rows of the 135M shape and could not take chunks past 128 positions
+// or head_dim 128.
 
-constexpr uint32_t AT_HD = 64, AT_CH = 128, AT_VROWS = 128;  // 16 groups x 8 positions
-constexpr int AT_VG = 16;  // value position groups (phase_attn: NCW waves x 4)
-static_assert(AT_VG == NCW * 4, "the value groups are phase_attn's");
-constexpr uint32_t AT_KP = 65, AT_VP = 66, AT_QP = 65, AT_SP = 193;  // LDS row pitches (floats)
-
-// Floats of the K + Q region, which the scores then take.
-__host__ __device__ inline size_t attn_tile_kq(uint32_t grp) {
-  const size_t kq = (size_t)AT_CH * AT_KP + (size_t)grp * 16 * AT_QP;
-  const size_t sc = (size_t)grp * 16 * AT_SP;
-  return kq > sc ? kq : sc;
+constexpr uint32_t AT_MAX_NB = 4;  // chunks of up to 512 positions (8192 cached)
+__host__ __device__ constexpr uint32_t at_pitch(uint32_t ch) { return ch + 17; }  // floats of a score row
+// LDS of a task of nj heads: the query operands (then one head's partial
+// sums per wave), the score rows, (m, l) per row.
+__host__ __device__ constexpr uint32_t attn_tile_lds(uint32_t hd, uint32_t nb, uint32_t nj) {
+  const uint32_t qo = nj * hd * 16, wx = NCW * 16 * hd;
+  return 4 * ((qo > wx ? qo : wx) + nj * 16 * (at_pitch(nb * ACHUNK) + 2));
 }
-__host__ __device__ inline size_t attn_tile_lds(uint32_t grp) {
-  return sizeof(float) * (attn_tile_kq(grp) + (size_t)AT_CH * AT_VP + grp * 32);
+// Partials of the tiled path: [row][nh][MAX_ACHUNKS][hd + 4] floats, acc
+// first, then m and l (16-byte aligned rows).
+__host__ __device__ constexpr uint32_t at_part_row(uint32_t hd) { return hd + 4; }
+
+// v[0..3] of lane (lr, lc) = elements 4*lc .. 4*lc+3 of row lr; afterwards
+// v[i] = element 4*i + lc (a 4x4 transpose between components and the wave's
+// four rows of 16 lanes).
+__device__ __forceinline__ void transpose4(float4& v) {
+  auto swap32 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  };
+  auto swap16 = [](float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  };
+  swap32(v.x, v.z);
+  swap32(v.y, v.w);
+  swap16(v.x, v.y);
+  swap16(v.z, v.w);
 }
 
-// tasks[x] = tile << 16 | chunk << 8 | kv head; tiles[m] .. tiles[m + 1] are
-// the batch rows of tile m. rows: the batch (one cache, consecutive
-// positions); qkvt: tagged q/k/v words per row; part: tagged partials.
+// The complete tree over N chain sums (N = 4 or 8).
+template <int N>
+__device__ __forceinline__ f4v chain_tree(const f4v (&a)[N]) {
+  const f4v t = (a[0] + a[1]) + (a[2] + a[3]);
+  if constexpr (N == 8) return t + ((a[4] + a[5]) + (a[6] + a[7]));
+  return t;
+}
+
+// tasks[x] = tile << 16 | chunk << 8 | kv head, each run ny times for nj
+// query heads (heads y*nj ..); tiles[m] .. tiles[m + 1] are the batch rows of
+// tile m. rows: the batch (one cache, consecutive positions); qf: the rows'
+// rotated queries [row][q]; part: the chunk partials.
+template <int HD, int NB>
 __global__ __launch_bounds__(256, 2) void k_b_attn_tile(const Dims d, const BRow* __restrict__ rows,
-                                                     const uint32_t* __restrict__ tasks,
-                                                     const uint32_t* __restrict__ tiles, uint32_t l,
-                                                     const u64* __restrict__ qkvt,
-                                                     u64* __restrict__ part, uint32_t part_w) {
+                                                     const uint32_t* __restrict__ tasks, uint32_t ny,
+                                                     uint32_t nj, const uint32_t* __restrict__ tiles,
+                                                     uint32_t l, const float* __restrict__ qf,
+                                                     float* __restrict__ part) {
+  constexpr int SUBS = HD / 16;                  // chains of a score
+  constexpr int PV = WAVE / (HD / 4);            // value position groups of a wave (phase_attn's pv)
+  constexpr int GV = NCW * PV;                   // ... of all waves: a group's positions are GV apart
+  constexpr int HH = HD / 64;                    // 64-dim halves of a V row
+  constexpr uint32_t CH = NB * ACHUNK, SP = at_pitch(CH);
+  constexpr int MB = ACHUNK / (4 * GV);          // value MFMA steps of 128 positions
+  constexpr bool HOLD = NB * HD <= 128;          // a chunk's V rows fit the registers for all heads
   extern __shared__ float at_lds[];
-  const uint32_t grp = d.group, hs = AT_HD + 2;
-  float* Ks = at_lds;                       // [AT_CH][AT_KP]
-  float* Qs = Ks + AT_CH * AT_KP;           // [grp][16][AT_QP]
-  float* Ss = at_lds;                       // [grp][16][AT_SP]: scores, then probabilities
-  float* Vs = at_lds + attn_tile_kq(grp);   // [AT_CH][AT_VP]
-  float* ML = Vs + AT_CH * AT_VP;           // [grp][16][2]: m, l
-  const uint32_t task = tasks[blockIdx.x];
+  const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+  const uint32_t lr = lane % 16, lc = lane / 16;
+  // Consecutive tasks (same chunk and kv head, the next tile) on one XCD.
+  const uint32_t n_wg = gridDim.x, xk = blockIdx.x % NXCD;
+  const uint32_t ti = xk * (n_wg / NXCD) + min(xk, n_wg % NXCD) + blockIdx.x / NXCD;
+  const uint32_t task = tasks[ti / ny], j0 = ti % ny * nj, njt = min(nj, d.group - j0);
   const uint32_t m = task >> 16, c = (task >> 8) & 0xffu, g = task & 0xffu;
   const uint32_t rb0 = tiles[m], nq = tiles[m + 1] - rb0;
   const BRow r0 = rows[rb0];
-  const uint32_t p_last = r0.pos + nq - 1;
-  const uint32_t t0 = c * AT_CH;
-  const uint32_t nk = min(AT_CH, p_last + 1 - t0);
-  const uint32_t tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE;
-  const float* kb = r0.kc + ((size_t)l * d.nkv + g) * r0.cap * d.kvs;
-  const float* vb = r0.vc + ((size_t)l * d.nkv + g) * r0.cap * d.kvs;
-  // 1. K rows, V rows and Q words of the chunk: each thread issues all its
-  // loads before its first LDS store (16 threads per K/V row).
-  constexpr int NR = AT_CH * 16 / 256;                 // K/V float4 per thread: 8
-  constexpr int NQ = MAX_GROUP * 16 * AT_HD / 256;     // Q words per thread: 16
-  float4 kr[NR], vr[NR];
-  u64 qw[NQ];
-  // Generation tags of this lane's output queries 4*lc + rr (values stage).
-  const uint32_t lr = lane % 16, lc = lane / 16;
-  u64 gtag[4];
-#pragma unroll
-  for (int rr = 0; rr < 4; ++rr) {
-    const uint32_t q = 4 * lc + rr;
-    gtag[rr] = q < nq ? (u64)gen_of(d, rows[rb0 + q].tick, l, PH_ATTN) << 32 : 0;
+  const uint32_t p_last = r0.pos + nq - 1, t0 = c * CH;
+  const uint32_t nk = min(CH, p_last + 1 - t0);
+  const uint32_t qo_n = nj * HD * 16, wx_n = NCW * 16 * HD;
+  float* Qo = at_lds;                                  // [nj][SUBS][lane][4]: MFMA operands
+  float* Wx = at_lds;                                  // [NCW][16][HD], once the scores are done
+  float* Ss = at_lds + (qo_n > wx_n ? qo_n : wx_n);    // [nj][16][SP]: scores, then probabilities
+  float* ML = Ss + nj * 16 * SP;                       // [nj][16][2]: m, l
+  const float* kb = r0.kc + ((size_t)l * d.nkv + g) * r0.cap * HD;
+  const float* vb = r0.vc + ((size_t)l * d.nkv + g) * r0.cap * HD;
+  // 1. Query operands: wave w prepares every fourth (head, chain).
+  const float* qrow = qf + (size_t)(rb0 + min(lr, nq - 1)) * d.q + (size_t)(g * d.group + j0) * HD + 4 * lc;
+  for (uint32_t u = wave; u < njt * SUBS; u += NCW) {
+    float4 v = ldg4(qrow + 16 * u);  // chains of consecutive heads are 16 elements apart
+    transpose4(v);
+    *reinterpret_cast<float4*>(Qo + (size_t)(u * WAVE + lane) * 4) = v;
   }
-#pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const uint32_t e = tid + 256 * k, t = e / 16, q4 = (e % 16) * 4;
-    kr[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    vr[k] = kr[k];
-    if (t < nk) {
-      kr[k] = *reinterpret_cast<const float4*>(kb + (size_t)(t0 + t) * d.kvs + q4);
-      vr[k] = *reinterpret_cast<const float4*>(vb + (size_t)(t0 + t) * d.kvs + q4);
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    const uint32_t e = tid + 256 * k, j = e / (16 * AT_HD), q = (e / AT_HD) % 16, dd = e % AT_HD;
-    qw[k] = 0;
-    if (j < grp && q < nq) qw[k] = qkvt[(size_t)(rb0 + q) * d.qkv_rows + (g * grp + j) * AT_HD + dd];
-  }
-#pragma unroll
-  for (int k = 0; k < NR; ++k) {
-    const uint32_t e = tid + 256 * k, t = e / 16, q4 = (e % 16) * 4;
-    float* kd = Ks + t * AT_KP + q4;
-    float* vd = Vs + t * AT_VP + q4;
-    kd[0] = kr[k].x;
-    kd[1] = kr[k].y;
-    kd[2] = kr[k].z;
-    kd[3] = kr[k].w;
-    vd[0] = vr[k].x;
-    vd[1] = vr[k].y;
-    vd[2] = vr[k].z;
-    vd[3] = vr[k].w;
-  }
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    const uint32_t e = tid + 256 * k, j = e / (16 * AT_HD), q = (e / AT_HD) % 16, dd = e % AT_HD;
-    if (j < grp) Qs[(j * 16 + q) * AT_QP + dd] = __uint_as_float((uint32_t)qw[k]);
-  }
-  __syncthreads();
-  // 2. scores: wave w takes key tiles w and w + 4, kept in registers until
-  // every wave is done with K and Q, whose LDS the scores then take. The
-  // (head, sub) chains of a key tile run interleaved.
+  // The wave's first key tile is requested before the barrier.
   const uint32_t nkt = (nk + 15) / 16;
-  float qa[MAX_GROUP][4][4];  // element 16*sub + 4*i + lc of query lr, head j
+  float4 kf[SUBS];
+  auto load_k = [&](uint32_t kt) {
+    const float* r = kb + (size_t)min(t0 + kt * 16 + lr, p_last) * HD + 4 * lc;
 #pragma unroll
-  for (uint32_t j = 0; j < MAX_GROUP; ++j)
+    for (int u = 0; u < SUBS; ++u) kf[u] = ldg4(r + 16 * u);
+  };
+  if (wave < nkt) load_k(wave);
+  __syncthreads();
+  // 2. Scores of the wave's key tiles, the next tile's rows in flight.
+#pragma unroll 1
+  for (uint32_t kt = wave; kt < nkt; kt += NCW) {
+    float4 ka[SUBS];
 #pragma unroll
-    for (int sub = 0; sub < 4; ++sub)
+    for (int u = 0; u < SUBS; ++u) {
+      ka[u] = kf[u];
+      transpose4(ka[u]);
+    }
+    if (kt + NCW < nkt) load_k(kt + NCW);
+#pragma unroll 1
+    for (uint32_t j = 0; j < njt; ++j) {
+      float4 qa[SUBS];
+#pragma unroll
+      for (int u = 0; u < SUBS; ++u)
+        qa[u] = *reinterpret_cast<const float4*>(Qo + (size_t)((j * SUBS + u) * WAVE + lane) * 4);
+      f4v acc[SUBS];
+#pragma unroll
+      for (int u = 0; u < SUBS; ++u) acc[u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        qa[j][sub][i] = j < grp ? Qs[(j * 16 + lr) * AT_QP + 16 * sub + 4 * i + lc] : 0.0f;
-  f4v sreg[2][MAX_GROUP];
 #pragma unroll
-  for (uint32_t u = 0; u < 2; ++u) {
-    const uint32_t kt = wave + 4 * u;
-    if (kt >= nkt) continue;
-    float ka[4][4];
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ka[sub][i] = Ks[(kt * 16 + lr) * AT_KP + 16 * sub + 4 * i + lc];
-    f4v acc[MAX_GROUP][4];
-#pragma unroll
-    for (uint32_t j = 0; j < MAX_GROUP; ++j)
-#pragma unroll
-      for (int sub = 0; sub < 4; ++sub) acc[j][sub] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (uint32_t j = 0; j < MAX_GROUP; ++j) {
-        if (j >= grp) continue;
-#pragma unroll
-        for (int sub = 0; sub < 4; ++sub)
-          acc[j][sub] = __builtin_amdgcn_mfma_f32_16x16x4f32(qa[j][sub][i], ka[sub][i], acc[j][sub],
-                                                             0, 0, 0);
-      }
-#pragma unroll
-    for (uint32_t j = 0; j < MAX_GROUP; ++j)
-      sreg[u][j] = (acc[j][0] + acc[j][1]) + (acc[j][2] + acc[j][3]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (uint32_t u = 0; u < 2; ++u) {
-    const uint32_t kt = wave + 4 * u;
-#pragma unroll
-    for (uint32_t j = 0; j < MAX_GROUP; ++j) {
-      if (kt >= nkt || j >= grp) continue;
+        for (int u = 0; u < SUBS; ++u)
+          acc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32((&qa[u].x)[i], (&ka[u].x)[i], acc[u], 0, 0, 0);
+      const f4v sc = chain_tree(acc);
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr)  // query 4*lc + rr, key kt*16 + lr
-        Ss[(j * 16 + 4 * lc + rr) * AT_SP + kt * 16 + lr] = sreg[u][j][rr] * d.scale;
+        Ss[(j * 16 + 4 * lc + rr) * SP + kt * 16 + lr] = sc[rr] * d.scale;
     }
   }
+  // The value rows of a 128-position block: wave w's groups PV*w + pl, group
+  // positions 4*mm + lc, dims 64*hh + 4*lr .. +3.
+  float4 vf[HOLD ? NB : 1][PV][MB][HH];
+  auto load_v = [&](int nb, float4 (&v)[PV][MB][HH]) {
+#pragma unroll
+    for (int pl = 0; pl < PV; ++pl)
+#pragma unroll
+      for (int mm = 0; mm < MB; ++mm) {
+        const uint32_t p = nb * ACHUNK + PV * wave + pl + GV * (4 * mm + lc);
+        const float* r = vb + (size_t)min(t0 + p, p_last) * HD + 4 * lr;
+#pragma unroll
+        for (int hh = 0; hh < HH; ++hh) v[pl][mm][hh] = ldg4(r + 64 * hh);
+      }
+  };
+  auto zero_v = [&](int nb, float4 (&v)[PV][MB][HH]) {  // rows past the tile's last position
+    if (nk == CH) return;
+#pragma unroll
+    for (int pl = 0; pl < PV; ++pl)
+#pragma unroll
+      for (int mm = 0; mm < MB; ++mm)
+        if (nb * ACHUNK + PV * wave + pl + GV * (4 * mm + lc) >= nk)
+#pragma unroll
+          for (int hh = 0; hh < HH; ++hh) v[pl][mm][hh] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  };
+  if constexpr (HOLD)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) load_v(nb, vf[nb]);
   __syncthreads();
-  // 3. softmax statistics and probabilities, 16 lanes per (query, head):
-  // lane sub holds phase_attn's lane slots L = sub + 16v (v = 0..3), each
-  // the sum of positions L, L + 64 from +0; the slots' tree is group_sum
-  // over the 16 lanes of each v, then (R3 + R2) + (R1 + R0) as wave_sum.
-  // A lane's eight positions sub + 16k are read at once; positions from n
-  // on (up to AT_VROWS) get probability +0.
-  {
-    const uint32_t sub = lane % 16;
-    for (uint32_t u0 = 4 * wave; u0 < grp * 16; u0 += 16) {
-      const uint32_t u = u0 + lane / 16;
-      const uint32_t j = u / 16, q = u % 16;
-      float* sh = Ss + u * AT_SP;
-      const uint32_t n = q < nq ? min(AT_CH, r0.pos + q + 1 - t0) : 0;
-      float sv[8];
+  // 3. Softmax statistics and probabilities, 16 lanes per (query, head):
+  // lane sub holds phase_attn's lane slots L = sub + 16v (v = 0..3); the
+  // slots' tree is group_sum over the 16 lanes of each v, then (R3 + R2) +
+  // (R1 + R0) as wave_sum. Positions from n on get probability +0.
+  for (uint32_t u0 = 4 * wave; u0 < njt * 16; u0 += 16) {
+    const uint32_t u = u0 + lane / 16, q = u % 16, sub = lane % 16;
+    float* sh = Ss + u * SP;
+    const uint32_t n = q < nq ? min(CH, r0.pos + q + 1 - t0) : 0;
+    float e[8 * NB];
+    float mx = -INFINITY;
 #pragma unroll
-      for (uint32_t k = 0; k < 8; ++k) {
-        const uint32_t i = sub + 16 * k;
-        sv[k] = i < n ? sh[i] : -INFINITY;
-      }
-      float mx = -INFINITY;
+    for (int k = 0; k < 8 * NB; ++k) {
+      const uint32_t i = sub + 16 * k;
+      e[k] = i < n ? sh[i] : -INFINITY;
+      mx = fmaxf(mx, e[k]);
+    }
+    mx = row_max(mx);
 #pragma unroll
-      for (uint32_t k = 0; k < 8; ++k) mx = fmaxf(mx, sv[k]);
-      mx = row_max(mx);
-      float e[8];
+    for (int k = 0; k < 8 * NB; ++k) {
+      const uint32_t i = sub + 16 * k;
+      e[k] = (i < n && mx != -INFINITY) ? expf(e[k] - mx) : 0.0f;
+      sh[i] = e[k];
+    }
+    float R[4];
 #pragma unroll
-      for (uint32_t k = 0; k < 8; ++k) {
-        const uint32_t i = sub + 16 * k;
-        e[k] = (i < n && mx != -INFINITY) ? expf(sv[k] - mx) : 0.0f;
-        sh[i] = e[k];
-      }
+    for (int v = 0; v < 4; ++v) {
+      float t = 0.0f;
 #pragma unroll
-      for (uint32_t k = 8; k < AT_VROWS / 16; ++k) sh[sub + 16 * k] = 0.0f;
-      float R[4];
-#pragma unroll
-      for (uint32_t v = 0; v < 4; ++v) R[v] = group_sum((0.0f + e[v]) + e[v + 4], 16);
-      const float lsum = (R[3] + R[2]) + (R[1] + R[0]);
-      if (sub == 0) {
-        ML[(j * 16 + q) * 2] = mx;
-        ML[(j * 16 + q) * 2 + 1] = lsum;
-      }
+      for (int k = 0; k < 2 * NB; ++k) t = t + e[v + 4 * k];
+      R[v] = group_sum(t, 16);
+    }
+    if (sub == 0) {
+      ML[u * 2] = mx;
+      ML[u * 2 + 1] = (R[3] + R[2]) + (R[1] + R[0]);
     }
   }
-  __syncthreads();
-  // 4. values: wave w computes dims 16w..16w+15 of every head; the V
-  // operands are read once for all heads.
-  float vop[AT_VG][2];
+  if constexpr (HOLD)
 #pragma unroll
-  for (int gi = 0; gi < AT_VG; ++gi)
+    for (int nb = 0; nb < NB; ++nb) zero_v(nb, vf[nb]);
+  // 4. Values, one head at a time.
+#pragma unroll 1
+  for (uint32_t j = 0; j < njt; ++j) {
+    f4v acc[PV][HH][4];
 #pragma unroll
-    for (int mm = 0; mm < 2; ++mm) {
-      const uint32_t pos = gi + AT_VG * (4 * mm + lc);  // group gi = 4*w' + pl
-      vop[gi][mm] = pos < AT_CH ? Vs[pos * AT_VP + 16 * wave + lr] : 0.0f;
+    for (int pl = 0; pl < PV; ++pl)
+#pragma unroll
+      for (int hh = 0; hh < HH; ++hh)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc[pl][hh][u] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (!HOLD) load_v(0, vf[0]);
+    __syncthreads();  // the probabilities (j = 0), or the last head's Wx read, are done
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if constexpr (!HOLD) {
+        if (nb > 0) load_v(nb, vf[0]);
+        zero_v(nb, vf[0]);
+      }
+      float4 (&v)[PV][MB][HH] = vf[HOLD ? nb : 0];
+#pragma unroll
+      for (int mm = 0; mm < MB; ++mm)
+#pragma unroll
+        for (int pl = 0; pl < PV; ++pl) {
+          const float p = Ss[(j * 16 + lr) * SP + nb * ACHUNK + PV * wave + pl + GV * (4 * mm + lc)];
+#pragma unroll
+          for (int hh = 0; hh < HH; ++hh)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+              acc[pl][hh][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(p, (&v[pl][mm][hh].x)[u],
+                                                                    acc[pl][hh][u], 0, 0, 0);
+        }
     }
-  for (uint32_t j = 0; j < grp; ++j) {
-    float pop[AT_VG][2];
 #pragma unroll
-    for (int gi = 0; gi < AT_VG; ++gi)
+    for (int hh = 0; hh < HH; ++hh) {
+      f4v w[4];
 #pragma unroll
-      for (int mm = 0; mm < 2; ++mm) pop[gi][mm] = Ss[(j * 16 + lr) * AT_SP + gi + AT_VG * (4 * mm + lc)];
-    f4v acc[AT_VG];
+      for (int u = 0; u < 4; ++u) {
+        w[u] = acc[0][hh][u] + acc[1][hh][u];
+        if constexpr (PV == 4) w[u] = w[u] + (acc[2][hh][u] + acc[3][hh][u]);
+      }
 #pragma unroll
-    for (int gi = 0; gi < AT_VG; ++gi) acc[gi] = f4v{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int mm = 0; mm < 2; ++mm)
-#pragma unroll
-      for (int gi = 0; gi < AT_VG; ++gi)
-        acc[gi] = __builtin_amdgcn_mfma_f32_16x16x4f32(pop[gi][mm], vop[gi][mm], acc[gi], 0, 0, 0);
-    f4v A = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int w4 = 0; w4 < AT_VG / 4; ++w4) {
-      const f4v W = (acc[4 * w4] + acc[4 * w4 + 1]) + (acc[4 * w4 + 2] + acc[4 * w4 + 3]);
-      A = A + W;
+      for (int rr = 0; rr < 4; ++rr)  // query 4*lc + rr, dims 64*hh + 4*lr ..
+        *reinterpret_cast<float4*>(Wx + (size_t)(wave * 16 + 4 * lc + rr) * HD + 64 * hh + 4 * lr) =
+            make_float4(w[0][rr], w[1][rr], w[2][rr], w[3][rr]);
     }
-    const uint32_t hh = g * grp + j;
+    __syncthreads();
+    const uint32_t hidx = g * d.group + j0 + j;
 #pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {  // query 4*lc + rr, dim 16*wave + lr
-      const uint32_t q = 4 * lc + rr;
+    for (uint32_t e = tid * 4; e < 16 * HD; e += 1024) {
+      const uint32_t q = e / HD, dd = e % HD;
+      float4 A = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+      for (uint32_t w = 0; w < NCW; ++w) {
+        const float4 x = *reinterpret_cast<const float4*>(Wx + (size_t)w * 16 * HD + e);
+        A = make_float4(A.x + x.x, A.y + x.y, A.z + x.z, A.w + x.w);
+      }
       if (q >= nq) continue;
-      u64* out = part + (size_t)(rb0 + q) * part_w + ((size_t)hh * MAX_ACHUNKS + c) * hs;
-      out[2 + 16 * wave + lr] = gtag[rr] | __float_as_uint(A[rr]);
-      if (wave == 0 && lr == 0) {
-        out[0] = gtag[rr] | __float_as_uint(ML[(j * 16 + q) * 2]);
-        out[1] = gtag[rr] | __float_as_uint(ML[(j * 16 + q) * 2 + 1]);
+      float* out = part + (((size_t)(rb0 + q) * d.nh + hidx) * MAX_ACHUNKS + c) * at_part_row(HD);
+      *reinterpret_cast<float4*>(out + dd) = A;
+      if (dd == 0) {
+        out[HD] = ML[(j * 16 + q) * 2];
+        out[HD + 1] = ML[(j * 16 + q) * 2 + 1];
       }
     }
   }
@@ -723,11 +766,13 @@ __global__ __launch_bounds__(256, 2) void k_b_attn_tile(const Dims d, const BRow
 // Combine of the chunk partials (combine_scales / combine_value, as the O
 // phase does) into the panel of att[b][q]: one workgroup per row and group of
 // heads; the weights of a head's chunks are formed once in LDS (a wave per
-// head, a lane per chunk), then a thread per (head, dim). The
-// partials were written by earlier launches on the same stream, so their
-// values are read directly (the low half of each tagged word).
+// head, a lane per chunk), then a thread per (head, dim). The partials were
+// written by earlier launches on the same stream, so their values are read
+// directly: TILED, the tiled attention's floats; otherwise the low half of
+// each tagged word (m, l, acc).
 constexpr uint32_t COMB_MAX_HEADS = 64;
 constexpr uint32_t COMB_HEADS_PER_BLOCK = 4;  // grid y: groups of heads
+template <bool TILED>
 __global__ __launch_bounds__(256) void k_b_comb(const Dims d, const BRow* __restrict__ rows,
                                                 const u64* __restrict__ part, uint32_t part_w,
                                                 float* __restrict__ attp) {
@@ -735,21 +780,26 @@ __global__ __launch_bounds__(256) void k_b_comb(const Dims d, const BRow* __rest
   __shared__ float ls[COMB_HEADS_PER_BLOCK];
   const uint32_t b = blockIdx.x, h0 = blockIdx.y * COMB_HEADS_PER_BLOCK;
   const uint32_t nh = min(COMB_HEADS_PER_BLOCK, d.nh - h0);
-  const uint32_t nch = attn_nchunks(rows[b].pos), hs = d.hd + 2;
+  const uint32_t nch = attn_nchunks(rows[b].pos);
+  // Float i (0: m, 1: l, 2 + dim: acc) of chunk c of head h0 + k.
   const u64* pb = part + (size_t)b * part_w;
+  const float* pf = reinterpret_cast<const float*>(part) + (size_t)b * d.nh * MAX_ACHUNKS * at_part_row(d.hd);
+  auto val = [&](uint32_t k, uint32_t c, uint32_t i) {
+    const size_t at = (size_t)(h0 + k) * MAX_ACHUNKS + c;
+    if (TILED) return pf[at * at_part_row(d.hd) + (i < 2 ? d.hd + i : i - 2)];
+    return __uint_as_float((uint32_t)pb[at * (d.hd + 2) + i]);
+  };
   const uint32_t wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  auto val = [](const u64* p) { return __uint_as_float((uint32_t)*p); };
   // combine_scales for head h0 + wave, one lane per chunk: M is a maximum
   // (the same in any order, NaN maxima dropped as fmaxf from -inf drops
   // them), each weight the same expf, and the weighted total summed in
   // chunk order by lane 0 from the lanes' products (no contraction).
   if (wave < nh) {
-    const u64* p = pb + (size_t)(h0 + wave) * MAX_ACHUNKS * hs;
     if (nch == 1) {
-      if (lane == 0) ls[wave] = val(p + 1) * 1.0f;
+      if (lane == 0) ls[wave] = val(wave, 0, 1) * 1.0f;
     } else {
-      const float mc = lane < nch ? val(p + lane * hs) : -INFINITY;
-      const float lc = lane < nch ? val(p + lane * hs + 1) : 0.0f;
+      const float mc = lane < nch ? val(wave, lane, 0) : -INFINITY;
+      const float lc = lane < nch ? val(wave, lane, 1) : 0.0f;
       float M = fmaxf(-INFINITY, mc);
       for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
       const float w = (mc == -INFINITY) ? 0.0f : expf(mc - M);
@@ -765,10 +815,9 @@ __global__ __launch_bounds__(256) void k_b_comb(const Dims d, const BRow* __rest
   // sum in chunk order).
   for (uint32_t v = threadIdx.x; v < nh * d.hd; v += blockDim.x) {
     const uint32_t k = v / d.hd, dd = v - k * d.hd, u = (h0 + k) * d.hd + dd;
-    const u64* p = pb + (size_t)(h0 + k) * MAX_ACHUNKS * hs + 2 + dd;
     float x[MAX_ACHUNKS];
 #pragma unroll
-    for (uint32_t c = 0; c < MAX_ACHUNKS; ++c) x[c] = c < nch ? val(p + c * hs) : 0.0f;
+    for (uint32_t c = 0; c < MAX_ACHUNKS; ++c) x[c] = c < nch ? val(k, c, 2 + dd) : 0.0f;
     float out;
     if (nch == 1) {
       out = (x[0] * 1.0f) / ls[k];

@@ -458,6 +458,24 @@ static size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 // LDS of one gfx950 compute unit, all of which a workgroup may take.
 static constexpr size_t LDS_BYTES_MAX = 160 * 1024;
 
+// The tiled attention for chunks of nb * 128 positions, if there is one.
+static const void* attn_tile_kernel(uint32_t hd, uint32_t nb) {
+  static const void* const k[2][AT_MAX_NB] = {
+      {(const void*)k_b_attn_tile<64, 1>, (const void*)k_b_attn_tile<64, 2>,
+       (const void*)k_b_attn_tile<64, 3>, (const void*)k_b_attn_tile<64, 4>},
+      {(const void*)k_b_attn_tile<128, 1>, (const void*)k_b_attn_tile<128, 2>,
+       (const void*)k_b_attn_tile<128, 3>, (const void*)k_b_attn_tile<128, 4>}};
+  if ((hd != 64 && hd != 128) || nb < 1 || nb > AT_MAX_NB) return nullptr;
+  return k[hd == 128][nb - 1];
+}
+// Query heads of a group in one task, at most: as many as leave LDS for two
+// workgroups per CU.
+static uint32_t attn_tile_heads(const Dims& d, uint32_t nb) {
+  uint32_t nj = d.group;
+  while (nj > 1 && attn_tile_lds(d.hd, nb, nj) > LDS_BYTES_MAX / 2) --nj;
+  return nj;
+}
+
 extern "C" size_t defer_gpu_model_tensor_count(const defer_gpu_config* c) {
   const size_t per_layer = c->has_bias ? 12 : 9;
   return 1 + (size_t)c->num_layers * per_layer + 1 + (c->tie_word_embeddings ? 0 : 1);
@@ -805,10 +823,12 @@ extern "C" int defer_gpu_model_create(const defer_gpu_config* cfg, const float* 
 
   rc = apply_layout(m, std::min<uint32_t>(m->ncu, min_items));
   if (rc) return cleanup(rc);
-  e = hipFuncSetAttribute((const void*)k_b_attn_tile, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)attn_tile_lds(MAX_GROUP));
-  if (e != hipSuccess)
-    return cleanup(fail(DEFER_GPU_E_HIP, "LDS attribute (tiled attention): %s", hipGetErrorString(e)));
+  for (uint32_t nb = 1; nb <= AT_MAX_NB && attn_tile_kernel(m->d.hd, nb); ++nb) {
+    e = hipFuncSetAttribute(attn_tile_kernel(m->d.hd, nb), hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)attn_tile_lds(m->d.hd, nb, attn_tile_heads(m->d, nb)));
+    if (e != hipSuccess)
+      return cleanup(fail(DEFER_GPU_E_HIP, "LDS attribute (tiled attention): %s", hipGetErrorString(e)));
+  }
   if (hipEventCreate(&m->ev0) != hipSuccess || hipEventCreate(&m->ev1) != hipSuccess)
     return cleanup(fail(DEFER_GPU_E_HIP, "event create"));
   *out = m;
@@ -1816,7 +1836,7 @@ static int ensure_ws(defer_gpu_model* m, uint32_t rows, uint32_t lm) {
   HIP_TRY(counted_malloc(&w.drows, (size_t)R * sizeof(BRow)));
   HIP_TRY(counted_malloc(&w.rargs, (size_t)R * sizeof(Args)));
   HIP_TRY(counted_malloc(&w.items, (size_t)R * d.nkv * MAX_ACHUNKS * d.group * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.tiles, ((size_t)R / 16 + 2) * sizeof(uint32_t)));
+  HIP_TRY(counted_malloc(&w.tiles, ((size_t)R / 16 + 3) * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&w.CNT, (size_t)R * d.nkv * sizeof(uint32_t)));
   HIP_TRY(hipMemset(w.CNT, 0, (size_t)R * d.nkv * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&w.sets, (size_t)R * sizeof(StateSet)));
@@ -2005,6 +2025,26 @@ static Args row_args(const defer_gpu_cache* c, const BatchWs& w, uint32_t b) {
   return a;
 }
 
+// n_items tiled attention tasks of one chunk size. Where all the heads of a
+// group in one task leave CUs without two workgroups, a task is one head
+// (its K/V rows then come from L2 once per head): 301 rows of the 135M shape
+// are 99 tasks, or 297 of one head.
+static void launch_attn_tile(defer_gpu_model* m, uint32_t nb, const uint32_t* items, uint32_t n_items,
+                             uint32_t l) {
+  const Dims& d = m->d;
+  BatchWs& w = *m->bw;
+  if (!n_items) return;
+  uint32_t nj = attn_tile_heads(d, nb);
+  if (n_items * ((d.group + nj - 1) / nj) < 2 * m->gemm_ncu) nj = 1;
+  uint32_t ny = (d.group + nj - 1) / nj;
+  const float* qf = reinterpret_cast<const float*>(w.QKVT);
+  float* part = reinterpret_cast<float*>(w.PART);
+  Dims dv = d;
+  void* args[] = {&dv, &w.drows, &items, &ny, &nj, &w.tiles, &l, &qf, &part};
+  (void)hipLaunchKernel(attn_tile_kernel(d.hd, nb), dim3(n_items * ny), dim3(256), args,
+                        attn_tile_lds(d.hd, nb, nj), m->stream);
+}
+
 // Runs n rows (n <= BATCH_MAX_ROWS) through every layer; logits rows
 // sel[0..nl) (batch row indices) get tagged logits and chunk maxima in the
 // workspace. Rows must already be validated (tokens, capacity).
@@ -2023,9 +2063,13 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   std::vector<Args> ra(n);
   for (uint32_t b = 0; b < n; ++b) ra[b] = row_args(rcache[b], w, b);
   // Attention: tiles of 16 aligned positions when the rows are one cache's
-  // consecutive positions (a prefill or a replay) and the shape is the tiled
-  // kernel's; otherwise one workgroup per (row, item).
-  bool tiled = d.hd == AT_HD && d.kvs == AT_HD && rows[n - 1].pos < ACHUNK * MAX_ACHUNKS;
+  // consecutive positions (a prefill or a replay) and the tiled kernel has
+  // the shape and the chunk sizes (at most two: the chunk grows every 2048
+  // positions, and a batch has at most 2048 rows); otherwise one workgroup
+  // per (row, item). 360M shape, 1452 rows from position 2048: 1,152 us per
+  // layer as items, 128-position chunks aside the only way before.
+  const uint32_t nb0 = attn_chunk(rows[0].pos) / ACHUNK, nb1 = attn_chunk(rows[n - 1].pos) / ACHUNK;
+  bool tiled = attn_tile_kernel(d.hd, nb0) && attn_tile_kernel(d.hd, nb1);
   for (uint32_t b = 1; b < n && tiled; ++b)
     tiled = rcache[b] == rcache[0] && rows[b].pos == rows[0].pos + b;
   // Rows of distinct caches (a lockstep step) run the attention with its
@@ -2038,15 +2082,23 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     fused = std::adjacent_find(cs.begin(), cs.end()) == cs.end();
   }
   std::vector<uint32_t> items, tiles;
+  uint32_t n_items0 = 0;  // tiled: tasks of the first chunk size
   if (tiled) {
     tiles.push_back(0);
     for (uint32_t b = 1; b < n; ++b)
       if (rows[b].pos % 16 == 0) tiles.push_back(b);
     tiles.push_back(n);
-    for (uint32_t t = 0; t + 1 < tiles.size(); ++t) {
-      const uint32_t nch = attn_nchunks(rows[tiles[t]].pos);
-      for (uint32_t c = 0; c < nch; ++c)
-        for (uint32_t g = 0; g < d.nkv; ++g) items.push_back(t << 16 | c << 8 | g);
+    // The tasks of each chunk size in order of (chunk, kv head, tile): a
+    // chunk's K/V rows are used by consecutive tasks.
+    for (uint32_t nb = nb0; nb <= nb1; ++nb) {
+      const uint32_t nch1 = attn_nchunks(rows[n - 1].pos);
+      for (uint32_t c = 0; c < MAX_ACHUNKS && (nb < nb1 || c < nch1); ++c)
+        for (uint32_t g = 0; g < d.nkv; ++g)
+          for (uint32_t t = 0; t + 1 < tiles.size(); ++t) {
+            const uint32_t p = rows[tiles[t]].pos;
+            if (attn_chunk(p) == nb * ACHUNK && c < attn_nchunks(p)) items.push_back(t << 16 | c << 8 | g);
+          }
+      if (nb == nb0) n_items0 = (uint32_t)items.size();
     }
   } else {
     // Grouped items x = (kv head, chunk): every query head of the group in
@@ -2093,19 +2145,25 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       k_b_attn_f<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(
           w.rargs, w.drows, w.items, l, w.Y, ldy, w.INV, w.CNT, w.XQ);
     } else {
-      k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
-          w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
+      const dim3 epi_grid((d.qkv_rows / 2 + 255) / 256, n);
+      if (tiled)
+        k_b_qkv_epi<true><<<epi_grid, 256, 0, s>>>(w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
+      else
+        k_b_qkv_epi<false><<<epi_grid, 256, 0, s>>>(w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
       {
         ProfSpan ps(m, 1, attn_flop);
-        if (tiled)
-          k_b_attn_tile<<<(uint32_t)items.size(), 256, attn_tile_lds(d.group), s>>>(
-              d, w.drows, w.items, w.tiles, l, w.QKVT, w.PART, part_words(d));
-        else
-          k_b_attn_w<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(w.rargs, w.drows,
-                                                                              w.items, l);
+        if (tiled) {
+          launch_attn_tile(m, nb0, w.items, n_items0, l);
+          if (nb1 != nb0) launch_attn_tile(m, nb1, w.items + n_items0, (uint32_t)items.size() - n_items0, l);
+        } else {
+          k_b_attn_w<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(w.rargs, w.drows, w.items, l);
+        }
       }
-      k_b_comb<<<dim3(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK), 256, 0, s>>>(
-          d, w.drows, w.PART, part_words(d), w.XQ);
+      const dim3 comb_grid(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK);
+      if (tiled)
+        k_b_comb<true><<<comb_grid, 256, 0, s>>>(d, w.drows, w.PART, part_words(d), w.XQ);
+      else
+        k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, w.drows, w.PART, part_words(d), w.XQ);
     }
     {
       ProfSpan ps(m, 0, 2.0 * d.h * d.q * n);
