@@ -72,7 +72,40 @@ __global__ void k_to_panel(const float* __restrict__ src0, const float* __restri
 enum GemmOut : uint32_t {
   GO_PLAIN = 0,  // Y[b][o] = y
   GO_RESID = 1,  // Y[b][o] = Y[b][o] + y   (the residual stream, in place; also into panel P)
-  GO_TAG = 2,    // T[b][o] = tag(gen[b], scale[b] * y)  (tagged logits)
+  GO_TAG = 2,    // T[b][o] = tag(gen[b], inv[b] * y)  (tagged logits)
+  // Outputs of a pair of rows, W the pairs' first rows and their partners
+  // stacked in blocks of `blk` row tiles (see GemmOutArgs):
+  GO_ACT = 3,    // P[b][o] = act(gate * inv[b]) * (up * inv[b])  (phase_gu)
+  GO_QKV = 4,    // rotated q to qf[b][q], k and v to the row's cache (phase_qkv)
+};
+constexpr bool gemm_pairs(uint32_t out) { return out == GO_ACT || out == GO_QKV; }
+
+// One row of a batch: the cache it extends, at which position and
+// generation base, with which token.
+struct BRow {
+  float* kc;
+  float* vc;
+  uint32_t cap, pos, tick, token;
+};
+
+// Where a product goes. A pair product's row tiles come in pairs: pair p is
+// tile p / blk * 2 * blk + p % blk and the one blk later (gate and up rows:
+// blk = all the gate tiles; the two halves of each rotated head: blk = half a
+// head).
+struct GemmOutArgs {
+  float* Y;             // GO_PLAIN, GO_RESID, GO_TAG (u64 words): [B][ldy]
+  uint32_t ldy;
+  float* P;             // GO_RESID (K = M), GO_ACT (K = M / 2): panel of the output
+  const float* inv;     // GO_TAG, GO_ACT, GO_QKV: the rows' 1/rms
+  const uint32_t* gen;  // GO_TAG
+  uint32_t blk;         // pair products
+  uint32_t act;         // GO_ACT
+  // GO_QKV
+  const BRow* rows;
+  const float2* rope;
+  const float* bias;    // or null
+  float* qf;
+  uint32_t l, hd, half, nh, nkv, kvs;
 };
 
 // 16 bytes at a byte offset from a wave-uniform base.
@@ -121,21 +154,24 @@ __host__ __device__ constexpr int gemm_depth(int tr, int tc) { return tr * tc >=
 template <int TR, int TC, uint32_t OUT, bool PARTIAL>
 __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, uint32_t M, uint32_t K,
                                                  const float* __restrict__ Xp, uint32_t B,
-                                                 float* __restrict__ Y, uint32_t ldy,
-                                                 const float* __restrict__ scale,
-                                                 const uint32_t* __restrict__ gen,
-                                                 float* __restrict__ P) {
+                                                 const GemmOutArgs out) {
   constexpr int D = gemm_depth(TR, TC), NT = TR * TC;
   __shared__ float4 sub[4 * NT * WAVE];  // [quarter][tile][lane]
   // The wave index is uniform: scalar registers for it and the tile bases.
   const uint32_t q = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
   const uint32_t nch = panel_chunks(K), nrt = (M + 15) / 16, nct = (B + 15) / 16;
   const TaskXY task = gemm_task(blockIdx.x, gridDim.x, (nrt + TR - 1) / TR, (nct + TC - 1) / TC, GEMM_BAND / TC);
-  // Tiles past the last one load a real tile, never used.
+  // Row tile r of the task. Tiles past the last one load a real tile, never
+  // used.
+  auto row_tile = [&](uint32_t r) {
+    if (!gemm_pairs(OUT)) return TR * task.x + r;
+    const uint32_t p = TR / 2 * task.x + r % (TR / 2);
+    return p / out.blk * 2 * out.blk + p % out.blk + (r < TR / 2 ? 0 : out.blk);
+  };
   const float *wa[TR], *xb[TC];
 #pragma unroll
   for (int r = 0; r < TR; ++r)
-    wa[r] = Wp + (size_t)min(TR * task.x + r, nrt - 1) * nch * PANEL_TILE + q * 256;
+    wa[r] = Wp + (size_t)min(row_tile(r), nrt - 1) * nch * PANEL_TILE + q * 256;
 #pragma unroll
   for (int c = 0; c < TC; ++c)
     xb[c] = Xp + (size_t)min(TC * task.y + c, nct - 1) * nch * PANEL_TILE + q * 256;
@@ -166,6 +202,57 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
   };
 #pragma unroll
   for (int d = 0; d < D; ++d) load(d);
+  // What the outputs need from memory: the small tasks request it here, so
+  // that its latency does not follow the main loop's (18 steps of 7 sessions,
+  // 135M shape: 29.3 -> 28.8 ms); the large ones after the loop (1 % faster
+  // there: registers, and another workgroup's MFMAs to wait behind).
+  constexpr bool EARLY = NT <= 2;
+  // Pair products: one pair per wave, pair p, column bc of each lane.
+  const uint32_t p = TR / 2 * task.x + q / TC, pbc = (TC * task.y + q % TC) * 16 + lane % 16;
+  const bool pair_out = gemm_pairs(OUT) && q < NT / 2 && 2 * p < nrt && pbc < B;
+  float iv = 0.0f;
+  BRow row;
+  uint32_t hb = 0, hi = 0;  // head block, first of the lane's four elements in its first half
+  float4 cs[2];
+  auto pair_inputs = [&]() {
+    if (!pair_out) return;
+    iv = out.inv[pbc];
+    if (OUT == GO_QKV) {
+      row = out.rows[pbc];
+      hb = p / out.blk;
+      hi = p % out.blk * 16 + 4 * (lane / 16);
+      const float4* rp = reinterpret_cast<const float4*>(out.rope + (size_t)row.pos * out.half + hi);
+      cs[0] = rp[0];
+      cs[1] = rp[1];
+    }
+  };
+  // Other products: tiles q, q + 4, ...; the residual's old values.
+  constexpr int NO = gemm_pairs(OUT) ? 1 : (NT + 3) / 4;
+  struct OutAt {
+    uint32_t bc, o;
+    bool on, vec;  // in range; four outputs inside M and 16-byte aligned
+  };
+  auto out_at = [&](int k) {
+    const uint32_t t = 4 * k + q, T = TR * task.x + t / TC;
+    OutAt r;
+    r.bc = (TC * task.y + t % TC) * 16 + lane % 16;
+    r.o = T * 16 + 4 * (lane / 16);
+    r.on = t < NT && T < nrt && r.bc < B;
+    r.vec = OUT != GO_TAG && r.o + 4 <= M && (((size_t)r.bc * out.ldy + r.o) & 3) == 0;
+    return r;
+  };
+  float4 old[NO];
+  auto old_values = [&]() {
+#pragma unroll
+    for (int k = 0; k < NO; ++k) {
+      const OutAt r = out_at(k);
+      if (r.on && r.vec) old[k] = *reinterpret_cast<const float4*>(out.Y + (size_t)r.bc * out.ldy + r.o);
+    }
+  };
+  if (EARLY) {
+    if (gemm_pairs(OUT)) pair_inputs();
+    if (OUT == GO_RESID) old_values();
+  }
   const uint32_t nfull = K / 64;
   uint32_t i = 0;
   for (; i + D <= nfull; i += D) {
@@ -197,32 +284,79 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
       sub[(q * NT + r * TC + c) * WAVE + lane] = make_float4(t[0], t[1], t[2], t[3]);
     }
   __syncthreads();
-#pragma unroll
-  for (int t0 = 0; t0 < NT; t0 += 4) {
-    const uint32_t t = t0 + q;  // this wave's tile
-    if (t >= NT) break;
-    const uint32_t T = TR * task.x + t / TC, bc = (TC * task.y + t % TC) * 16 + lane % 16;
-    const uint32_t o = T * 16 + 4 * (lane / 16);
-    if (T >= nrt || bc >= B) continue;
+  // Tile t's outputs: rows 4*(lane/16) .. +3, column lane % 16.
+  auto total = [&](uint32_t t, float (&v)[4]) {
     float4 s[4];
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) s[k] = sub[(k * NT + t) * WAVE + lane];
-    const float v[4] = {(s[0].x + s[1].x) + (s[2].x + s[3].x), (s[0].y + s[1].y) + (s[2].y + s[3].y),
-                        (s[0].z + s[1].z) + (s[2].z + s[3].z), (s[0].w + s[1].w) + (s[2].w + s[3].w)};
-    const size_t at = (size_t)bc * ldy + o;
+    v[0] = (s[0].x + s[1].x) + (s[2].x + s[3].x);
+    v[1] = (s[0].y + s[1].y) + (s[2].y + s[3].y);
+    v[2] = (s[0].z + s[1].z) + (s[2].z + s[3].z);
+    v[3] = (s[0].w + s[1].w) + (s[2].w + s[3].w);
+  };
+  if constexpr (gemm_pairs(OUT)) {
+    static_assert(NT / 2 <= 4 && TR % 2 == 0, "a pair of tiles per wave");
+    if (!pair_out) return;
+    if (!EARLY) pair_inputs();
+    float y0[4], y1[4];
+    total(q, y0);
+    total(NT / 2 + q, y1);
+    if (OUT == GO_ACT) {
+      const uint32_t nchp = panel_chunks(M / 2), o = p * 16 + 4 * (lane / 16);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        out.P[panel_at(pbc, o + j, nchp)] = act_fn(y0[j] * iv, out.act) * (y1[j] * iv);
+    } else {
+      // phase_qkv's epilogue (qkv_epi_pair's expressions) of four pairs.
+      const bool rotated = hb < out.nh + out.nkv;
+      const float* bias = out.bias ? out.bias + hb * out.hd + hi : nullptr;
+      float a0[4], a1[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float e0 = bias ? bias[j] : 0.0f, e1 = bias ? bias[out.half + j] : 0.0f;
+        y0[j] = y0[j] * iv + e0;
+        y1[j] = y1[j] * iv + e1;
+        a0[j] = y0[j];
+        a1[j] = y1[j];
+        if (rotated) {
+          const float cx = (&cs[j / 2].x)[j % 2 * 2], cy = (&cs[j / 2].x)[j % 2 * 2 + 1];
+          a0[j] = y0[j] * cx - y1[j] * cy;
+          a1[j] = y1[j] * cx + y0[j] * cy;
+        }
+      }
+      float* dst;
+      if (hb < out.nh) {
+        dst = out.qf + ((size_t)pbc * out.nh + hb) * out.hd;
+      } else {
+        const uint32_t gi = rotated ? hb - out.nh : hb - out.nh - out.nkv;
+        dst = (rotated ? row.kc : row.vc) + (((size_t)out.l * out.nkv + gi) * row.cap + row.pos) * out.kvs;
+      }
+      *reinterpret_cast<float4*>(dst + hi) = make_float4(a0[0], a0[1], a0[2], a0[3]);
+      *reinterpret_cast<float4*>(dst + hi + out.half) = make_float4(a1[0], a1[1], a1[2], a1[3]);
+    }
+    return;
+  }
+  if (!EARLY && OUT == GO_RESID) old_values();
+#pragma unroll
+  for (int k = 0; k < NO; ++k) {
+    const OutAt r = out_at(k);
+    if (!r.on) continue;
+    const uint32_t bc = r.bc, o = r.o;
+    float v[4];
+    total(4 * k + q, v);
+    float* Y = out.Y;
+    const size_t at = (size_t)bc * out.ldy + o;
     const uint32_t nchp = panel_chunks(M);  // the residual's panel: K = M
-    if (OUT != GO_TAG && o + 4 <= M && (at & 3) == 0) {
-      float4* y4 = reinterpret_cast<float4*>(Y + at);
+    if (r.vec) {
       float4 w = make_float4(v[0], v[1], v[2], v[3]);
       if (OUT == GO_RESID) {
-        const float4 old = *y4;
-        w = make_float4(old.x + v[0], old.y + v[1], old.z + v[2], old.w + v[3]);
-        P[panel_at(bc, o, nchp)] = w.x;
-        P[panel_at(bc, o + 1, nchp)] = w.y;
-        P[panel_at(bc, o + 2, nchp)] = w.z;
-        P[panel_at(bc, o + 3, nchp)] = w.w;
+        w = make_float4(old[k].x + v[0], old[k].y + v[1], old[k].z + v[2], old[k].w + v[3]);
+        out.P[panel_at(bc, o, nchp)] = w.x;
+        out.P[panel_at(bc, o + 1, nchp)] = w.y;
+        out.P[panel_at(bc, o + 2, nchp)] = w.z;
+        out.P[panel_at(bc, o + 3, nchp)] = w.w;
       }
-      *y4 = w;
+      *reinterpret_cast<float4*>(Y + at) = w;
       continue;
     }
 #pragma unroll
@@ -233,9 +367,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
       } else if (OUT == GO_RESID) {
         const float w = Y[at + j] + v[j];
         Y[at + j] = w;
-        P[panel_at(bc, o + j, nchp)] = w;
+        out.P[panel_at(bc, o + j, nchp)] = w;
       } else {
-        reinterpret_cast<u64*>(Y)[at + j] = ((u64)gen[bc] << 32) | (u64)__float_as_uint(scale[bc] * v[j]);
+        reinterpret_cast<u64*>(Y)[at + j] =
+            ((u64)out.gen[bc] << 32) | (u64)__float_as_uint(out.inv[bc] * v[j]);
       }
     }
   }
@@ -258,14 +393,6 @@ __device__ __forceinline__ float rms_row_inv(const float* __restrict__ x, uint32
 }
 
 // ------------------------------------------------------------- rows
-
-// One row of a batch: the cache it extends, at which position and
-// generation base, with which token.
-struct BRow {
-  float* kc;
-  float* vc;
-  uint32_t cap, pos, tick, token;
-};
 
 // X[b] = E[token_b] (model.rs:428), and its panel XP; token_b from dtok
 // (device, e.g. just sampled) when given, else from the row.
@@ -333,10 +460,8 @@ __device__ __forceinline__ void qkv_epi_cache(const Dims& d, const BRow& r, uint
   row[i + d.half] = v.y;
 }
 
-// QKV epilogue per (row, pair): k, v into the row's cache at its position;
-// for the attention, q/k/v words tagged, or (TILED: it reads k and v from the
-// cache) the queries alone as floats [row][q].
-template <bool TILED>
+// QKV epilogue per (row, pair) for the attention items of rows that do not
+// run as tiles: q/k/v words tagged; k, v into the row's cache at its position.
 __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict__ rows, uint32_t l,
                             const float* __restrict__ Y, uint32_t ldy, const float* __restrict__ inv,
                             u64* __restrict__ qkvt, uint32_t ldq) {
@@ -348,17 +473,10 @@ __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict_
   const uint32_t hb = p / d.half, i = p - hb * d.half;
   const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
   const float2 v = qkv_epi_pair(*ap, l, r.pos, b, hb, i, Y, ldy, inv[b]);
-  if (hb >= d.nh) qkv_epi_cache(d, r, l, hb, i, v);
-  if (TILED) {
-    if (hb >= d.nh) return;
-    float* qf = reinterpret_cast<float*>(qkvt) + (size_t)b * d.q;
-    qf[r0] = v.x;
-    qf[r1] = v.y;
-    return;
-  }
   const u64 g = (u64)gen_of(d, r.tick, l, PH_QKV) << 32;
   qkvt[(size_t)b * ldq + r0] = g | __float_as_uint(v.x);
   qkvt[(size_t)b * ldq + r1] = g | __float_as_uint(v.y);
+  if (hb >= d.nh) qkv_epi_cache(d, r, l, hb, i, v);
 }
 
 // LDS of the batched kernels that run one-token functions: no weight
@@ -832,8 +950,8 @@ __global__ __launch_bounds__(256) void k_b_comb(const Dims d, const BRow* __rest
   }
 }
 
-// g = act(gate * inv) * (up * inv) (phase_gu), into the panel GP; Y holds
-// gate rows then up rows.
+// g = act(gate * inv) * (up * inv) (phase_gu), into the panel GP, where the
+// product cannot do it itself (GO_ACT: whole 16-row tiles of gate rows); Y holds gate rows then up rows.
 __global__ void k_b_act(const float* __restrict__ Y, uint32_t ldy, const float* __restrict__ inv,
                         uint32_t ff, uint32_t act, float* __restrict__ GP) {
   const uint32_t b = blockIdx.y;

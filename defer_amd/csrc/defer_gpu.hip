@@ -1912,10 +1912,9 @@ static int ensure_panels(defer_gpu_model* m) {
 
 template <int TR, int TC, uint32_t OUT, bool PARTIAL = false>
 static void launch_gemm_tile(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
-                             uint32_t B, float* Y, uint32_t ldy, const float* scale,
-                             const uint32_t* gen, float* P) {
+                             uint32_t B, const GemmOutArgs& out) {
   const uint32_t n = ((M + 16 * TR - 1) / (16 * TR)) * ((B + 16 * TC - 1) / (16 * TC));
-  k_gemm<TR, TC, OUT, PARTIAL><<<n, 256, 0, s>>>(Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+  k_gemm<TR, TC, OUT, PARTIAL><<<n, 256, 0, s>>>(Wp, M, K, Xp, B, out);
 }
 // The task shape of a product: the one whose busiest CU has the least work,
 // counted as tasks per CU (rounded up) x tiles per task x the cost of a tile
@@ -1924,36 +1923,25 @@ static void launch_gemm_tile(hipStream_t s, const float* Wp, uint32_t M, uint32_
 // 4x2, 93, 86 and 76 for 3072 x 576 by 2048 rows). E.g. 576 x 1536: 2048
 // rows 44.2 us at 4x2 (2.25 tasks per CU), 38.4 at 2x2; 301 rows 15.0, 10.0,
 // and 9.2 at 1x1. Every output is computed the same way in every shape.
-// A K that ends inside a chunk takes the 1x1 tasks.
+// A K that ends inside a chunk takes the smallest tasks; pair products need
+// two row tiles.
 template <uint32_t OUT>
-static void launch_gemm_out(hipStream_t s, const float* Wp, uint32_t M, uint32_t K, const float* Xp,
-                            uint32_t B, float* Y, uint32_t ldy, const float* scale,
-                            const uint32_t* gen, uint32_t ncu, float* P) {
-  if (K % 64 != 0)
-    return launch_gemm_tile<1, 1, OUT, true>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+static void launch_gemm(hipStream_t s, uint32_t ncu, const float* Wp, uint32_t M, uint32_t K,
+                        const float* Xp, uint32_t B, const GemmOutArgs& out) {
+  constexpr bool PAIRS = gemm_pairs(OUT);
+  if (K % 64 != 0) return launch_gemm_tile<PAIRS ? 2 : 1, 1, OUT, true>(s, Wp, M, K, Xp, B, out);
   auto cost = [&](uint32_t tr, uint32_t tc, float per_tile) {
     const uint32_t n = ((M + 16 * tr - 1) / (16 * tr)) * ((B + 16 * tc - 1) / (16 * tc));
     return (float)((n + ncu - 1) / ncu * tr * tc) * per_tile;
   };
   const float c[4] = {cost(4, 2, 1.0f), cost(2, 2, 1.06f), cost(2, 1, 1.15f), cost(1, 1, 1.3f)};
-  switch (std::min_element(c, c + 4) - c) {
-    case 0: return launch_gemm_tile<4, 2, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
-    case 1: return launch_gemm_tile<2, 2, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
-    case 2: return launch_gemm_tile<2, 1, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
-    default: return launch_gemm_tile<1, 1, OUT>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, P);
+  switch (std::min_element(c, c + (PAIRS ? 3 : 4)) - c) {
+    case 0: return launch_gemm_tile<4, 2, OUT>(s, Wp, M, K, Xp, B, out);
+    case 1: return launch_gemm_tile<2, 2, OUT>(s, Wp, M, K, Xp, B, out);
+    case 2: return launch_gemm_tile<2, 1, OUT>(s, Wp, M, K, Xp, B, out);
+    default: break;
   }
-}
-// P: GO_RESID's panel of the updated rows (K = M).
-static void launch_gemm(hipStream_t s, uint32_t ncu, uint32_t out, const float* Wp, uint32_t M,
-                        uint32_t K, const float* Xp, uint32_t B, float* Y, uint32_t ldy,
-                        const float* scale = nullptr, const uint32_t* gen = nullptr,
-                        float* P = nullptr) {
-  if (out == GO_PLAIN)
-    launch_gemm_out<GO_PLAIN>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
-  else if (out == GO_RESID)
-    launch_gemm_out<GO_RESID>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
-  else
-    launch_gemm_out<GO_TAG>(s, Wp, M, K, Xp, B, Y, ldy, scale, gen, ncu, P);
+  if constexpr (!PAIRS) launch_gemm_tile<1, 1, OUT>(s, Wp, M, K, Xp, B, out);
 }
 
 // Timing of one launch (profiling on): events recorded around it on the
@@ -2132,24 +2120,47 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     HIP_TRY(hipMemcpyAsync(w.lgen, lgen.data(), nl * sizeof(uint32_t), hipMemcpyHostToDevice, s));
   }
   if (!deferred) k_begin<<<1, 1, 0, s>>>(w.st);
-  const uint32_t ldy = batch_ldy(d);
+  const uint32_t ldy = batch_ldy(d), ncu = m->gemm_ncu;
+  // The QKV and gate/up products write what their consumers read -- rotated
+  // queries and cache rows (tiled attention: head sizes 64 and 128, so both
+  // halves of a head are whole tiles), the activation's panel (where the
+  // gate rows are whole tiles). A 301-row layer of the 135M shape drops from 8
+  // launches to 6, a 2048-row one saves the 25 MB of gate and up rows.
+  const bool act_out = d.ff % 16 == 0;
   k_b_embed<<<n, 256, 0, s>>>(w.drows, dtok, m->embed, d.h, w.X, w.XP);
   k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   for (uint32_t l = 0; l < d.L; ++l) {
+    GemmOutArgs o{};
+    o.Y = w.Y;
+    o.ldy = ldy;
+    o.inv = w.INV;
     {
       ProfSpan ps(m, 0, 2.0 * d.qkv_rows * d.h * n);
-      launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_qkv[l], d.qkv_rows, d.h, w.XP, n, w.Y, ldy);
+      if (tiled) {
+        o.blk = d.half / 16;
+        o.rows = w.drows;
+        o.rope = m->rope;
+        o.bias = m->layers[l].bqkv;
+        o.qf = reinterpret_cast<float*>(w.QKVT);
+        o.l = l;
+        o.hd = d.hd;
+        o.half = d.half;
+        o.nh = d.nh;
+        o.nkv = d.nkv;
+        o.kvs = d.kvs;
+        launch_gemm<GO_QKV>(s, ncu, m->p_qkv[l], d.qkv_rows, d.h, w.XP, n, o);
+      } else {
+        launch_gemm<GO_PLAIN>(s, ncu, m->p_qkv[l], d.qkv_rows, d.h, w.XP, n, o);
+      }
     }
     if (fused) {
       ProfSpan ps(m, 1, attn_flop);
       k_b_attn_f<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(
           w.rargs, w.drows, w.items, l, w.Y, ldy, w.INV, w.CNT, w.XQ);
     } else {
-      const dim3 epi_grid((d.qkv_rows / 2 + 255) / 256, n);
-      if (tiled)
-        k_b_qkv_epi<true><<<epi_grid, 256, 0, s>>>(w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
-      else
-        k_b_qkv_epi<false><<<epi_grid, 256, 0, s>>>(w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
+      if (!tiled)
+        k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
+            w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
       {
         ProfSpan ps(m, 1, attn_flop);
         if (tiled) {
@@ -2165,21 +2176,30 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       else
         k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, w.drows, w.PART, part_words(d), w.XQ);
     }
+    GemmOutArgs x{};  // the residual rows and their panel
+    x.Y = w.X;
+    x.ldy = d.h;
+    x.P = w.XP;
     {
       ProfSpan ps(m, 0, 2.0 * d.h * d.q * n);
-      launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_o[l], d.h, d.q, w.XQ, n, w.X, d.h, nullptr, nullptr,
-                  w.XP);
+      launch_gemm<GO_RESID>(s, ncu, m->p_o[l], d.h, d.q, w.XQ, n, x);
     }
     k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
     {
       ProfSpan ps(m, 0, 2.0 * 2 * d.ff * d.h * n);
-      launch_gemm(s, m->gemm_ncu, GO_PLAIN, m->p_gu[l], 2 * d.ff, d.h, w.XP, n, w.Y, ldy);
+      o.P = w.XQ;
+      o.blk = d.ff / 16;
+      o.act = d.act;
+      if (act_out)
+        launch_gemm<GO_ACT>(s, ncu, m->p_gu[l], 2 * d.ff, d.h, w.XP, n, o);
+      else
+        launch_gemm<GO_PLAIN>(s, ncu, m->p_gu[l], 2 * d.ff, d.h, w.XP, n, o);
     }
-    k_b_act<<<dim3((d.ff + 255) / 256, n), 256, 0, s>>>(w.Y, ldy, w.INV, d.ff, d.act, w.XQ);
+    if (!act_out)
+      k_b_act<<<dim3((d.ff + 255) / 256, n), 256, 0, s>>>(w.Y, ldy, w.INV, d.ff, d.act, w.XQ);
     {
       ProfSpan ps(m, 0, 2.0 * d.h * d.ff * n);
-      launch_gemm(s, m->gemm_ncu, GO_RESID, m->p_d[l], d.h, d.ff, w.XQ, n, w.X, d.h, nullptr, nullptr,
-                  w.XP);
+      launch_gemm<GO_RESID>(s, ncu, m->p_d[l], d.h, d.ff, w.XQ, n, x);
     }
     if (l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   }
@@ -2187,8 +2207,12 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     k_b_final<<<nl, 64, 0, s>>>(w.X, w.sel, d.h, m->norm, d.eps, w.XQ, w.LINV);
     {
       ProfSpan ps(m, 0, 2.0 * d.V * d.h * nl);
-      launch_gemm(s, m->gemm_ncu, GO_TAG, m->p_lm, d.V, d.h, w.XQ, nl, reinterpret_cast<float*>(w.LOGT), d.V,
-                  w.LINV, w.lgen);
+      GemmOutArgs o{};
+      o.Y = reinterpret_cast<float*>(w.LOGT);
+      o.ldy = d.V;
+      o.inv = w.LINV;
+      o.gen = w.lgen;
+      launch_gemm<GO_TAG>(s, ncu, m->p_lm, d.V, d.h, w.XQ, nl, o);
     }
     k_b_chunkmax<<<dim3((d.nvc + 4 * CM_CPW - 1) / (4 * CM_CPW), nl), 256, 0, s>>>(d, w.LOGT, w.lgen, w.VMAX,
                                                                                    w.VARG, nl);

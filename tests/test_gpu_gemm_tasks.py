@@ -2,7 +2,8 @@
 
 The task shape of a product (4x2, 2x2, 2x1 or 1x1 tiles of 16) follows from the
 rows, the columns and the compute units the launch is shaped for; every shape
-must give each output the one-token order's bits. The compute-unit count is
+must give each output the one-token order's bits, whatever the product writes
+(plain rows, the residual, logits, rotated queries and cache rows, activations). The compute-unit count is
 forced so that each shape is chosen, at row counts on both sides of the tile
 edges, with dimensions that are not whole tiles or whole 64-element chunks.
 """
@@ -15,18 +16,21 @@ from defer_amd import synthetic
 pytestmark = pytest.mark.gpu
 
 SHAPES = {
-    # hidden, intermediate, heads, kv heads, head_dim, vocabulary
-    "whole-chunks": (128, 192, 4, 2, 32, 250),
-    "odd-tiles": (192, 320, 3, 1, 64, 331),
-    "partial-chunks": (96, 200, 6, 2, 16, 77),
+    # hidden, intermediate, heads, kv heads, head_dim, vocabulary, activation, biases
+    "whole-chunks": (128, 192, 4, 2, 32, 250, 0, 0),
+    "odd-tiles": (192, 320, 3, 1, 64, 331, 0, 0),
+    "biases-gelu": (128, 144, 2, 1, 128, 90, 1, 1),
+    "partial-chunks": (96, 200, 6, 2, 16, 77, 0, 1),
+    "partial-chunks-tiled": (96, 208, 3, 1, 64, 77, 0, 1),
 }
 
 
 @pytest.mark.parametrize("shape", SHAPES)
 @pytest.mark.parametrize("cus", [1, 3, 16, 0])
 def test_rows_equal_single_forwards_for_every_task_shape(shape, cus):
-    h, ff, nh, nkv, hd, V = SHAPES[shape]
-    cfg = synthetic._cfg(V, h, ff, 2, nh, nkv, hd, 10000.0, False, max_seq=256)
+    h, ff, nh, nkv, hd, V, act, bias = SHAPES[shape]
+    cfg = synthetic._cfg(V, h, ff, 2, nh, nkv, hd, 10000.0, False, max_seq=256,
+                         act=act, bias=bias)
     m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 11, std=0.08))
     m.set_grid(0, cus)
     rng = np.random.Generator(np.random.PCG64(cus))
