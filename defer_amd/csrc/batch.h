@@ -100,6 +100,8 @@ struct GemmOutArgs {
   const uint32_t* gen;  // GO_TAG
   uint32_t blk;         // pair products
   uint32_t act;         // GO_ACT
+  const float* X;       // GO_ACT, at most 16 rows: form 1/rms from the rows [B][K] instead of inv
+  float eps;
   // GO_QKV
   const BRow* rows;
   const float2* rope;
@@ -107,6 +109,39 @@ struct GemmOutArgs {
   float* qf;
   uint32_t l, hd, half, nh, nkv, kvs;
 };
+
+// 1/rms of N rows of n floats, by one wave: lane partials over the float4s
+// at 4*lane + 256*i (i ascending), then the wave tree. The rows' loads and
+// chains run side by side.
+template <int N>
+__device__ __forceinline__ void rms_rows_inv(const float* const (&x)[N], uint32_t n, float eps,
+                                             uint32_t lane, float (&inv)[N]) {
+  float ss[N];
+#pragma unroll
+  for (int r = 0; r < N; ++r) ss[r] = 0.0f;
+  for (uint32_t j = lane * 4; j < n; j += 256) {
+    float4 v[N];
+#pragma unroll
+    for (int r = 0; r < N; ++r) v[r] = *reinterpret_cast<const float4*>(x[r] + j);
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+      ss[r] = fmaf(v[r].x, v[r].x, ss[r]);
+      ss[r] = fmaf(v[r].y, v[r].y, ss[r]);
+      ss[r] = fmaf(v[r].z, v[r].z, ss[r]);
+      ss[r] = fmaf(v[r].w, v[r].w, ss[r]);
+    }
+  }
+  wave_sum_n<N>(ss);
+#pragma unroll
+  for (int r = 0; r < N; ++r) inv[r] = 1.0f / sqrtf(ss[r] / (float)n + eps);
+}
+__device__ __forceinline__ float rms_row_inv(const float* __restrict__ x, uint32_t n, float eps,
+                                             uint32_t lane) {
+  const float* const p[1] = {x};
+  float inv[1];
+  rms_rows_inv(p, n, eps, lane, inv);
+  return inv[0];
+}
 
 // 16 bytes at a byte offset from a wave-uniform base.
 __device__ __forceinline__ float4 ldg4_at(const float* base, uint32_t byte_off) {
@@ -165,8 +200,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
   // used.
   auto row_tile = [&](uint32_t r) {
     if (!gemm_pairs(OUT)) return TR * task.x + r;
-    const uint32_t p = TR / 2 * task.x + r % (TR / 2);
-    return p / out.blk * 2 * out.blk + p % out.blk + (r < TR / 2 ? 0 : out.blk);
+    constexpr uint32_t HT = TR >= 2 ? TR / 2 : 1;
+    const uint32_t p = HT * task.x + r % HT;
+    return p / out.blk * 2 * out.blk + p % out.blk + (r < HT ? 0 : out.blk);
   };
   const float *wa[TR], *xb[TC];
 #pragma unroll
@@ -216,7 +252,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
   float4 cs[2];
   auto pair_inputs = [&]() {
     if (!pair_out) return;
-    iv = out.inv[pbc];
+    if (!(OUT == GO_ACT && out.X)) iv = out.inv[pbc];
     if (OUT == GO_QKV) {
       row = out.rows[pbc];
       hb = p / out.blk;
@@ -249,6 +285,18 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
       if (r.on && r.vec) old[k] = *reinterpret_cast<const float4*>(out.Y + (size_t)r.bc * out.ldy + r.o);
     }
   };
+  // Few rows: every workgroup forms their 1/rms itself (wave q: rows 4q ..),
+  // a third more bytes from L2 than its operands but no launch of its own
+  // before this product: 2.6 us per layer of 7 rows (135M shape).
+  __shared__ float row_inv[16];
+  if (OUT == GO_ACT && TC == 1 && out.X) {
+    const float* xr[4];
+    float ri[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) xr[u] = out.X + (size_t)min(4 * q + u, B - 1) * K;
+    rms_rows_inv(xr, K, out.eps, lane, ri);
+    if (lane < 4) row_inv[4 * q + lane] = lane == 0 ? ri[0] : lane == 1 ? ri[1] : lane == 2 ? ri[2] : ri[3];
+  }
   if (EARLY) {
     if (gemm_pairs(OUT)) pair_inputs();
     if (OUT == GO_RESID) old_values();
@@ -302,12 +350,13 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
     total(q, y0);
     total(NT / 2 + q, y1);
     if (OUT == GO_ACT) {
+      if (TC == 1 && out.X) iv = row_inv[lane % 16];
       const uint32_t nchp = panel_chunks(M / 2), o = p * 16 + 4 * (lane / 16);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         out.P[panel_at(pbc, o + j, nchp)] = act_fn(y0[j] * iv, out.act) * (y1[j] * iv);
     } else {
-      // phase_qkv's epilogue (qkv_epi_pair's expressions) of four pairs.
+      // phase_qkv's epilogue (QkvEpiPair's expressions) of four pairs.
       const bool rotated = hb < out.nh + out.nkv;
       const float* bias = out.bias ? out.bias + hb * out.hd + hi : nullptr;
       float a0[4], a1[4];
@@ -376,22 +425,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const float* __restrict__ Wp, u
   }
 }
 
-// 1/rms of one row of n floats, by one wave: lane partials over the float4s
-// at 4*lane + 256*i (i ascending), then the wave tree.
-__device__ __forceinline__ float rms_row_inv(const float* __restrict__ x, uint32_t n, float eps,
-                                             uint32_t lane) {
-  float ss = 0.0f;
-  for (uint32_t j = lane * 4; j < n; j += 256) {
-    const float4 v = *reinterpret_cast<const float4*>(x + j);
-    ss = fmaf(v.x, v.x, ss);
-    ss = fmaf(v.y, v.y, ss);
-    ss = fmaf(v.z, v.z, ss);
-    ss = fmaf(v.w, v.w, ss);
-  }
-  ss = wave_sum(ss);
-  return 1.0f / sqrtf(ss / (float)n + eps);
-}
-
 // ------------------------------------------------------------- rows
 
 // X[b] = E[token_b] (model.rs:428), and its panel XP; token_b from dtok
@@ -419,35 +452,37 @@ __global__ __launch_bounds__(256) void k_b_rms(const float* __restrict__ X, uint
 }
 
 // QKV epilogue of the one-token path (phase_qkv) for pair i of head block
-// hb of batch row b: the product's rows r0 = hb * hd + i and r1 = r0 + half
-// (from Y), scaled by the row's 1/rms, biased, and rotated (q and k heads)
-// -- phase_qkv's expressions.
-__device__ __forceinline__ float2 qkv_epi_pair(const Args& a, uint32_t l, uint32_t pos, uint32_t b,
-                                               uint32_t hb, uint32_t i, const float* __restrict__ Y,
-                                               uint32_t ldy, float iv) {
-  const Dims& d = a.d;
-  const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
-  float4 e = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
-  if (hb < d.nh + d.nkv) {
-    const float2 cs = a.rope[(size_t)pos * d.half + i];
-    e.x = cs.x;
-    e.y = cs.y;
+// hb of a batch row at position pos: the product's rows r0 = hb * hd + i and
+// r1 = r0 + half (y: the row's product), scaled by the row's 1/rms, biased,
+// and rotated (q and k heads) -- phase_qkv's expressions. load() reads what
+// it needs from memory, value() computes.
+struct QkvEpiPair {
+  float y0, y1;
+  float4 e;
+  bool rotated;
+  __device__ __forceinline__ void load(const Dims& d, const float2* rope, const float* bias, uint32_t pos,
+                                       uint32_t hb, uint32_t i, const float* __restrict__ y) {
+    const uint32_t r0 = hb * d.hd + i;
+    y0 = y[r0];
+    y1 = y[r0 + d.half];
+    e = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+    rotated = hb < d.nh + d.nkv;
+    if (rotated) {
+      const float2 cs = rope[(size_t)pos * d.half + i];
+      e.x = cs.x;
+      e.y = cs.y;
+    }
+    if (bias) {
+      e.z = bias[r0];
+      e.w = bias[r0 + d.half];
+    }
   }
-  const float* bias = a.layers[l].bqkv;
-  if (bias) {
-    e.z = bias[r0];
-    e.w = bias[r0 + d.half];
+  __device__ __forceinline__ float2 value(float iv) const {
+    const float z0 = y0 * iv + e.z, z1 = y1 * iv + e.w;
+    if (!rotated) return make_float2(z0, z1);
+    return make_float2(z0 * e.x - z1 * e.y, z1 * e.x + z0 * e.y);
   }
-  float y0 = Y[(size_t)b * ldy + r0], y1 = Y[(size_t)b * ldy + r1];
-  y0 = y0 * iv + e.z;
-  y1 = y1 * iv + e.w;
-  float a0 = y0, a1 = y1;
-  if (hb < d.nh + d.nkv) {
-    a0 = y0 * e.x - y1 * e.y;
-    a1 = y1 * e.x + y0 * e.y;
-  }
-  return make_float2(a0, a1);
-}
+};
 
 // k (hb < nh + nkv) or v rows of head block hb into the row's cache at its
 // position (model.rs:466-467).
@@ -472,7 +507,9 @@ __global__ void k_b_qkv_epi(const Args* __restrict__ ap, const BRow* __restrict_
   const BRow r = rows[b];
   const uint32_t hb = p / d.half, i = p - hb * d.half;
   const uint32_t r0 = hb * d.hd + i, r1 = r0 + d.half;
-  const float2 v = qkv_epi_pair(*ap, l, r.pos, b, hb, i, Y, ldy, inv[b]);
+  QkvEpiPair ep;
+  ep.load(d, ap->rope, ap->layers[l].bqkv, r.pos, hb, i, Y + (size_t)b * ldy);
+  const float2 v = ep.value(inv[b]);
   const u64 g = (u64)gen_of(d, r.tick, l, PH_QKV) << 32;
   qkvt[(size_t)b * ldq + r0] = g | __float_as_uint(v.x);
   qkvt[(size_t)b * ldq + r1] = g | __float_as_uint(v.y);
@@ -525,70 +562,235 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
   phase_attn<true, 0, NCW, 1, 4>(a, l, r.tick, r.pos, x, 0x10000u, s);
 }
 
-// The same attention items of rows with distinct caches (a lockstep step)
-// with the QKV epilogue before and the chunk combine after, so that one
-// launch replaces three. Each item forms its kv group's q/k/v from the QKV
-// product itself (qkv_epi_pair; the chunk-0 item also writes k and v into
-// the cache: no item of the step reads that row, as position pos comes from
-// LDS), runs phase_attn, and counts itself done in cnt[b][g] (an
-// agent-scope add); the group's last item waits for the tags of the group's
-// chunk partials, combines them (combine_scales / combine_value, as
-// k_b_comb) into the attention panel and sets the count back to 0.
-__global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_b_attn_f(
-    const Args* __restrict__ rargs, const BRow* __restrict__ rows,
-    const uint32_t* __restrict__ items, uint32_t l, const float* __restrict__ Y, uint32_t ldy,
-    const float* __restrict__ inv, uint32_t* __restrict__ cnt, float* __restrict__ attp) {
-  const uint32_t e = items[blockIdx.x], b = e >> 16, x = e & 0xffffu;
-  const Args& a = rargs[b];
-  const Lds s = lds_init_attn();
-  const BRow r = rows[b];
+// Attention of rows with distinct caches (a lockstep step), QKV epilogue and
+// chunk combine included: one workgroup per (row, kv head), of TEAMS teams of
+// NCW waves. The first waves form 1/rms of the row and the group's q/k/v from
+// the QKV product (QkvEpiPair; k and v go to the cache too: no chunk reads
+// that row, as position pos comes from LDS). The teams take the chunks in
+// turn (team t: chunks t, t + TEAMS, ...), each computing its chunk's
+// partials as phase_attn's grouped form does -- the same lanes, chains and
+// folds per head, with the next chunk's first K and V rows in flight -- into
+// LDS, where combine_scales / combine_value then merge them in chunk order
+// into the attention panel.
+//
+// Bound by latency for few rows (a chain of dependent loads and barriers),
+// by memory for many. One workgroup per (row, kv head, chunk) instead, the
+// last of a group (an agent-scope count) polling the others' partials, took
+// 13.7 us per layer for 7 rows of the 135M shape at 150 positions (11.8 now,
+// with the rows' 1/rms inside) and 30 us for 64 of the 1B shape at 256 (27.4).
+// HD: the head size, or 0 to read it from d.
+struct AttnRowsLds {
+  uint32_t ml, sc, wp, part, sw, total;  // float offsets: after q, k and v
+};
+__host__ __device__ inline AttnRowsLds attn_rows_lds(uint32_t hd, uint32_t grp, uint32_t teams,
+                                                     uint32_t ch, uint32_t nch) {
+  AttnRowsLds o;
+  o.ml = (grp + 2) * hd;                         // [teams][grp][2]
+  o.sc = o.ml + teams * 2 * MAX_GROUP;           // [teams][grp][ch]
+  o.wp = o.sc + teams * grp * ch;                // [teams][NCW][grp][hd]
+  o.part = o.wp + teams * NCW * grp * hd;        // [grp][nch][hd + 2]
+  o.sw = o.part + grp * nch * (hd + 2);          // [grp][nch] weights, then [grp] totals
+  o.total = o.sw + grp * nch + MAX_GROUP;
+  return o;
+}
+template <uint32_t HD, uint32_t TEAMS>
+__global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_b_attn_f(
+    const Args* __restrict__ ap, const BRow* __restrict__ rows, uint32_t l,
+    const float* __restrict__ X, const float* __restrict__ Y, uint32_t ldy, uint32_t max_nch,
+    uint32_t max_ch, float* __restrict__ attp) {
+  extern __shared__ float lds_raw[];
+  // K rows of KU score passes and V rows of VE value steps are requested a
+  // chunk ahead, V rows up to VU steps once the scores have freed K's registers.
+  constexpr uint32_t KU = HD ? 2 : 1, VE = 4, VU = HD == 64 ? 8 : HD ? 6 : 4, NW = TEAMS * NCW;
+  const Args& a = *ap;  // by reference: as kernel arguments its fields took registers (spills, 32 against 27 us at 1B)
   const Dims& d = a.d;
-  const uint32_t nch = attn_nchunks(r.pos), g = x / nch, c = x - g * nch;
-  const float iv = inv[b];
-  auto fill = [&](uint32_t gg, float* qs, float* kn, float* vn) {
-    for (uint32_t u = threadIdx.x; u < (d.group + 2) * d.half; u += blockDim.x) {
-      const uint32_t j = u / d.half, i = u - j * d.half;
-      const uint32_t hb = j < d.group ? gg * d.group + j : (j == d.group ? d.nh + gg : d.nh + d.nkv + gg);
-      const float2 v = qkv_epi_pair(a, l, r.pos, b, hb, i, Y, ldy, iv);
-      float* dst = j < d.group ? qs + j * d.hd : (j == d.group ? kn : vn);
-      lds_st(dst + i, v.x);
-      lds_st(dst + i + d.half, v.y);
-      if (j >= d.group && c == 0) qkv_epi_cache(d, r, l, hb, i, v);
-    }
-    __syncthreads();
-    return true;
+  const uint32_t b = blockIdx.x / d.nkv, g = blockIdx.x - b * d.nkv;
+  const BRow r = rows[b];
+  const uint32_t pos = r.pos, nch = attn_nchunks(pos), CH = attn_chunk(pos);
+  const uint32_t hd = HD ? HD : d.hd, half = hd / 2, grp = d.group, hs = hd + 2;
+  const AttnRowsLds o = attn_rows_lds(hd, grp, TEAMS, max_ch, max_nch);
+  const uint32_t wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+  const uint32_t team = wave / NCW, aw = wave % NCW, tt = threadIdx.x % (NCW * WAVE);
+  float* qs = lds_raw;  // [grp][hd]
+  float* kn = qs + grp * hd;
+  float* vn = kn + hd;
+  float* ml = lds_raw + o.ml + team * 2 * MAX_GROUP;
+  float* sc = lds_raw + o.sc + team * grp * max_ch;  // [grp][CH]
+  float* wp = lds_raw + o.wp + team * NCW * grp * hd;
+  float* part = lds_raw + o.part;
+  AttGeo ge = att_geo(hd);
+  const uint32_t ps = lane / ge.lps, sub = lane % ge.lps, pl = lane / ge.lv, dl = lane % ge.lv;
+  const uint32_t sstep = NCW * ge.pw, vstep = NCW * ge.pv;
+  const uint32_t tw = aw * ge.pw + ps, vw = aw * ge.pv + pl;
+  // Uniform bases and 32-bit byte offsets: K and V rows of this kv head.
+  const float* kb = r.kc + ((size_t)l * d.nkv + g) * r.cap * d.kvs;
+  const float* vb = r.vc + ((size_t)l * d.nkv + g) * r.cap * d.kvs;
+  auto load_k = [&](float4 (&k)[4], uint32_t t) {
+    const uint32_t at = (t * d.kvs + sub * 16) * 4;
+#pragma unroll
+    for (uint32_t i = 0; i < 4; ++i) k[i] = ldg4_at(kb, at + 16 * i);
   };
-  phase_attn<true, 0, NCW, 1, 4>(a, l, r.tick, r.pos, x, 0x10000u, s, fill);
-  // Every wave has issued its partials' stores. No fence: the last item
-  // waits for the partials' tags instead (a device-scope fence would write
-  // back and invalidate the whole L2 of the XCD).
-  __syncthreads();
-  AS_LDS uint32_t* last = lptr(reinterpret_cast<uint32_t*>(s.red));
-  if (threadIdx.x == 0) {
-    uint32_t* cg = cnt + (size_t)b * d.nkv + g;
-    const uint32_t done = __hip_atomic_fetch_add(cg, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    *last = done + 1 == nch;
-    if (done + 1 == nch) __hip_atomic_store(cg, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  auto load_v = [&](uint32_t t) { return ldg4_at(vb, (t * d.kvs + dl * 4) * 4); };
+  float4 kr[KU][4], vr[VU];
+  // Rows at or past pos are clamped to the last one before it and never
+  // used; the loads have no condition (also for a chunk past the last), so
+  // no old value is kept alive for them.
+  const uint32_t t_last = max(pos, 1u) - 1;
+  auto prefetch = [&](uint32_t c) {
+    const uint32_t t0 = c * CH;
+#pragma unroll
+    for (uint32_t u = 0; u < KU; ++u) load_k(kr[u], min(t0 + tw + u * sstep, t_last));
+#pragma unroll
+    for (uint32_t u = 0; u < VE; ++u) vr[u] = load_v(min(t0 + vw + u * vstep, t_last));
+  };
+  prefetch(team);
+  // q, k and v of the group: one thread per pair of rotated elements.
+  const uint32_t pairs = (grp + 2) * half;
+  if (wave * WAVE < pairs) {
+    const float iv = rms_row_inv(X + (size_t)b * d.h, d.h, d.eps, lane);
+    for (uint32_t u = threadIdx.x; u < pairs; u += NW * WAVE) {
+      const uint32_t j = u / half, i = u - j * half;
+      const uint32_t hb = j < grp ? g * grp + j : (j == grp ? d.nh + g : d.nh + d.nkv + g);
+      QkvEpiPair ep;
+      ep.load(d, a.rope, a.layers[l].bqkv, pos, hb, i, Y + (size_t)b * ldy);
+      const float2 v = ep.value(iv);
+      float* dst = qs + j * hd;  // k and v follow the queries
+      lds_st(dst + i, v.x);
+      lds_st(dst + i + half, v.y);
+      if (j >= grp) qkv_epi_cache(d, r, l, hb, i, v);
+    }
   }
   __syncthreads();
-  if (!*last) return;
-  const uint32_t hs = d.hd + 2, grp = d.group, n1 = nch * hs;
-  float* part = s.scr;                      // [grp][nch][hs]
-  float* sc = part + MAX_GROUP * MAX_ACHUNKS * hs;  // [MAX_GROUP][MAX_ACHUNKS]
-  float* ls = sc + MAX_GROUP * MAX_ACHUNKS;  // [MAX_GROUP]
-  if (!poll_gather<4>(gather_strided(a.mb_part + (size_t)g * grp * MAX_ACHUNKS * hs, n1, grp,
-                                     MAX_ACHUNKS * hs, gen_of(d, r.tick, l, PH_ATTN), part),
-                      NCW, a.st, s.ctl))
-    return;
-  for (uint32_t k = threadIdx.x; k < grp; k += blockDim.x)
-    ls[k] = combine_scales([&](uint32_t i) { return lds_ld(part + k * n1 + i); }, nch, hs,
-                           sc + k * MAX_ACHUNKS);
+  const uint32_t rounds = (nch + TEAMS - 1) / TEAMS;
+  for (uint32_t rd = 0; rd < rounds; ++rd) {
+    const uint32_t c = rd * TEAMS + team, t0 = c * CH;
+    const uint32_t t1 = c < nch ? min(t0 + CH, pos + 1) : t0;  // an idle team only meets the barriers
+    // scores, KU passes per round
+    for (uint32_t pb0 = t0; pb0 < t1; pb0 += KU * sstep) {
+#pragma unroll
+      for (uint32_t u = 0; u < KU; ++u) {
+        const uint32_t ts = pb0 + u * sstep + tw;
+        if (ts == pos) {
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) kr[u][i] = lds4(kn + sub * 16 + 4 * i);
+        }
+#pragma unroll 1
+        for (uint32_t j = 0; j < grp; ++j) {
+          float acc = 0.0f;
+#pragma unroll
+          for (uint32_t i = 0; i < 4; ++i) {
+            const float4 qq = lds4(qs + j * hd + sub * 16 + 4 * i);
+            acc = fmaf(qq.x, kr[u][i].x, acc);
+            acc = fmaf(qq.y, kr[u][i].y, acc);
+            acc = fmaf(qq.z, kr[u][i].z, acc);
+            acc = fmaf(qq.w, kr[u][i].w, acc);
+          }
+          const float v = group_sum(acc, ge.lps);
+          if (ts < t1 && sub == 0) lds_st(sc + j * CH + (ts - t0), v * d.scale);
+        }
+        const uint32_t tn = ts + KU * sstep;
+        if (tn < t1 && tn < pos) load_k(kr[u], tn);
+      }
+    }
+#pragma unroll
+    for (uint32_t u = VE; u < VU; ++u) vr[u] = load_v(min(t0 + vw + u * vstep, t_last));
+    __syncthreads();
+    // softmax statistics, one wave of the team per query head
+    const uint32_t n = t1 - t0;
+    if (n > 0 && aw < grp) {
+      float* sh = sc + aw * CH;
+      float m = -INFINITY;
+      for (uint32_t i = lane; i < n; i += WAVE) m = fmaxf(m, lds_ld(sh + i));
+      m = wave_max(m);
+      float ls = 0.0f;
+      for (uint32_t i = lane; i < n; i += WAVE) {
+        const float e = (m == -INFINITY) ? 0.0f : expf(lds_ld(sh + i) - m);
+        lds_st(sh + i, e);
+        ls += e;
+      }
+      ls = wave_sum(ls);
+      if (lane == 0) {
+        lds_st(ml + 2 * aw, m);
+        lds_st(ml + 2 * aw + 1, ls);
+      }
+    }
+    __syncthreads();
+    // exp-weighted V rows: positions t0 + vw + k*vstep, k = 0, 1, ...
+    float4 acc[MAX_GROUP];
+#pragma unroll
+    for (uint32_t j = 0; j < MAX_GROUP; ++j) acc[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const uint32_t nk = t0 + vw < t1 ? (t1 - t0 - vw + vstep - 1) / vstep : 0;
+    for (uint32_t k0 = 0; k0 < nk; k0 += VU) {
+#pragma unroll
+      for (uint32_t u = 0; u < VU; ++u) {
+        const uint32_t k = k0 + u;
+        if (k < nk) {
+          const uint32_t t = t0 + vw + k * vstep;
+          const float4 v = (t == pos) ? lds4(vn + dl * 4) : vr[u];
+          const uint32_t tf = t + VU * vstep;
+          if (k + VU < nk && tf < pos) vr[u] = load_v(tf);
+#pragma unroll
+          for (uint32_t j = 0; j < MAX_GROUP; ++j) {
+            if (j >= grp) break;
+            const float p = lds_ld(sc + j * CH + (t - t0));
+            acc[j].x = fmaf(p, v.x, acc[j].x);
+            acc[j].y = fmaf(p, v.y, acc[j].y);
+            acc[j].z = fmaf(p, v.z, acc[j].z);
+            acc[j].w = fmaf(p, v.w, acc[j].w);
+          }
+        }
+      }
+    }
+    prefetch(c + TEAMS);
+    for (uint32_t x = ge.lv; x < WAVE; x <<= 1) {
+#pragma unroll
+      for (uint32_t j = 0; j < MAX_GROUP; ++j) {
+        if (j >= grp) break;
+        acc[j].x += __shfl_xor(acc[j].x, x);
+        acc[j].y += __shfl_xor(acc[j].y, x);
+        acc[j].z += __shfl_xor(acc[j].z, x);
+        acc[j].w += __shfl_xor(acc[j].w, x);
+      }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < MAX_GROUP; ++j)
+      if (j < grp && pl == 0) {
+        float* dst = wp + (aw * grp + j) * hd + dl * 4;
+        lds_st(dst + 0, acc[j].x);
+        lds_st(dst + 1, acc[j].y);
+        lds_st(dst + 2, acc[j].z);
+        lds_st(dst + 3, acc[j].w);
+      }
+    __syncthreads();
+    // The four waves' sums, in wave order, and (m, l). The next round's
+    // barriers order these reads before its writes of wp and ml.
+    if (n > 0)
+      for (uint32_t u = tt; u < grp * hd; u += NCW * WAVE) {
+        const uint32_t j = u / hd, dd = u - j * hd;
+        float A = 0.0f;
+#pragma unroll
+        for (uint32_t w = 0; w < NCW; ++w) A += lds_ld(wp + (w * grp + j) * hd + dd);
+        float* out = part + (j * nch + c) * hs;
+        lds_st(out + 2 + dd, A);
+        if (dd == 0) {
+          lds_st(out, lds_ld(ml + 2 * j));
+          lds_st(out + 1, lds_ld(ml + 2 * j + 1));
+        }
+      }
+  }
   __syncthreads();
-  for (uint32_t v = threadIdx.x; v < grp * d.hd; v += blockDim.x) {
-    const uint32_t k = v / d.hd, dd = v - k * d.hd, u = (g * grp + k) * d.hd + dd;
+  float* sw = lds_raw + o.sw;         // [grp][nch]
+  float* ls = sw + grp * max_nch;     // [grp]
+  if (threadIdx.x < grp) {
+    const float* pj = part + threadIdx.x * nch * hs;
+    ls[threadIdx.x] = combine_scales([&](uint32_t i) { return lds_ld(pj + i); }, nch, hs, sw + threadIdx.x * nch);
+  }
+  __syncthreads();
+  for (uint32_t v = threadIdx.x; v < grp * hd; v += NW * WAVE) {
+    const uint32_t k = v / hd, dd = v - k * hd, u = (g * grp + k) * hd + dd;
     attp[panel_at(b, u, panel_chunks(d.q))] =
-        combine_value([&](uint32_t i) { return lds_ld(part + k * n1 + i); }, nch, hs, dd,
-                      sc + k * MAX_ACHUNKS, ls[k]);
+        combine_value([&](uint32_t i) { return lds_ld(part + k * nch * hs + i); }, nch, hs, dd,
+                      sw + k * nch, ls[k]);
   }
 }
 

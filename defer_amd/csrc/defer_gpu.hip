@@ -468,6 +468,13 @@ static const void* attn_tile_kernel(uint32_t hd, uint32_t nb) {
   if ((hd != 64 && hd != 128) || nb < 1 || nb > AT_MAX_NB) return nullptr;
   return k[hd == 128][nb - 1];
 }
+// The attention of a lockstep step's rows with `teams` teams per workgroup.
+static const void* attn_rows_kernel(uint32_t hd, uint32_t teams) {
+#define DG_ROWS(HD) \
+  (teams == 4 ? (const void*)k_b_attn_f<HD, 4> : teams == 2 ? (const void*)k_b_attn_f<HD, 2> : (const void*)k_b_attn_f<HD, 1>)
+  return hd == 64 ? DG_ROWS(64) : hd == 128 ? DG_ROWS(128) : DG_ROWS(0);
+#undef DG_ROWS
+}
 // Query heads of a group in one task, at most: as many as leave LDS for two
 // workgroups per CU.
 static uint32_t attn_tile_heads(const Dims& d, uint32_t nb) {
@@ -604,9 +611,7 @@ static int apply_layout(defer_gpu_model* m, uint32_t G) {
   m->lds_bytes = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr + d.lds_stg) * sizeof(float) +
                  (size_t)d.lds_pub * 2 * sizeof(u64) + (d.lds_stg ? 0 : 1024);
   m->lds_rows = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr) * sizeof(float);
-  // k_b_attn_f's combine: the group's chunk partials, their weights and totals.
-  const uint32_t scr_fcomb = MAX_GROUP * MAX_ACHUNKS * hs + MAX_GROUP * MAX_ACHUNKS + MAX_GROUP;
-  m->lds_attn = (size_t)(4 + 64 + ((std::max(scr_attn, scr_fcomb) + 3) & ~3u)) * sizeof(float);
+  m->lds_attn = (size_t)(4 + 64 + ((scr_attn + 3) & ~3u)) * sizeof(float);
 
   m->G = G;
   const void* kernels[] = {m->persistent[0], m->persistent[1], (const void*)k_phase, (const void*)k_samp_a,
@@ -625,11 +630,17 @@ static int apply_layout(defer_gpu_model* m, uint32_t G) {
       return fail(DEFER_GPU_E_HIP, "LDS attribute (%zu bytes): %s", samp_lds_bytes(m),
                   hipGetErrorString(e));
   }
-  for (const void* kf : {(const void*)k_b_attn_w, (const void*)k_b_attn_f}) {
+  for (const void* kf : {(const void*)k_b_attn_w}) {
     const hipError_t e =
         hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)m->lds_attn);
     if (e != hipSuccess)
       return fail(DEFER_GPU_E_HIP, "LDS attribute (%zu bytes): %s", m->lds_attn, hipGetErrorString(e));
+  }
+  for (uint32_t teams = 1; teams <= 4; teams *= 2) {
+    const hipError_t e = hipFuncSetAttribute(attn_rows_kernel(d.hd, teams),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES_MAX);
+    if (e != hipSuccess)
+      return fail(DEFER_GPU_E_HIP, "LDS attribute (rows' attention): %s", hipGetErrorString(e));
   }
   for (const void* kf : m->persistent) {
     int occ = 0;
@@ -1795,7 +1806,6 @@ struct BatchWs {
   uint32_t *sel = nullptr, *lgen = nullptr, *stick = nullptr, *swords = nullptr, *sout = nullptr;
   uint32_t* items = nullptr;  // attention (row, item) list, or tiled attention tasks
   uint32_t* tiles = nullptr;  // tiled attention: first batch row of each tile
-  uint32_t* CNT = nullptr;    // [rows][nkv] finished attention items (k_b_attn_f), 0 between launches
   StateSet* sets = nullptr;   // [rows] cache states to set after a batch
   DevState* st = nullptr;
 };
@@ -1804,7 +1814,7 @@ static void batch_ws_release(BatchWs* w) {
   if (!w) return;
   void* ps[] = {w->X, w->Y, w->INV, w->XP, w->XQ, w->LINV, w->QKVT, w->PART,
                 w->LOGT, w->VMAX, w->VARG, w->VSUM, w->VP, w->drows, w->rargs, w->largs, w->sel,
-                w->lgen, w->stick, w->swords, w->sout, w->items, w->tiles, w->CNT, w->sets, w->st};
+                w->lgen, w->stick, w->swords, w->sout, w->items, w->tiles, w->sets, w->st};
   for (void* p : ps) (void)hipFree(p);
   *w = BatchWs();
 }
@@ -1837,8 +1847,6 @@ static int ensure_ws(defer_gpu_model* m, uint32_t rows, uint32_t lm) {
   HIP_TRY(counted_malloc(&w.rargs, (size_t)R * sizeof(Args)));
   HIP_TRY(counted_malloc(&w.items, (size_t)R * d.nkv * MAX_ACHUNKS * d.group * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&w.tiles, ((size_t)R / 16 + 3) * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.CNT, (size_t)R * d.nkv * sizeof(uint32_t)));
-  HIP_TRY(hipMemset(w.CNT, 0, (size_t)R * d.nkv * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&w.sets, (size_t)R * sizeof(StateSet)));
   const uint32_t L1 = std::max(Lm, 1u);
   HIP_TRY(counted_malloc(&w.XQ, panel_floats(std::max(R, L1), kmax) * sizeof(float)));
@@ -1934,6 +1942,7 @@ static void launch_gemm(hipStream_t s, uint32_t ncu, const float* Wp, uint32_t M
     const uint32_t n = ((M + 16 * tr - 1) / (16 * tr)) * ((B + 16 * tc - 1) / (16 * tc));
     return (float)((n + ncu - 1) / ncu * tr * tc) * per_tile;
   };
+  if (OUT == GO_ACT && out.X) return launch_gemm_tile<2, 1, OUT>(s, Wp, M, K, Xp, B, out);
   const float c[4] = {cost(4, 2, 1.0f), cost(2, 2, 1.06f), cost(2, 1, 1.15f), cost(1, 1, 1.3f)};
   switch (std::min_element(c, c + (PAIRS ? 3 : 4)) - c) {
     case 0: return launch_gemm_tile<4, 2, OUT>(s, Wp, M, K, Xp, B, out);
@@ -2048,8 +2057,6 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   rc = ensure_ws(m, n, nl);
   if (rc) return rc;
   BatchWs& w = *m->bw;
-  std::vector<Args> ra(n);
-  for (uint32_t b = 0; b < n; ++b) ra[b] = row_args(rcache[b], w, b);
   // Attention: tiles of 16 aligned positions when the rows are one cache's
   // consecutive positions (a prefill or a replay) and the tiled kernel has
   // the shape and the chunk sizes (at most two: the chunk grows every 2048
@@ -2068,6 +2075,23 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     std::vector<const defer_gpu_cache*> cs(rcache, rcache + n);
     std::sort(cs.begin(), cs.end());
     fused = std::adjacent_find(cs.begin(), cs.end()) == cs.end();
+  }
+  // Its teams per workgroup: as many as the longest row has chunks, as long
+  // as every workgroup's waves are resident at once (16 per CU), so that a
+  // few rows spread over the waves of a CU and many rows over the CUs.
+  uint32_t teams = 1, max_ch = 0, max_nch = 0;
+  size_t lds_rows_attn = 0;
+  if (fused) {
+    for (uint32_t b = 0; b < n; ++b) {
+      max_ch = std::max(max_ch, attn_chunk(rows[b].pos));
+      max_nch = std::max(max_nch, attn_nchunks(rows[b].pos));
+    }
+    auto lds = [&](uint32_t t) { return attn_rows_lds(d.hd, d.group, t, max_ch, max_nch).total * sizeof(float); };
+    while (teams < 4 && teams < max_nch && n * d.nkv * 2 * teams * NCW <= 16 * m->ncu &&
+           lds(2 * teams) <= LDS_BYTES_MAX)
+      teams *= 2;
+    lds_rows_attn = lds(teams);
+    fused = lds_rows_attn <= LDS_BYTES_MAX;  // else the chunks as items
   }
   std::vector<uint32_t> items, tiles;
   uint32_t n_items0 = 0;  // tiled: tasks of the first chunk size
@@ -2088,7 +2112,7 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
           }
       if (nb == nb0) n_items0 = (uint32_t)items.size();
     }
-  } else {
+  } else if (!fused) {
     // Grouped items x = (kv head, chunk): every query head of the group in
     // one (rows <= 2048, items < 2^16). Full chunks are listed before each
     // row's last, shorter one, so that the longest items are dispatched
@@ -2109,9 +2133,14 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   std::vector<uint32_t> lgen(nl);
   for (uint32_t i = 0; i < nl; ++i) lgen[i] = gen_lm(d, rows[sel[i]].tick);
   HIP_TRY(hipMemcpyAsync(w.drows, rows, n * sizeof(BRow), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(w.rargs, ra.data(), n * sizeof(Args), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(w.items, items.data(), items.size() * sizeof(uint32_t),
-                         hipMemcpyHostToDevice, s));
+  // Every row's one-token arguments for attention items (else the first's
+  // model pointers serve all rows).
+  std::vector<Args> ra(tiled || fused ? 1 : n);
+  for (uint32_t b = 0; b < ra.size(); ++b) ra[b] = row_args(rcache[b], w, b);
+  HIP_TRY(hipMemcpyAsync(w.rargs, ra.data(), ra.size() * sizeof(Args), hipMemcpyHostToDevice, s));
+  if (!items.empty())
+    HIP_TRY(hipMemcpyAsync(w.items, items.data(), items.size() * sizeof(uint32_t),
+                           hipMemcpyHostToDevice, s));
   if (tiled)
     HIP_TRY(hipMemcpyAsync(w.tiles, tiles.data(), tiles.size() * sizeof(uint32_t),
                            hipMemcpyHostToDevice, s));
@@ -2127,8 +2156,10 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   // gate rows are whole tiles). A 301-row layer of the 135M shape drops from 8
   // launches to 6, a 2048-row one saves the 25 MB of gate and up rows.
   const bool act_out = d.ff % 16 == 0;
+  const bool own_rms = act_out && n <= 16;  // the gate/up product forms the rows' 1/rms
   k_b_embed<<<n, 256, 0, s>>>(w.drows, dtok, m->embed, d.h, w.X, w.XP);
-  k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
+  // 1/rms for the QKV product's outputs (k_b_attn_f forms its rows' own).
+  if (!fused) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   for (uint32_t l = 0; l < d.L; ++l) {
     GemmOutArgs o{};
     o.Y = w.Y;
@@ -2155,8 +2186,11 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     }
     if (fused) {
       ProfSpan ps(m, 1, attn_flop);
-      k_b_attn_f<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(
-          w.rargs, w.drows, w.items, l, w.Y, ldy, w.INV, w.CNT, w.XQ);
+      uint32_t li = l, ld = ldy;
+      const float *xr = w.X, *yr = w.Y;
+      void* args[] = {&w.rargs, &w.drows, &li, &xr, &yr, &ld, &max_nch, &max_ch, &w.XQ};
+      HIP_TRY(hipLaunchKernel(attn_rows_kernel(d.hd, teams), dim3(n * d.nkv), dim3(teams * NCW * WAVE), args,
+                              lds_rows_attn, s));
     } else {
       if (!tiled)
         k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
@@ -2184,9 +2218,13 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       ProfSpan ps(m, 0, 2.0 * d.h * d.q * n);
       launch_gemm<GO_RESID>(s, ncu, m->p_o[l], d.h, d.q, w.XQ, n, x);
     }
-    k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
+    if (own_rms)
+      o.X = w.X;
+    else
+      k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
     {
       ProfSpan ps(m, 0, 2.0 * 2 * d.ff * d.h * n);
+      o.eps = d.eps;
       o.P = w.XQ;
       o.blk = d.ff / 16;
       o.act = d.act;
@@ -2201,7 +2239,7 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       ProfSpan ps(m, 0, 2.0 * d.h * d.ff * n);
       launch_gemm<GO_RESID>(s, ncu, m->p_d[l], d.h, d.ff, w.XQ, n, x);
     }
-    if (l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
+    if (!fused && l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   }
   if (nl) {
     k_b_final<<<nl, 64, 0, s>>>(w.X, w.sel, d.h, m->norm, d.eps, w.XQ, w.LINV);
