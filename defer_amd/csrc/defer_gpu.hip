@@ -30,7 +30,7 @@ using namespace dg;
   namespace NS {                                              \
   struct Args;                                                \
   struct RunDesc;                                             \
-  template <bool RANDOM>                                      \
+  template <bool RANDOM, bool TRACE>                          \
   __global__ void k_persistent(const Args* ap, const RunDesc* run); \
   }
 DG_DECLARE_SPECIALISED(dg135)
@@ -99,7 +99,7 @@ __global__ void k_begin(DevState* st) {
 enum : uint32_t { PH_LM_KERNEL = 100 };
 
 __global__ __launch_bounds__(BLOCK) void k_phase(const Args* __restrict__ ap, uint32_t ph,
-                                                 uint32_t layer) {
+                                                 uint32_t layer, float* trace_q) {
   const Args& a = *ap;
   const Lds s = lds_init(a.d);
   const DevState* st = a.st;
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(BLOCK) void k_phase(const Args* __restrict__ ap, ui
   const uint32_t wg = blockIdx.x, G = gridDim.x;
   const Stager sg = make_stager(a, s, wg, G, false);
   switch (ph) {
-    case PH_QKV: phase_qkv(a, layer, tick, pos, token, wg, G, s, sg); break;
+    case PH_QKV: phase_qkv<true>(a, layer, tick, pos, token, wg, G, s, sg, trace_q); break;
     case PH_ATTN: phase_attn(a, layer, tick, pos, wg, G, s); break;
     case PH_COMB: phase_comb(a, layer, tick, pos, wg, G, s); break;
     case PH_O: phase_o(a, layer, tick, pos, token, wg, G, s, sg); break;
@@ -183,31 +183,43 @@ __global__ void k_commit(const Args* __restrict__ ap, const RunDesc* __restrict_
   if (run->mode == RUN_GENERATE && is_stop(*run, st->token)) st->halt = 1;
 }
 
-// The attention probabilities of one layer for the forward in flight (the
-// trace of forward_ext, model.rs:486-488), written as [nh][pos + 1]: scores
-// in phase_attn's order (16-element fma chains per lane group, the group's
-// tree, then the scale; masked positions -inf), then p_t = exp(s_t - M) / S
-// with M the context's max and S the sum of exp(s_t - M) (thread-strided
-// partials in position order, then a fixed tree). One workgroup per head;
-// runs after the layer's attention and before the next layer's q/k/v.
-__global__ __launch_bounds__(256) void k_trace(const Args* __restrict__ ap, uint32_t l,
-                                               float* __restrict__ out) {
+// The attention probabilities of a traced forward at position pos (the
+// trace of forward_ext, model.rs:486-488), written as [L][nh][pos + 1]: scores
+// of layer blockIdx.y's queries (kept by the run, [L][q]) in phase_attn's
+// order (16-element fma chains per lane group, the group's tree, then the
+// scale; masked positions -inf), then p_t = exp(s_t - M) / S with M the
+// context's max and S the sum of exp(s_t - M) (thread-strided partials in
+// position order, then a fixed tree). One workgroup per (head, layer), all in
+// one launch after the run: a launch per layer between the phases' kernels
+// took 30 x 10.8 us at 400 positions (135M shape).
+__global__ __launch_bounds__(256) void k_trace(const Args* __restrict__ ap, uint32_t pos,
+                                               const float* __restrict__ q, float* __restrict__ out) {
   const Args& a = *ap;
   const Dims& d = a.d;
-  const uint32_t hh = blockIdx.x, g = hh / d.group, pos = a.st->pos, n = pos + 1;
+  const uint32_t hh = blockIdx.x, l = blockIdx.y, g = hh / d.group, n = pos + 1;
   const uint32_t hd = d.hd, lps = hd / 16;
-  float* o = out + (size_t)hh * n;
+  float* o = out + ((size_t)l * d.nh + hh) * n;
   __shared__ float red[256 / WAVE];
+  __shared__ float qv[256];  // head_dim <= 256
+  for (uint32_t i = threadIdx.x; i < hd; i += blockDim.x) qv[i] = q[(size_t)l * d.q + hh * hd + i];
+  __syncthreads();
   const float* kb = a.kc + ((size_t)l * d.nkv + g) * d.cap * d.kvs;
   float mx = -INFINITY;
   for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) {
+    const float4* row = reinterpret_cast<const float4*>(kb + (size_t)t * d.kvs);
     float part[16];
     for (uint32_t sb = 0; sb < lps; ++sb) {
+      float4 k[4];
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) k[e] = row[sb * 4 + e];
       float acc = 0.0f;
-      for (uint32_t e = 0; e < 16; ++e) {
-        const uint32_t i = sb * 16 + e;
-        const float q = __uint_as_float((uint32_t)a.mb_qkv[hh * hd + i]);
-        acc = fmaf(q, kb[(size_t)t * d.kvs + i], acc);
+#pragma unroll
+      for (uint32_t e = 0; e < 4; ++e) {
+        const float* qe = qv + sb * 16 + 4 * e;
+        acc = fmaf(qe[0], k[e].x, acc);
+        acc = fmaf(qe[1], k[e].y, acc);
+        acc = fmaf(qe[2], k[e].z, acc);
+        acc = fmaf(qe[3], k[e].w, acc);
       }
       part[sb] = acc;
     }
@@ -320,35 +332,56 @@ __global__ void k_kv_gather(const float* src, float* dst, uint32_t len, uint32_t
 }
 
 // ValueNorms::sync (attribution.rs:116-148): ||W_o,h . v_{t,kv(h)}|| for
-// positions t0 + blockIdx.y, query head blockIdx.x, layer blockIdx.z. Thread
-// i forms o_i = sum_d Wo[i][h*hd + d] * v[d] as a sequential sum of rounded
-// products (built without contraction, so no fused multiply-add), the
-// squares go to LDS, and one thread adds them in order i = 0, 1, ... before
-// the square root -- the reference's loop order exactly.
+// positions t0 + TB * blockIdx.y .., query head blockIdx.x, layer blockIdx.z.
+// A thread forms o_i = sum_d Wo[i][h*hd + d] * v[d] as a sequential sum of
+// rounded products (built without contraction, so no fused multiply-add), the
+// squares go to LDS, and one thread per position adds them in order i = 0, 1,
+// ... before the square root -- the reference's loop order exactly. Bound by
+// the reads of W_o's head slices from L2: TB positions share one (64
+// positions of the 135M shape: 367 us with one position per workgroup, 152
+// with eight; two rows per lane, a line's loads back to back and scalar loads
+// of the value rows took 246 to 282).
+template <uint32_t TB>
 __global__ __launch_bounds__(256) void k_value_norms(const LayerW* __restrict__ layers,
                                                      const float* __restrict__ vc, Dims d,
                                                      uint32_t cap, uint32_t t0, uint32_t nt,
                                                      float* __restrict__ out) {
-  extern __shared__ float vn_lds[];  // [hd] value row, then [h] squares
-  const uint32_t h = blockIdx.x, t = t0 + blockIdx.y, l = blockIdx.z;
-  const uint32_t kvh = h / d.group, hd = d.hd;
+  extern __shared__ float vn_lds[];  // [TB][hd] value rows, then [h][TB] squares
+  const uint32_t h = blockIdx.x, tb = blockIdx.y * TB, l = blockIdx.z;
+  const uint32_t kvh = h / d.group, hd = d.hd, n = min(TB, nt - tb);
   float* v = vn_lds;
-  float* sq = vn_lds + hd;
-  const float* vrow = vc + (((size_t)l * d.nkv + kvh) * cap + t) * d.kvs;
-  for (uint32_t x = threadIdx.x; x < hd; x += blockDim.x) v[x] = vrow[x];
+  float* sq = vn_lds + TB * hd;
+  const float* vrow = vc + (((size_t)l * d.nkv + kvh) * cap + t0 + tb) * d.kvs;
+  for (uint32_t x = threadIdx.x; x < TB * hd; x += blockDim.x)
+    v[x] = x / hd < n ? vrow[(size_t)(x / hd) * d.kvs + x % hd] : 0.0f;
   __syncthreads();
   const float* wo = layers[l].wo;
   for (uint32_t i = threadIdx.x; i < d.h; i += blockDim.x) {
-    const float* row = wo + (size_t)i * d.q + h * hd;
-    float o = 0.0f;
-    for (uint32_t x = 0; x < hd; ++x) o = o + row[x] * v[x];
-    sq[i] = o * o;
+    const float4* row = reinterpret_cast<const float4*>(wo + (size_t)i * d.q + h * hd);
+    float o[TB];
+#pragma unroll
+    for (uint32_t t = 0; t < TB; ++t) o[t] = 0.0f;
+#pragma unroll 4
+    for (uint32_t x = 0; x < hd / 4; ++x) {
+      const float4 w = row[x];
+#pragma unroll
+      for (uint32_t t = 0; t < TB; ++t) {
+        const float4 u = *reinterpret_cast<const float4*>(v + t * hd + 4 * x);
+        o[t] = o[t] + w.x * u.x;
+        o[t] = o[t] + w.y * u.y;
+        o[t] = o[t] + w.z * u.z;
+        o[t] = o[t] + w.w * u.w;
+      }
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < TB; ++t) sq[i * TB + t] = o[t] * o[t];
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < n) {
     float s = 0.0f;
-    for (uint32_t i = 0; i < d.h; ++i) s = s + sq[i];
-    out[((size_t)l * nt + blockIdx.y) * d.nh + h] = sqrtf(s);
+#pragma unroll 16
+    for (uint32_t i = 0; i < d.h; ++i) s = s + sq[i * TB + threadIdx.x];
+    out[((size_t)l * nt + tb + threadIdx.x) * d.nh + h] = sqrtf(s);
   }
 }
 
@@ -372,7 +405,7 @@ struct defer_gpu_model {
   const float* head = nullptr;
   float2* rope = nullptr;
   uint32_t exec_mode = DEFER_GPU_EXEC_PERSISTENT;
-  const void* persistent[2] = {};  // the persistent kernel for this shape: greedy, random
+  const void* persistent[3] = {};  // the persistent kernel for this shape: greedy, random, traced
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_ms = 0.0;
   // Batched path (built on first use): weight panels and the workspace.
@@ -411,14 +444,14 @@ static bool has_shape(const Dims& d, const Dims& f) {
   return d.h == f.h && d.nh == f.nh && d.nkv == f.nkv && d.hd == f.hd && d.ff == f.ff &&
          d.V == f.V && d.L == f.L && d.act == f.act && d.has_bias == f.has_bias && d.tied == f.tied;
 }
-template <bool RANDOM>
+template <bool RANDOM, bool TRACE>
 static const void* persistent_kernel_for(const Dims& d) {
   if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_135M)) && d.stg_mask == 0xFu)
-    return (const void*)dg135::k_persistent<RANDOM>;
-  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_360M))) return (const void*)dg360::k_persistent<RANDOM>;
-  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_1B))) return (const void*)dg1b::k_persistent<RANDOM>;
-  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_8B))) return (const void*)dg8b::k_persistent<RANDOM>;
-  return (const void*)k_persistent<RANDOM>;
+    return (const void*)dg135::k_persistent<RANDOM, TRACE>;
+  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_360M))) return (const void*)dg360::k_persistent<RANDOM, TRACE>;
+  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_1B))) return (const void*)dg1b::k_persistent<RANDOM, TRACE>;
+  if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_8B))) return (const void*)dg8b::k_persistent<RANDOM, TRACE>;
+  return (const void*)k_persistent<RANDOM, TRACE>;
 }
 
 struct defer_gpu_cache {
@@ -442,8 +475,9 @@ struct defer_gpu_cache {
   size_t ring_cap = 0;
   float* d_logits = nullptr;
   float* d_tmp = nullptr;  // kv gather staging
-  float* d_trace = nullptr;   // [L][nh][cap] staging of a traced forward
-  float* trace_to = nullptr;  // set during a traced forward: where k_trace writes
+  float* d_trace = nullptr;   // a traced forward: probabilities [L][nh][cap], then queries [L][q]
+  float* d_norms = nullptr;   // staging of defer_gpu_value_norms
+  size_t norms_cap = 0;
   uint32_t pos = 0;        // host mirror of st->pos
   uint32_t tick = 0;
   uint32_t samp_next = 1;  // tag of the next sampling event's chunk sums (RunDesc)
@@ -606,15 +640,16 @@ static int apply_layout(defer_gpu_model* m, uint32_t G) {
     d.stg_mask = mask;
     d.lds_stg = stg;
   }
-  m->persistent[0] = persistent_kernel_for<false>(d);
-  m->persistent[1] = persistent_kernel_for<true>(d);
+  m->persistent[0] = persistent_kernel_for<false, false>(d);
+  m->persistent[1] = persistent_kernel_for<true, false>(d);
+  m->persistent[2] = persistent_kernel_for<false, true>(d);
   m->lds_bytes = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr + d.lds_stg) * sizeof(float) +
                  (size_t)d.lds_pub * 2 * sizeof(u64) + (d.lds_stg ? 0 : 1024);
   m->lds_rows = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr) * sizeof(float);
   m->lds_attn = (size_t)(4 + 64 + ((scr_attn + 3) & ~3u)) * sizeof(float);
 
   m->G = G;
-  const void* kernels[] = {m->persistent[0], m->persistent[1], (const void*)k_phase, (const void*)k_samp_a,
+  const void* kernels[] = {m->persistent[0], m->persistent[1], m->persistent[2], (const void*)k_phase, (const void*)k_samp_a,
                            (const void*)k_op};
   for (const void* kf : kernels) {
     const hipError_t e =
@@ -966,6 +1001,7 @@ static void cache_free(defer_gpu_cache* c) {
   (void)hipFree(c->d_logits);
   (void)hipFree(c->d_tmp);
   (void)hipFree(c->d_trace);
+  (void)hipFree(c->d_norms);
   (void)hipFree(c->d_args);
   if (c->h_ring) (void)hipHostFree(c->h_ring);
 }
@@ -1087,16 +1123,30 @@ extern "C" int defer_gpu_value_norms(const defer_gpu_cache* cc, uint32_t t0, uin
   const uint32_t nt = t1 - t0;
   if (nt == 0) return DEFER_GPU_OK;
   const size_t n = (size_t)d.L * nt * d.nh;
-  float* dout = nullptr;
-  HIP_TRY(counted_malloc(&dout, n * sizeof(float)));
+  if (n > c->norms_cap) {
+    (void)hipFree(c->d_norms);
+    c->d_norms = nullptr;
+    c->norms_cap = 0;
+    HIP_TRY(counted_malloc(&c->d_norms, n * sizeof(float)));
+    c->norms_cap = n;
+  }
   const hipStream_t s = m->stream;
-  k_value_norms<<<dim3(d.nh, nt, d.L), 256, (d.hd + d.h) * sizeof(float), s>>>(
-      m->d_layers, c->vc, d, c->cap, t0, nt, dout);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(out, dout, n * sizeof(float), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess) e = hipStreamSynchronize(s);
-  (void)hipFree(dout);
-  if (e != hipSuccess) return fail(DEFER_GPU_E_HIP, "value norms: %s", hipGetErrorString(e));
+  // Positions per workgroup: eight, or two where fewer are asked for or the
+  // squares of eight would not leave LDS for two workgroups per CU.
+  auto launch = [&](auto tb) {
+    constexpr uint32_t TB = decltype(tb)::value;
+    k_value_norms<TB><<<dim3(d.nh, (nt + TB - 1) / TB, d.L), 256, TB * (d.hd + d.h) * sizeof(float), s>>>(
+        m->d_layers, c->vc, d, c->cap, t0, nt, c->d_norms);
+  };
+  if (nt > 2 && 8 * (d.hd + d.h) * sizeof(float) <= 64 * 1024)
+    launch(std::integral_constant<uint32_t, 8>{});
+  else if (nt > 1)
+    launch(std::integral_constant<uint32_t, 2>{});
+  else
+    launch(std::integral_constant<uint32_t, 1>{});
+  HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(out, c->d_norms, n * sizeof(float), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipStreamSynchronize(s));
   return DEFER_GPU_OK;
 }
 
@@ -1128,7 +1178,7 @@ static int ensure_run_buffers(defer_gpu_cache* c, size_t n_ops, size_t n_stop) {
   return DEFER_GPU_OK;
 }
 
-static int launch_op_kernels(defer_gpu_cache* c, hipStream_t s) {
+static int launch_op_kernels(defer_gpu_cache* c, hipStream_t s, float* trace_q) {
   const defer_gpu_model* m = c->m;
   const Dims& d = m->d;
   const Args* a = c->d_args;
@@ -1137,34 +1187,32 @@ static int launch_op_kernels(defer_gpu_cache* c, hipStream_t s) {
   k_samp_a<<<G, BLOCK, lds, s>>>(a, c->d_run);
   k_op<<<1, BLOCK, lds, s>>>(a, c->d_run);
   for (uint32_t l = 0; l < d.L; ++l) {
-    for (uint32_t ph = 0; ph < PH_PER_LAYER; ++ph) {
-      k_phase<<<G, BLOCK, lds, s>>>(a, ph, l);
-      if (ph == PH_COMB && c->trace_to)
-        k_trace<<<d.nh, 256, 0, s>>>(a, l, c->trace_to + (size_t)l * d.nh * (c->pos + 1));
-    }
+    for (uint32_t ph = 0; ph < PH_PER_LAYER; ++ph) k_phase<<<G, BLOCK, lds, s>>>(a, ph, l, trace_q);
   }
-  k_phase<<<G, BLOCK, lds, s>>>(a, PH_LM_KERNEL, 0);
+  k_phase<<<G, BLOCK, lds, s>>>(a, PH_LM_KERNEL, 0, nullptr);
   k_commit<<<1, 1, 0, s>>>(a, c->d_run);
   HIP_TRY(hipGetLastError());
   return DEFER_GPU_OK;
 }
 
 // Queues n_ops ops described by `r` (host copy, device pointers filled in)
-// on the model's stream; run_finish waits for them.
-static int run_launch(defer_gpu_cache* c, RunDesc r, bool force_eager) {
+// on the model's stream; run_finish waits for them. no_graph: the phase kernels
+// one by one where the mode is a graph.
+static int run_launch(defer_gpu_cache* c, RunDesc r, bool no_graph = false) {
   defer_gpu_model* m = const_cast<defer_gpu_model*>(c->m);
   const hipStream_t s = m->stream;
   HIP_TRY(hipMemcpyAsync(c->d_run, &r, sizeof(r), hipMemcpyHostToDevice, s));
   k_begin<<<1, 1, 0, s>>>(c->st);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(m->ev0, s));
-  const uint32_t mode = force_eager ? DEFER_GPU_EXEC_EAGER : m->exec_mode;
+  const uint32_t mode =
+      no_graph && m->exec_mode == DEFER_GPU_EXEC_GRAPH ? (uint32_t)DEFER_GPU_EXEC_EAGER : m->exec_mode;
   if (r.n_ops > 0) {
     if (mode == DEFER_GPU_EXEC_PERSISTENT) {
       const Args* a = c->d_args;
       const RunDesc* dr = c->d_run;
       void* params[] = {&a, &dr};
-      const hipError_t e = hipLaunchCooperativeKernel(m->persistent[r.temperature != 0.0f], dim3(m->G),
+      const hipError_t e = hipLaunchCooperativeKernel(m->persistent[r.trace_q ? 2 : r.temperature != 0.0f], dim3(m->G),
                                                       dim3(BLOCK), params,
                                                       (unsigned)m->lds_bytes, s);
       if (e != hipSuccess) {
@@ -1174,7 +1222,7 @@ static int run_launch(defer_gpu_cache* c, RunDesc r, bool force_eager) {
         (void)hipGetLastError();
         ++m->coop_refused;
         for (uint32_t i = 0; i < r.n_ops; ++i) {
-          const int rc = launch_op_kernels(c, s);
+          const int rc = launch_op_kernels(c, s, r.trace_q);
           if (rc) return rc;
         }
       }
@@ -1182,7 +1230,7 @@ static int run_launch(defer_gpu_cache* c, RunDesc r, bool force_eager) {
       if (!c->graph) {
         hipGraph_t g;
         HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        const int rc = launch_op_kernels(c, s);
+        const int rc = launch_op_kernels(c, s, r.trace_q);
         hipError_t e = hipStreamEndCapture(s, &g);
         if (rc) return rc;
         if (e != hipSuccess) return fail(DEFER_GPU_E_HIP, "graph capture: %s", hipGetErrorString(e));
@@ -1194,7 +1242,7 @@ static int run_launch(defer_gpu_cache* c, RunDesc r, bool force_eager) {
       for (uint32_t i = 0; i < r.n_ops; ++i) HIP_TRY(hipGraphLaunch(c->graph, s));
     } else {
       for (uint32_t i = 0; i < r.n_ops; ++i) {
-        const int rc = launch_op_kernels(c, s);
+        const int rc = launch_op_kernels(c, s, r.trace_q);
         if (rc) return rc;
       }
     }
@@ -1221,8 +1269,8 @@ static int run_finish(defer_gpu_cache* c) {
   return DEFER_GPU_OK;
 }
 
-static int run_ops(defer_gpu_cache* c, RunDesc r, bool force_eager) {
-  const int rc = run_launch(c, r, force_eager);
+static int run_ops(defer_gpu_cache* c, RunDesc r, bool no_graph = false) {
+  const int rc = run_launch(c, r, no_graph);
   return rc ? rc : run_finish(c);
 }
 
@@ -1271,7 +1319,7 @@ extern "C" int defer_gpu_last_logits(const defer_gpu_cache* cc, float* logits_ou
 }
 
 static int feed_tokens(const defer_gpu_model* m, defer_gpu_cache* c, const uint32_t* tokens,
-                       size_t n, bool eager) {
+                       size_t n, bool no_graph = false, float* trace_q = nullptr) {
   for (size_t i = 0; i < n; ++i)
     if (tokens[i] >= m->d.V) return fail(DEFER_GPU_E_TOKEN, "token id %u out of range", tokens[i]);
   if ((size_t)c->pos + n > c->cap)
@@ -1288,7 +1336,8 @@ static int feed_tokens(const defer_gpu_model* m, defer_gpu_cache* c, const uint3
   r.words = c->d_words;
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
-  return run_ops(c, r, eager);
+  r.trace_q = trace_q;
+  return run_ops(c, r, no_graph);
 }
 
 extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, uint32_t token,
@@ -1317,18 +1366,22 @@ extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, u
     if (rc) return rc;
   }
   const uint32_t pos0 = c->pos;
-  if (trace_out) {
-    if (!c->d_trace)
-      HIP_TRY(counted_malloc(&c->d_trace, (size_t)m->d.L * m->d.nh * c->cap * sizeof(float)));
-    c->trace_to = c->d_trace;
-  }
-  rc = feed_tokens(m, c, &token, 1, use_mask || trace_out);
-  c->trace_to = nullptr;
-  if (!rc && trace_out)
-    rc = hipMemcpy(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
-                   hipMemcpyDeviceToHost) == hipSuccess
+  const size_t n_probs = (size_t)m->d.L * m->d.nh * c->cap;
+  if (trace_out && !c->d_trace)
+    rc = counted_malloc(&c->d_trace, (n_probs + (size_t)m->d.L * m->d.q) * sizeof(float)) == hipSuccess
+             ? DEFER_GPU_OK
+             : fail(DEFER_GPU_E_HIP, "trace allocation failed");
+  float* tq = trace_out ? c->d_trace + n_probs : nullptr;
+  // The captured graph's kernels keep no queries.
+  if (!rc) rc = feed_tokens(m, c, &token, 1, use_mask || trace_out, tq);
+  if (!rc && trace_out) {
+    k_trace<<<dim3(m->d.nh, m->d.L), 256, 0, m->stream>>>(c->d_args, pos0, tq, c->d_trace);
+    rc = hipMemcpyAsync(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
+                        hipMemcpyDeviceToHost, m->stream) == hipSuccess &&
+                 hipStreamSynchronize(m->stream) == hipSuccess
              ? DEFER_GPU_OK
              : fail(DEFER_GPU_E_HIP, "trace copy failed");
+  }
   if (use_mask) {
     c->args.mask = nullptr;
     const int rc2 = sync_args(c);
@@ -1385,7 +1438,7 @@ extern "C" int defer_gpu_prompt(const defer_gpu_model* m, defer_gpu_cache* c,
   if (use_batch(m, n_ok))
     rc = timed(m, [&] { return feed_batched(const_cast<defer_gpu_model*>(m), c, tokens, n_ok); });
   else
-    rc = feed_tokens(m, c, tokens, n_ok, false);
+    rc = feed_tokens(m, c, tokens, n_ok);
   if (rc) return rc;
   if (err == DEFER_GPU_E_TOKEN) return fail(err, "token id %u out of range", bad);
   if (err == DEFER_GPU_E_CONTEXT)
@@ -1435,7 +1488,7 @@ extern "C" int defer_gpu_generate(const defer_gpu_model* m, defer_gpu_cache* c, 
   r.words = c->d_words;
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
-  rc = run_ops(c, r, false);
+  rc = run_ops(c, r);
   if (rc) return rc;
   const DevState h = read_state(c);
   if (h.n_done) HIP_TRY(hipMemcpy(tokens_out, c->d_out, h.n_done * sizeof(uint32_t),
@@ -1505,7 +1558,7 @@ extern "C" int defer_gpu_generate_cb(const defer_gpu_model* m, defer_gpu_cache* 
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
   r.ring = c->d_ring;
-  rc = run_launch(c, r, false);
+  rc = run_launch(c, r);
   if (rc) return rc;
   // Hand each committed token to on_token, in order, as it lands; the run
   // is over once the stream is idle and the slot after the last is unset.
@@ -1677,7 +1730,7 @@ extern "C" int defer_gpu_generate_static(const defer_gpu_model* m, defer_gpu_cac
   r.out_tokens = d_out;
   // A graph would be instantiated (allocated) on first use: in graph mode the
   // same phase kernels run one by one instead (identical bits).
-  rc = run_ops(c, r, m->exec_mode == DEFER_GPU_EXEC_GRAPH);
+  rc = run_ops(c, r, true);
   if (rc) return rc;
   const DevState h = read_state(c);
   if (h.n_done) HIP_TRY(hipMemcpy(tokens_out, d_out, h.n_done * sizeof(uint32_t), hipMemcpyDeviceToHost));
@@ -1776,7 +1829,7 @@ extern "C" int defer_gpu_replay(const defer_gpu_model* m, defer_gpu_cache* c,
   r.words = c->d_words;
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
-  rc = run_ops(c, r, false);
+  rc = run_ops(c, r);
   if (rc) return rc;
   const DevState h = read_state(c);
   if (h.first_div >= 0) {

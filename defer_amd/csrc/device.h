@@ -109,6 +109,8 @@ struct RunDesc {
   const uint32_t* words;
   const uint32_t* stop;
   uint32_t* out_tokens;
+  // A traced run, nullable: every layer's rotated queries are kept, [L][q].
+  float* trace_q;
   // Generate runs only, nullable: pinned host words the host reads while the
   // run goes on; op i's token is committed as ((i + 1) << 32) | token.
   u64* ring;

@@ -15,9 +15,10 @@ __device__ __forceinline__ Lds lds_init(const Dims& d) {
   return s;
 }
 
+template <bool TRACE = false>
 __device__ __forceinline__ bool forward_all(const Args& a, uint32_t tok, uint32_t pos, uint32_t tick,
                                             uint32_t wg, uint32_t G, const Lds& s,
-                                            const Stager& sg) {
+                                            const Stager& sg, float* trace_q = nullptr) {
   const uint32_t L = shape_dims(a.d).L;
   for (uint32_t l = 0; l < L; ++l) {
     // Hidden from the optimiser per layer, so values derived from the
@@ -27,7 +28,7 @@ __device__ __forceinline__ bool forward_all(const Args& a, uint32_t tok, uint32_
     uint32_t wgl = wg;
     asm volatile("" : "+s"(wgl));
     const uint32_t wg = wgl;
-    if (!phase_qkv(a, l, tick, pos, tok, wg, G, s, sg)) return false;
+    if (!phase_qkv<TRACE>(a, l, tick, pos, tok, wg, G, s, sg, trace_q)) return false;
     if (!phase_attn(a, l, tick, pos, wg, G, s)) return false;
     if (!phase_comb(a, l, tick, pos, wg, G, s)) return false;
     if (!phase_o(a, l, tick, pos, tok, wg, G, s, sg)) return false;
@@ -47,8 +48,10 @@ __device__ __forceinline__ bool is_stop(const RunDesc& r, uint32_t tok) {
 // code, same token), so no broadcast is needed. RANDOM: the run samples at a
 // temperature above 0 (the host launches the instance that matches the run's
 // temperature); the greedy instance holds none of the random sampler's code,
-// whose registers would otherwise crowd the forward's.
-template <bool RANDOM>
+// whose registers would otherwise crowd the forward's. TRACE: fed runs that
+// also keep every layer's queries (an instance of its own for the same
+// reason).
+template <bool RANDOM, bool TRACE>
 __global__ __launch_bounds__(BLOCK) void k_persistent(const Args* __restrict__ ap,
                                                       const RunDesc* __restrict__ run) {
   const Args& a = *ap;
@@ -109,7 +112,7 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(const Args* __restrict__ a
       const Lds sf = lds_layout(lds_raw, dl);
       const Stager sgt = make_stager(a, sf, wgt, G, a.d.lds_stg != 0);
       if (!forward_all(a, tok, pos, tick, wgt, G, sf, sgt)) break;
-    } else if (!forward_all(a, tok, pos, tick, wg, G, s, sg)) {
+    } else if (!forward_all<TRACE>(a, tok, pos, tick, wg, G, s, sg, r.trace_q)) {
       break;
     }
     ++pos;
@@ -130,7 +133,8 @@ __global__ __launch_bounds__(BLOCK) void k_persistent(const Args* __restrict__ a
   // Staged loads of a layer that will not run land before the wave ends.
   if (sg.on && sg.loader) stage_wait(0);
 }
-template __global__ void k_persistent<false>(const Args* __restrict__, const RunDesc* __restrict__);
-template __global__ void k_persistent<true>(const Args* __restrict__, const RunDesc* __restrict__);
+template __global__ void k_persistent<false, false>(const Args* __restrict__, const RunDesc* __restrict__);
+template __global__ void k_persistent<true, false>(const Args* __restrict__, const RunDesc* __restrict__);
+template __global__ void k_persistent<false, true>(const Args* __restrict__, const RunDesc* __restrict__);
 
 }  // namespace DG_NS

@@ -877,10 +877,12 @@ __device__ __forceinline__ float4 qkv_epi_load(const Args& a, uint32_t l, uint32
 constexpr uint32_t QKV_PRE = 2;  // epilogue inputs a compute wave loads before the wait
 
 // rmsnorm -> q/k/v rows (+bias) -> RoPE on q and k (model.rs:460-465) ->
-// k, v appended to the cache at `pos` (model.rs:466-467).
+// k, v appended to the cache at `pos` (model.rs:466-467). TRACE: the layer's
+// rotated queries also go to trace_q (nullable) [L][q].
+template <bool TRACE = false>
 __device__ __forceinline__ bool phase_qkv(const Args& a, uint32_t l, uint32_t tick, uint32_t pos,
                                           uint32_t token, uint32_t wg, uint32_t G, const Lds& s,
-                                          const Stager& sg) {
+                                          const Stager& sg, float* trace_q = nullptr) {
   const Dims d = shape_dims(a.d);
   const uint32_t lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
   const MvWaves mw = mv_waves(sg, wave, a, IK_QKV, wg, G);
@@ -948,6 +950,9 @@ __device__ __forceinline__ bool phase_qkv(const Args& a, uint32_t l, uint32_t ti
         float* row = (is_k ? a.kc : a.vc) + (((size_t)l * d.nkv + g) * d.cap + pos) * d.kvs;
         pub_float(pub, 4 * k, row + i, a0, lane);
         pub_float(pub, 4 * k + 1, row + i + d.half, a1, lane);
+      } else if (TRACE && trace_q) {
+        pub_float(pub, 4 * k, trace_q + (size_t)l * d.q + r0, a0, lane);
+        pub_float(pub, 4 * k + 1, trace_q + (size_t)l * d.q + r1, a1, lane);
       } else {
         pub_none(pub, 4 * k, lane);
         pub_none(pub, 4 * k + 1, lane);
