@@ -87,13 +87,42 @@ static std::atomic<uint64_t> g_live_models{0}, g_live_caches{0}, g_devices_used{
 #include "batch.h"
 
 // Per-run reset of the counters (pos / tick / token are kept).
-__global__ void k_begin(DevState* st) {
+__device__ __forceinline__ void reset_counters(DevState* st) {
   st->abort = 0;
   st->halt = 0;
   st->n_done = 0;
   st->op = 0;
   st->first_div = -1;
   st->sampled_div = 0;
+}
+__global__ void k_begin(DevState* st) { reset_counters(st); }
+
+// Everything a run starts from, handed over as kernel arguments: the cache's
+// length and generation base (the host's copy is the authority, so a
+// truncation touches no device memory), the run's description, its mask and,
+// for short runs, its tokens and rng words. Copies of each took a forward
+// of the 135M shape 628 us where its kernel takes 505 (565 now).
+constexpr uint32_t BEGIN_WORDS = 16;
+struct RunBegin {
+  DevState* st;
+  Args* args;
+  RunDesc* run;
+  const uint32_t* mask;
+  uint32_t *tokens, *words;      // device destinations
+  uint32_t pos, tick, n_tokens, n_words;
+  uint32_t token[BEGIN_WORDS], word[BEGIN_WORDS];
+  RunDesc desc;
+};
+__global__ void k_begin_run(const RunBegin b) {
+  const uint32_t i = threadIdx.x;
+  if (i < b.n_tokens) b.tokens[i] = b.token[i];
+  if (i < b.n_words) b.words[i] = b.word[i];
+  if (i != 0) return;
+  reset_counters(b.st);
+  b.st->pos = b.pos;
+  b.st->tick = b.tick;
+  b.args->mask = b.mask;
+  *b.run = b.desc;
 }
 
 enum : uint32_t { PH_LM_KERNEL = 100 };
@@ -250,22 +279,12 @@ __global__ __launch_bounds__(256) void k_trace(const Args* __restrict__ ap, uint
   for (uint32_t t = threadIdx.x; t < n; t += blockDim.x) o[t] = o[t] / S;
 }
 
-// Length and generation base of many caches at once (batched calls).
+// A cache of a batch commit: its tagged logits and chunk maxima, filled from
+// workspace logits row li.
 struct StateSet {
-  DevState* st;
-  uint32_t pos, tick;
-  // batch commits: the cache's tagged logits and chunk maxima, filled from
-  // workspace logits row li
   u64 *logit, *vmax, *varg;
   uint32_t li;
 };
-__global__ void k_set_state(const StateSet* __restrict__ set, uint32_t n) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
-  set[k].st->pos = set[k].pos;
-  set[k].st->tick = set[k].tick;
-}
-
 // Batch commit: cache k's tagged logits and chunk (max, argmax) words from
 // the workspace's logits row set[k].li, all caches in one launch (grid y = k).
 __global__ void k_commit_rows(const StateSet* __restrict__ set, const u64* __restrict__ logt,
@@ -315,9 +334,9 @@ __global__ __launch_bounds__(VCHUNK) void k_set_logits(const Args* __restrict__ 
   }
 }
 
-// Strip the tags of logits (or any tagged vector) into plain floats.
-__global__ void k_untag(const u64* src, float* dst, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// Strip the tags of logits (or any tagged words) into plain floats.
+__global__ void k_untag(const u64* src, float* dst, size_t n) {
+  const size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   if (i < n) dst[i] = __uint_as_float((uint32_t)src[i]);
 }
 
@@ -462,6 +481,7 @@ struct defer_gpu_cache {
   u64* mb = nullptr;
   size_t mb_words = 0;
   DevState* st = nullptr;
+  DevState* h_st = nullptr;  // pinned: the state as a run left it
   RunDesc* d_run = nullptr;
   uint32_t* d_mask = nullptr;
   uint32_t* d_tokens = nullptr;
@@ -941,6 +961,7 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   HIP_TRY(hipMemset(c->mb, 0, words * sizeof(u64)));
   HIP_TRY(counted_malloc(&c->st, sizeof(DevState)));
   HIP_TRY(hipMemset(c->st, 0, sizeof(DevState)));
+  HIP_TRY(counted_host_malloc((void**)&c->h_st, sizeof(DevState), hipHostMallocDefault));
   HIP_TRY(counted_malloc(&c->d_run, sizeof(RunDesc)));
   HIP_TRY(counted_malloc(&c->d_mask, ((cap + 31) / 32) * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&c->d_logits, (size_t)d.V * sizeof(float)));
@@ -977,11 +998,6 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   return DEFER_GPU_OK;
 }
 
-static int sync_args(defer_gpu_cache* c) {
-  HIP_TRY(hipMemcpy(c->d_args, &c->args, sizeof(Args), hipMemcpyHostToDevice));
-  return DEFER_GPU_OK;
-}
-
 static void cache_free(defer_gpu_cache* c) {
   if (!c) return;
   --g_live_caches;  // every cache_free follows a cache_alloc
@@ -1002,6 +1018,7 @@ static void cache_free(defer_gpu_cache* c) {
   (void)hipFree(c->d_tmp);
   (void)hipFree(c->d_trace);
   (void)hipFree(c->d_norms);
+  if (c->h_st) (void)hipHostFree(c->h_st);
   (void)hipFree(c->d_args);
   if (c->h_ring) (void)hipHostFree(c->h_ring);
 }
@@ -1034,21 +1051,12 @@ extern "C" void defer_gpu_cache_destroy(defer_gpu_cache* c) {
 extern "C" uint32_t defer_gpu_cache_len(const defer_gpu_cache* c) { return c ? c->pos : 0; }
 extern "C" uint32_t defer_gpu_cache_capacity(const defer_gpu_cache* c) { return c ? c->cap : 0; }
 
-static int push_state(defer_gpu_cache* c) {
-  DevState h;
-  HIP_TRY(hipMemcpy(&h, c->st, sizeof(h), hipMemcpyDeviceToHost));
-  h.pos = c->pos;
-  h.tick = c->tick;
-  HIP_TRY(hipMemcpy(c->st, &h, sizeof(h), hipMemcpyHostToDevice));
-  return DEFER_GPU_OK;
-}
-
 extern "C" int defer_gpu_cache_truncate(defer_gpu_cache* c, uint32_t n) {
   if (!c) return fail(DEFER_GPU_E_INVALID, "null cache");
   if (n >= c->pos) return DEFER_GPU_OK;
   c->pos = n;
   c->has_logits = false;
-  return push_state(c);
+  return DEFER_GPU_OK;
 }
 
 extern "C" int defer_gpu_cache_clone(const defer_gpu_cache* src, defer_gpu_cache** out) {
@@ -1195,18 +1203,54 @@ static int launch_op_kernels(defer_gpu_cache* c, hipStream_t s, float* trace_q) 
   return DEFER_GPU_OK;
 }
 
+// What a run takes from the host: tokens and rng words (copied to the run's
+// device buffers, short ones as kernel arguments), the mask (device).
+struct RunInput {
+  const uint32_t* tokens = nullptr;
+  size_t n_tokens = 0;
+  const uint32_t* words = nullptr;
+  size_t n_words = 0;
+  const uint32_t* mask = nullptr;
+  bool no_graph = false;
+};
+static int run_begin(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
+  const hipStream_t s = c->m->stream;
+  RunBegin b;
+  memset(&b, 0, sizeof(b));
+  b.st = c->st;
+  b.args = c->d_args;
+  b.run = c->d_run;
+  b.mask = in.mask;
+  b.tokens = const_cast<uint32_t*>(r.tokens);
+  b.words = const_cast<uint32_t*>(r.words);
+  b.pos = c->pos;
+  b.tick = c->tick;
+  b.desc = r;
+  auto put = [&](const uint32_t* src, size_t n, uint32_t* dev, uint32_t* arg, uint32_t* n_arg) {
+    if (n > BEGIN_WORDS) return hipMemcpyAsync(dev, src, n * sizeof(uint32_t), hipMemcpyHostToDevice, s);
+    if (n) memcpy(arg, src, n * sizeof(uint32_t));
+    *n_arg = (uint32_t)n;
+    return hipSuccess;
+  };
+  HIP_TRY(put(in.tokens, in.n_tokens, b.tokens, b.token, &b.n_tokens));
+  HIP_TRY(put(in.words, in.n_words, b.words, b.word, &b.n_words));
+  k_begin_run<<<1, WAVE, 0, s>>>(b);
+  HIP_TRY(hipGetLastError());
+  return DEFER_GPU_OK;
+}
+
 // Queues n_ops ops described by `r` (host copy, device pointers filled in)
-// on the model's stream; run_finish waits for them. no_graph: the phase kernels
-// one by one where the mode is a graph.
-static int run_launch(defer_gpu_cache* c, RunDesc r, bool no_graph = false) {
+// on the model's stream, then the copy of the state they leave; run_finish
+// waits for them. in.no_graph: the phase kernels one by one where the mode is
+// a graph.
+static int run_launch(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
   defer_gpu_model* m = const_cast<defer_gpu_model*>(c->m);
   const hipStream_t s = m->stream;
-  HIP_TRY(hipMemcpyAsync(c->d_run, &r, sizeof(r), hipMemcpyHostToDevice, s));
-  k_begin<<<1, 1, 0, s>>>(c->st);
-  HIP_TRY(hipGetLastError());
+  const int rb = run_begin(c, r, in);
+  if (rb) return rb;
   HIP_TRY(hipEventRecord(m->ev0, s));
   const uint32_t mode =
-      no_graph && m->exec_mode == DEFER_GPU_EXEC_GRAPH ? (uint32_t)DEFER_GPU_EXEC_EAGER : m->exec_mode;
+      in.no_graph && m->exec_mode == DEFER_GPU_EXEC_GRAPH ? (uint32_t)DEFER_GPU_EXEC_EAGER : m->exec_mode;
   if (r.n_ops > 0) {
     if (mode == DEFER_GPU_EXEC_PERSISTENT) {
       const Args* a = c->d_args;
@@ -1248,6 +1292,7 @@ static int run_launch(defer_gpu_cache* c, RunDesc r, bool no_graph = false) {
     }
   }
   HIP_TRY(hipEventRecord(m->ev1, s));
+  HIP_TRY(hipMemcpyAsync(c->h_st, c->st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   return DEFER_GPU_OK;
 }
 
@@ -1257,8 +1302,7 @@ static int run_finish(defer_gpu_cache* c) {
   float ms = 0.0f;
   HIP_TRY(hipEventElapsedTime(&ms, m->ev0, m->ev1));
   m->last_ms = ms;
-  DevState h;
-  HIP_TRY(hipMemcpy(&h, c->st, sizeof(h), hipMemcpyDeviceToHost));
+  const DevState& h = *c->h_st;
   if (h.abort) {
     c->has_logits = false;
     return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound; cache state is undefined");
@@ -1269,16 +1313,9 @@ static int run_finish(defer_gpu_cache* c) {
   return DEFER_GPU_OK;
 }
 
-static int run_ops(defer_gpu_cache* c, RunDesc r, bool no_graph = false) {
-  const int rc = run_launch(c, r, no_graph);
+static int run_ops(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
+  const int rc = run_launch(c, r, in);
   return rc ? rc : run_finish(c);
-}
-
-static DevState read_state(defer_gpu_cache* c) {
-  DevState h;
-  memset(&h, 0, sizeof(h));
-  if (hipMemcpy(&h, c->st, sizeof(h), hipMemcpyDeviceToHost) != hipSuccess) h.first_div = -2;
-  return h;
 }
 
 static int check_pair(const defer_gpu_model* m, const defer_gpu_cache* c) {
@@ -1287,13 +1324,13 @@ static int check_pair(const defer_gpu_model* m, const defer_gpu_cache* c) {
   return DEFER_GPU_OK;
 }
 
-static int copy_logits(defer_gpu_cache* c, float* out) {
+// Queues the copy of the last logits to the host.
+static int queue_logits(defer_gpu_cache* c, float* out) {
   const Dims& d = c->m->d;
   const hipStream_t s = c->m->stream;
   k_untag<<<(d.V + 255) / 256, 256, 0, s>>>(c->args.mb_logit, c->d_logits, d.V);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpyAsync(out, c->d_logits, (size_t)d.V * sizeof(float), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
   return DEFER_GPU_OK;
 }
 
@@ -1315,18 +1352,17 @@ extern "C" int defer_gpu_last_logits(const defer_gpu_cache* cc, float* logits_ou
   defer_gpu_cache* c = const_cast<defer_gpu_cache*>(cc);
   if (!c || !logits_out) return fail(DEFER_GPU_E_INVALID, "null argument");
   if (!c->has_logits) return fail(DEFER_GPU_E_NO_LOGITS, "no context: provide a non-empty prompt");
-  return copy_logits(c, logits_out);
+  const int rc = queue_logits(c, logits_out);
+  if (rc) return rc;
+  HIP_TRY(hipStreamSynchronize(c->m->stream));
+  return DEFER_GPU_OK;
 }
 
-static int feed_tokens(const defer_gpu_model* m, defer_gpu_cache* c, const uint32_t* tokens,
-                       size_t n, bool no_graph = false, float* trace_q = nullptr) {
-  for (size_t i = 0; i < n; ++i)
-    if (tokens[i] >= m->d.V) return fail(DEFER_GPU_E_TOKEN, "token id %u out of range", tokens[i]);
-  if ((size_t)c->pos + n > c->cap)
-    return fail(DEFER_GPU_E_CONTEXT, "context length %u exceeded", m->cfg.max_seq_len);
+// Queues a run that feeds tokens[0..n) (checked by the caller).
+static int feed_launch(defer_gpu_cache* c, const uint32_t* tokens, size_t n, RunInput in = {},
+                       float* trace_q = nullptr) {
   int rc = ensure_run_buffers(c, n, 0);
   if (rc) return rc;
-  if (n) HIP_TRY(hipMemcpy(c->d_tokens, tokens, n * sizeof(uint32_t), hipMemcpyHostToDevice));
   RunDesc r;
   memset(&r, 0, sizeof(r));
   r.n_ops = (uint32_t)n;
@@ -1337,7 +1373,18 @@ static int feed_tokens(const defer_gpu_model* m, defer_gpu_cache* c, const uint3
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
   r.trace_q = trace_q;
-  return run_ops(c, r, no_graph);
+  in.tokens = tokens;
+  in.n_tokens = n;
+  return run_launch(c, r, in);
+}
+
+static int feed_tokens(const defer_gpu_model* m, defer_gpu_cache* c, const uint32_t* tokens, size_t n) {
+  for (size_t i = 0; i < n; ++i)
+    if (tokens[i] >= m->d.V) return fail(DEFER_GPU_E_TOKEN, "token id %u out of range", tokens[i]);
+  if ((size_t)c->pos + n > c->cap)
+    return fail(DEFER_GPU_E_CONTEXT, "context length %u exceeded", m->cfg.max_seq_len);
+  const int rc = feed_launch(c, tokens, n);
+  return rc ? rc : run_finish(c);
 }
 
 extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, uint32_t token,
@@ -1360,35 +1407,28 @@ extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, u
       HIP_TRY(hipMemcpy(c->d_mask, bits.data(), bits.size() * sizeof(uint32_t),
                         hipMemcpyHostToDevice));
   }
-  if (use_mask) {
-    c->args.mask = c->d_mask;
-    rc = sync_args(c);
-    if (rc) return rc;
-  }
   const uint32_t pos0 = c->pos;
+  const hipStream_t s = m->stream;
   const size_t n_probs = (size_t)m->d.L * m->d.nh * c->cap;
   if (trace_out && !c->d_trace)
-    rc = counted_malloc(&c->d_trace, (n_probs + (size_t)m->d.L * m->d.q) * sizeof(float)) == hipSuccess
-             ? DEFER_GPU_OK
-             : fail(DEFER_GPU_E_HIP, "trace allocation failed");
+    HIP_TRY(counted_malloc(&c->d_trace, (n_probs + (size_t)m->d.L * m->d.q) * sizeof(float)));
   float* tq = trace_out ? c->d_trace + n_probs : nullptr;
-  // The captured graph's kernels keep no queries.
-  if (!rc) rc = feed_tokens(m, c, &token, 1, use_mask || trace_out, tq);
-  if (!rc && trace_out) {
-    k_trace<<<dim3(m->d.nh, m->d.L), 256, 0, m->stream>>>(c->d_args, pos0, tq, c->d_trace);
-    rc = hipMemcpyAsync(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
-                        hipMemcpyDeviceToHost, m->stream) == hipSuccess &&
-                 hipStreamSynchronize(m->stream) == hipSuccess
-             ? DEFER_GPU_OK
-             : fail(DEFER_GPU_E_HIP, "trace copy failed");
-  }
-  if (use_mask) {
-    c->args.mask = nullptr;
-    const int rc2 = sync_args(c);
-    if (!rc) rc = rc2;
-  }
+  RunInput in;
+  in.mask = use_mask ? c->d_mask : nullptr;
+  in.no_graph = use_mask || trace_out;  // the captured graph's kernels keep no queries
+  rc = feed_launch(c, &token, 1, in, tq);
   if (rc) return rc;
-  return logits_out ? copy_logits(c, logits_out) : DEFER_GPU_OK;
+  // The results' copies are queued behind the run: one wait for all.
+  if (trace_out) {
+    k_trace<<<dim3(m->d.nh, m->d.L), 256, 0, s>>>(c->d_args, pos0, tq, c->d_trace);
+    HIP_TRY(hipMemcpyAsync(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
+                           hipMemcpyDeviceToHost, s));
+  }
+  if (logits_out) {
+    rc = queue_logits(c, logits_out);
+    if (rc) return rc;
+  }
+  return run_finish(c);
 }
 
 static bool use_batch(const defer_gpu_model* m, size_t n);
@@ -1472,8 +1512,9 @@ extern "C" int defer_gpu_generate(const defer_gpu_model* m, defer_gpu_cache* c, 
   if (!tokens_out) return fail(DEFER_GPU_E_INVALID, "null tokens_out");
   rc = ensure_run_buffers(c, n, n_stop);
   if (rc) return rc;
-  if (temperature != 0.0f)
-    HIP_TRY(hipMemcpy(c->d_words, rng_words, n * sizeof(uint32_t), hipMemcpyHostToDevice));
+  RunInput in;
+  in.words = rng_words;
+  in.n_words = temperature != 0.0f ? n : 0;
   if (n_stop) HIP_TRY(hipMemcpy(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice));
   RunDesc r;
   memset(&r, 0, sizeof(r));
@@ -1488,9 +1529,9 @@ extern "C" int defer_gpu_generate(const defer_gpu_model* m, defer_gpu_cache* c, 
   r.words = c->d_words;
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
-  rc = run_ops(c, r);
+  rc = run_ops(c, r, in);
   if (rc) return rc;
-  const DevState h = read_state(c);
+  const DevState h = *c->h_st;
   if (h.n_done) HIP_TRY(hipMemcpy(tokens_out, c->d_out, h.n_done * sizeof(uint32_t),
                                   hipMemcpyDeviceToHost));
   if (n_out) *n_out = h.n_done;
@@ -1540,8 +1581,9 @@ extern "C" int defer_gpu_generate_cb(const defer_gpu_model* m, defer_gpu_cache* 
   rc = ensure_ring(c, n);
   if (rc) return rc;
   memset(c->h_ring, 0, n * sizeof(u64));  // no index tag is 0
-  if (temperature != 0.0f)
-    HIP_TRY(hipMemcpy(c->d_words, rng_words, n * sizeof(uint32_t), hipMemcpyHostToDevice));
+  RunInput in;
+  in.words = rng_words;
+  in.n_words = temperature != 0.0f ? n : 0;
   if (n_stop) HIP_TRY(hipMemcpy(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice));
   const uint32_t pos0 = c->pos;
   RunDesc r;
@@ -1558,7 +1600,7 @@ extern "C" int defer_gpu_generate_cb(const defer_gpu_model* m, defer_gpu_cache* 
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
   r.ring = c->d_ring;
-  rc = run_launch(c, r);
+  rc = run_launch(c, r, in);
   if (rc) return rc;
   // Hand each committed token to on_token, in order, as it lands; the run
   // is over once the stream is idle and the slot after the last is unset.
@@ -1585,7 +1627,7 @@ extern "C" int defer_gpu_generate_cb(const defer_gpu_model* m, defer_gpu_cache* 
   }
   rc = run_finish(c);
   if (rc) return rc;
-  const DevState h = read_state(c);
+  const DevState h = *c->h_st;
   if (cb_rc != 0) {
     // on_token failed at token next - 1: as the reference's generate returns
     // there, the call ends with the tokens up to it; the ones the device ran
@@ -1730,9 +1772,11 @@ extern "C" int defer_gpu_generate_static(const defer_gpu_model* m, defer_gpu_cac
   r.out_tokens = d_out;
   // A graph would be instantiated (allocated) on first use: in graph mode the
   // same phase kernels run one by one instead (identical bits).
-  rc = run_ops(c, r, true);
+  RunInput in;  // the words are staged above
+  in.no_graph = true;
+  rc = run_ops(c, r, in);
   if (rc) return rc;
-  const DevState h = read_state(c);
+  const DevState h = *c->h_st;
   if (h.n_done) HIP_TRY(hipMemcpy(tokens_out, d_out, h.n_done * sizeof(uint32_t), hipMemcpyDeviceToHost));
   if (n_out) *n_out = h.n_done;
   if (n < max_tokens && !h.halt)
@@ -1752,7 +1796,9 @@ extern "C" int defer_gpu_sample(const defer_gpu_model* m, defer_gpu_cache* c, fl
   if (!token_out) return fail(DEFER_GPU_E_INVALID, "null token_out");
   rc = ensure_run_buffers(c, 1, 0);
   if (rc) return rc;
-  HIP_TRY(hipMemcpy(c->d_words, &rng_word, sizeof(uint32_t), hipMemcpyHostToDevice));
+  RunInput in;
+  in.words = &rng_word;
+  in.n_words = 1;
   RunDesc r;
   memset(&r, 0, sizeof(r));
   r.n_ops = 1;
@@ -1765,13 +1811,14 @@ extern "C" int defer_gpu_sample(const defer_gpu_model* m, defer_gpu_cache* c, fl
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
   const hipStream_t s = m->stream;
-  HIP_TRY(hipMemcpyAsync(c->d_run, &r, sizeof(r), hipMemcpyHostToDevice, s));
-  k_begin<<<1, 1, 0, s>>>(c->st);
+  rc = run_begin(c, r, in);
+  if (rc) return rc;
   k_samp_a<<<m->G, BLOCK, m->lds_bytes, s>>>(c->d_args, c->d_run);
   k_op<<<1, BLOCK, m->lds_bytes, s>>>(c->d_args, c->d_run);
   HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(c->h_st, c->st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  const DevState h = read_state(c);
+  const DevState h = *c->h_st;
   if (h.abort) return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound");
   HIP_TRY(hipMemcpy(token_out, c->d_out, sizeof(uint32_t), hipMemcpyDeviceToHost));
   return DEFER_GPU_OK;
@@ -1812,11 +1859,12 @@ extern "C" int defer_gpu_replay(const defer_gpu_model* m, defer_gpu_cache* c,
     });
   rc = ensure_run_buffers(c, n_history, 0);
   if (rc) return rc;
-  if (n_history)
-    HIP_TRY(hipMemcpy(c->d_tokens, history, n_history * sizeof(uint32_t), hipMemcpyHostToDevice));
   const size_t n_sampled = n_history - prompt_len;
-  if (n_sampled && temperature != 0.0f)
-    HIP_TRY(hipMemcpy(c->d_words, rng_words, n_sampled * sizeof(uint32_t), hipMemcpyHostToDevice));
+  RunInput in;
+  in.tokens = history;
+  in.n_tokens = n_history;
+  in.words = rng_words;
+  in.n_words = temperature != 0.0f ? n_sampled : 0;
   RunDesc r;
   memset(&r, 0, sizeof(r));
   r.n_ops = (uint32_t)n_history;
@@ -1829,9 +1877,9 @@ extern "C" int defer_gpu_replay(const defer_gpu_model* m, defer_gpu_cache* c,
   r.words = c->d_words;
   r.stop = c->d_stop;
   r.out_tokens = c->d_out;
-  rc = run_ops(c, r);
+  rc = run_ops(c, r, in);
   if (rc) return rc;
-  const DevState h = read_state(c);
+  const DevState h = *c->h_st;
   if (h.first_div >= 0) {
     if (first_div) *first_div = h.first_div;
     if (sampled_at_div) *sampled_at_div = h.sampled_div;
@@ -1853,22 +1901,28 @@ struct BatchWs {
   float* LINV = nullptr;
   u64 *QKVT = nullptr, *PART = nullptr, *LOGT = nullptr, *VMAX = nullptr, *VARG = nullptr,
       *VSUM = nullptr, *VP = nullptr;
-  BRow* drows = nullptr;
-  Args* rargs = nullptr;
-  Args* largs = nullptr;
-  uint32_t *sel = nullptr, *lgen = nullptr, *stick = nullptr, *swords = nullptr, *sout = nullptr;
-  uint32_t* items = nullptr;  // attention (row, item) list, or tiled attention tasks
-  uint32_t* tiles = nullptr;  // tiled attention: first batch row of each tile
-  StateSet* sets = nullptr;   // [rows] cache states to set after a batch
+  uint32_t* sout = nullptr;
   DevState* st = nullptr;
+  float* LOGF = nullptr;  // untagged logits of a batch that returns them
+  size_t logf_cap = 0;
+  // A batch's small host arrays (rows, tasks, ...) go to the device as one
+  // copy per stage, from pinned memory: h_up is filled in order and copied to
+  // the same offsets of d_up. Reset at the start of a call, when the stream
+  // is idle.
+  char *h_up = nullptr, *d_up = nullptr;
+  size_t up_cap = 0, up_used = 0, up_sent = 0;
+  DevState* h_st = nullptr;   // pinned
+  uint32_t* h_out = nullptr;  // pinned [lm]: sampled tokens
 };
 
 static void batch_ws_release(BatchWs* w) {
   if (!w) return;
   void* ps[] = {w->X, w->Y, w->INV, w->XP, w->XQ, w->LINV, w->QKVT, w->PART,
-                w->LOGT, w->VMAX, w->VARG, w->VSUM, w->VP, w->drows, w->rargs, w->largs, w->sel,
-                w->lgen, w->stick, w->swords, w->sout, w->items, w->tiles, w->sets, w->st};
+                w->LOGT, w->VMAX, w->VARG, w->VSUM, w->VP, w->sout, w->d_up, w->LOGF, w->st};
   for (void* p : ps) (void)hipFree(p);
+  if (w->h_up) (void)hipHostFree(w->h_up);
+  if (w->h_st) (void)hipHostFree(w->h_st);
+  if (w->h_out) (void)hipHostFree(w->h_out);
   *w = BatchWs();
 }
 
@@ -1896,11 +1950,6 @@ static int ensure_ws(defer_gpu_model* m, uint32_t rows, uint32_t lm) {
   HIP_TRY(counted_malloc(&w.XP, panel_floats(R, d.h) * sizeof(float)));
   HIP_TRY(counted_malloc(&w.QKVT, (size_t)R * d.qkv_rows * sizeof(u64)));
   HIP_TRY(counted_malloc(&w.PART, (size_t)R * part_words(d) * sizeof(u64)));
-  HIP_TRY(counted_malloc(&w.drows, (size_t)R * sizeof(BRow)));
-  HIP_TRY(counted_malloc(&w.rargs, (size_t)R * sizeof(Args)));
-  HIP_TRY(counted_malloc(&w.items, (size_t)R * d.nkv * MAX_ACHUNKS * d.group * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.tiles, ((size_t)R / 16 + 3) * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.sets, (size_t)R * sizeof(StateSet)));
   const uint32_t L1 = std::max(Lm, 1u);
   HIP_TRY(counted_malloc(&w.XQ, panel_floats(std::max(R, L1), kmax) * sizeof(float)));
   HIP_TRY(counted_malloc(&w.LINV, (size_t)L1 * sizeof(float)));
@@ -1909,21 +1958,50 @@ static int ensure_ws(defer_gpu_model* m, uint32_t rows, uint32_t lm) {
   HIP_TRY(counted_malloc(&w.VARG, (size_t)L1 * d.nvc * sizeof(u64)));
   HIP_TRY(counted_malloc(&w.VSUM, (size_t)L1 * 3 * d.nvc * sizeof(u64)));
   HIP_TRY(counted_malloc(&w.VP, (size_t)L1 * d.V * sizeof(u64)));
-  HIP_TRY(counted_malloc(&w.largs, (size_t)L1 * sizeof(Args)));
-  HIP_TRY(counted_malloc(&w.sel, (size_t)L1 * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.lgen, (size_t)L1 * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.stick, (size_t)L1 * sizeof(uint32_t)));
-  HIP_TRY(counted_malloc(&w.swords, (size_t)L1 * sizeof(uint32_t)));
+  // Rows with their arguments, attention items (at most a row's kv heads by
+  // chunks) and tiles, the commit's caches; logits rows with the sampler's
+  // arguments; each array padded to 256 bytes.
+  w.up_cap = (size_t)R * (sizeof(BRow) + sizeof(Args) + (size_t)d.nkv * MAX_ACHUNKS * 4 + sizeof(StateSet) + 4) +
+             (size_t)L1 * (sizeof(Args) + 16) + 16 * 256;
+  HIP_TRY(counted_host_malloc((void**)&w.h_up, w.up_cap, hipHostMallocDefault));
+  HIP_TRY(counted_malloc(&w.d_up, w.up_cap));
+  HIP_TRY(counted_host_malloc((void**)&w.h_st, sizeof(DevState), hipHostMallocDefault));
+  HIP_TRY(counted_host_malloc((void**)&w.h_out, (size_t)L1 * sizeof(uint32_t), hipHostMallocDefault));
   HIP_TRY(counted_malloc(&w.sout, (size_t)L1 * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&w.st, sizeof(DevState)));
-  HIP_TRY(hipMemset(w.st, 0, sizeof(DevState)));
-  // Tags start at 1, so zeroed sums never match a wait; sampled tokens
+  HIP_TRY(hipMemsetAsync(w.st, 0, sizeof(DevState), m->stream));
+  // Cleared on the stream that uses them (a clear on the null stream could
+  // land after the first batch's words). Tags start at 1, so zeroed sums never match a wait; sampled tokens
   // start in range.
-  HIP_TRY(hipMemset(w.VSUM, 0, (size_t)L1 * 3 * d.nvc * sizeof(u64)));
-  HIP_TRY(hipMemset(w.VP, 0, (size_t)L1 * d.V * sizeof(u64)));
-  HIP_TRY(hipMemset(w.sout, 0, (size_t)L1 * sizeof(uint32_t)));
+  HIP_TRY(hipMemsetAsync(w.VSUM, 0, (size_t)L1 * 3 * d.nvc * sizeof(u64), m->stream));
+  HIP_TRY(hipMemsetAsync(w.VP, 0, (size_t)L1 * d.V * sizeof(u64), m->stream));
+  HIP_TRY(hipMemsetAsync(w.sout, 0, (size_t)L1 * sizeof(uint32_t), m->stream));
   w.rows = R;
   w.lm = Lm;
+  return DEFER_GPU_OK;
+}
+
+// An array for the device: where it will be once up_send has run.
+template <class T>
+static T* up_put(BatchWs& w, const T* src, size_t n) {
+  const size_t at = w.up_used, bytes = n * sizeof(T);
+  if (at + bytes > w.up_cap) return nullptr;
+  if (bytes) memcpy(w.h_up + at, src, bytes);
+  w.up_used = (at + bytes + 255) & ~(size_t)255;
+  return reinterpret_cast<T*>(w.d_up + at);
+}
+static int up_send(BatchWs& w, hipStream_t s) {
+  if (w.up_used > w.up_cap) w.up_used = w.up_cap;
+  if (w.up_used > w.up_sent)
+    HIP_TRY(hipMemcpyAsync(w.d_up + w.up_sent, w.h_up + w.up_sent, w.up_used - w.up_sent,
+                           hipMemcpyHostToDevice, s));
+  w.up_sent = w.up_used;
+  return DEFER_GPU_OK;
+}
+static int up_reset(defer_gpu_model* m) {
+  if (!m->bw) return DEFER_GPU_OK;
+  HIP_TRY(hipStreamSynchronize(m->stream));
+  m->bw->up_used = m->bw->up_sent = 0;
   return DEFER_GPU_OK;
 }
 
@@ -2080,7 +2158,7 @@ static Args row_args(const defer_gpu_cache* c, const BatchWs& w, uint32_t b) {
 // (its K/V rows then come from L2 once per head): 301 rows of the 135M shape
 // are 99 tasks, or 297 of one head.
 static void launch_attn_tile(defer_gpu_model* m, uint32_t nb, const uint32_t* items, uint32_t n_items,
-                             uint32_t l) {
+                             const BRow* rows, const uint32_t* tiles, uint32_t l) {
   const Dims& d = m->d;
   BatchWs& w = *m->bw;
   if (!n_items) return;
@@ -2090,7 +2168,7 @@ static void launch_attn_tile(defer_gpu_model* m, uint32_t nb, const uint32_t* it
   const float* qf = reinterpret_cast<const float*>(w.QKVT);
   float* part = reinterpret_cast<float*>(w.PART);
   Dims dv = d;
-  void* args[] = {&dv, &w.drows, &items, &ny, &nj, &w.tiles, &l, &qf, &part};
+  void* args[] = {&dv, &rows, &items, &ny, &nj, &tiles, &l, &qf, &part};
   (void)hipLaunchKernel(attn_tile_kernel(d.hd, nb), dim3(n_items * ny), dim3(256), args,
                         attn_tile_lds(d.hd, nb, nj), m->stream);
 }
@@ -2185,22 +2263,20 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   for (uint32_t b = 0; b < n; ++b) attn_flop += 4.0 * d.nh * d.hd * (rows[b].pos + 1.0);
   std::vector<uint32_t> lgen(nl);
   for (uint32_t i = 0; i < nl; ++i) lgen[i] = gen_lm(d, rows[sel[i]].tick);
-  HIP_TRY(hipMemcpyAsync(w.drows, rows, n * sizeof(BRow), hipMemcpyHostToDevice, s));
   // Every row's one-token arguments for attention items (else the first's
   // model pointers serve all rows).
   std::vector<Args> ra(tiled || fused ? 1 : n);
   for (uint32_t b = 0; b < ra.size(); ++b) ra[b] = row_args(rcache[b], w, b);
-  HIP_TRY(hipMemcpyAsync(w.rargs, ra.data(), ra.size() * sizeof(Args), hipMemcpyHostToDevice, s));
-  if (!items.empty())
-    HIP_TRY(hipMemcpyAsync(w.items, items.data(), items.size() * sizeof(uint32_t),
-                           hipMemcpyHostToDevice, s));
-  if (tiled)
-    HIP_TRY(hipMemcpyAsync(w.tiles, tiles.data(), tiles.size() * sizeof(uint32_t),
-                           hipMemcpyHostToDevice, s));
-  if (nl) {
-    HIP_TRY(hipMemcpyAsync(w.sel, sel, nl * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(w.lgen, lgen.data(), nl * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-  }
+  const BRow* drows = up_put(w, rows, n);
+  const Args* rargs = up_put(w, ra.data(), ra.size());
+  const uint32_t* d_items = up_put(w, items.data(), items.size());
+  const uint32_t* d_tiles = up_put(w, tiles.data(), tiles.size());
+  const uint32_t* d_sel = up_put(w, sel, nl);
+  const uint32_t* d_lgen = up_put(w, lgen.data(), nl);
+  if (!drows || !rargs || !d_items || !d_tiles || !d_sel || !d_lgen)
+    return fail(DEFER_GPU_E_HIP, "batch staging of %zu bytes exceeded", w.up_cap);
+  rc = up_send(w, s);
+  if (rc) return rc;
   if (!deferred) k_begin<<<1, 1, 0, s>>>(w.st);
   const uint32_t ldy = batch_ldy(d), ncu = m->gemm_ncu;
   // The QKV and gate/up products write what their consumers read -- rotated
@@ -2210,7 +2286,7 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   // launches to 6, a 2048-row one saves the 25 MB of gate and up rows.
   const bool act_out = d.ff % 16 == 0;
   const bool own_rms = act_out && n <= 16;  // the gate/up product forms the rows' 1/rms
-  k_b_embed<<<n, 256, 0, s>>>(w.drows, dtok, m->embed, d.h, w.X, w.XP);
+  k_b_embed<<<n, 256, 0, s>>>(drows, dtok, m->embed, d.h, w.X, w.XP);
   // 1/rms for the QKV product's outputs (k_b_attn_f forms its rows' own).
   if (!fused) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   for (uint32_t l = 0; l < d.L; ++l) {
@@ -2222,7 +2298,7 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       ProfSpan ps(m, 0, 2.0 * d.qkv_rows * d.h * n);
       if (tiled) {
         o.blk = d.half / 16;
-        o.rows = w.drows;
+        o.rows = drows;
         o.rope = m->rope;
         o.bias = m->layers[l].bqkv;
         o.qf = reinterpret_cast<float*>(w.QKVT);
@@ -2241,27 +2317,28 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       ProfSpan ps(m, 1, attn_flop);
       uint32_t li = l, ld = ldy;
       const float *xr = w.X, *yr = w.Y;
-      void* args[] = {&w.rargs, &w.drows, &li, &xr, &yr, &ld, &max_nch, &max_ch, &w.XQ};
+      void* args[] = {&rargs, &drows, &li, &xr, &yr, &ld, &max_nch, &max_ch, &w.XQ};
       HIP_TRY(hipLaunchKernel(attn_rows_kernel(d.hd, teams), dim3(n * d.nkv), dim3(teams * NCW * WAVE), args,
                               lds_rows_attn, s));
     } else {
       if (!tiled)
         k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
-            w.rargs, w.drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
+            rargs, drows, l, w.Y, ldy, w.INV, w.QKVT, d.qkv_rows);
       {
         ProfSpan ps(m, 1, attn_flop);
         if (tiled) {
-          launch_attn_tile(m, nb0, w.items, n_items0, l);
-          if (nb1 != nb0) launch_attn_tile(m, nb1, w.items + n_items0, (uint32_t)items.size() - n_items0, l);
+          launch_attn_tile(m, nb0, d_items, n_items0, drows, d_tiles, l);
+          if (nb1 != nb0)
+            launch_attn_tile(m, nb1, d_items + n_items0, (uint32_t)items.size() - n_items0, drows, d_tiles, l);
         } else {
-          k_b_attn_w<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(w.rargs, w.drows, w.items, l);
+          k_b_attn_w<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(rargs, drows, d_items, l);
         }
       }
       const dim3 comb_grid(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK);
       if (tiled)
-        k_b_comb<true><<<comb_grid, 256, 0, s>>>(d, w.drows, w.PART, part_words(d), w.XQ);
+        k_b_comb<true><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
       else
-        k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, w.drows, w.PART, part_words(d), w.XQ);
+        k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
     }
     GemmOutArgs x{};  // the residual rows and their panel
     x.Y = w.X;
@@ -2295,26 +2372,25 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     if (!fused && l + 1 < d.L) k_b_rms<<<(n + 3) / 4, 256, 0, s>>>(w.X, n, d.h, d.eps, w.INV);
   }
   if (nl) {
-    k_b_final<<<nl, 64, 0, s>>>(w.X, w.sel, d.h, m->norm, d.eps, w.XQ, w.LINV);
+    k_b_final<<<nl, 64, 0, s>>>(w.X, d_sel, d.h, m->norm, d.eps, w.XQ, w.LINV);
     {
       ProfSpan ps(m, 0, 2.0 * d.V * d.h * nl);
       GemmOutArgs o{};
       o.Y = reinterpret_cast<float*>(w.LOGT);
       o.ldy = d.V;
       o.inv = w.LINV;
-      o.gen = w.lgen;
+      o.gen = d_lgen;
       launch_gemm<GO_TAG>(s, ncu, m->p_lm, d.V, d.h, w.XQ, nl, o);
     }
-    k_b_chunkmax<<<dim3((d.nvc + 4 * CM_CPW - 1) / (4 * CM_CPW), nl), 256, 0, s>>>(d, w.LOGT, w.lgen, w.VMAX,
+    k_b_chunkmax<<<dim3((d.nvc + 4 * CM_CPW - 1) / (4 * CM_CPW), nl), 256, 0, s>>>(d, w.LOGT, d_lgen, w.VMAX,
                                                                                    w.VARG, nl);
   }
   HIP_TRY(hipGetLastError());
+  HIP_TRY(hipMemcpyAsync(w.h_st, w.st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   if (deferred && !m->prof) return DEFER_GPU_OK;
   HIP_TRY(hipStreamSynchronize(s));
   if (m->prof) prof_collect(m);
-  DevState h;
-  HIP_TRY(hipMemcpy(&h, w.st, sizeof(h), hipMemcpyDeviceToHost));
-  if (h.abort) return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound");
+  if (w.h_st->abort) return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound");
   return DEFER_GPU_OK;
 }
 
@@ -2350,63 +2426,68 @@ static int batch_sample(defer_gpu_model* m, defer_gpu_cache* const* ocache, cons
     a.mask = nullptr;
     la[j] = a;
   }
-  HIP_TRY(hipMemcpyAsync(w.largs, la.data(), nops * sizeof(Args), hipMemcpyHostToDevice, s));
-  HIP_TRY(hipMemcpyAsync(w.stick, tick, nops * sizeof(uint32_t), hipMemcpyHostToDevice, s));
-  if (T != 0.0f)
-    HIP_TRY(hipMemcpyAsync(w.swords, words, nops * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+  const Args* largs = up_put(w, la.data(), nops);
+  const uint32_t* stick = up_put(w, tick, nops);
+  const uint32_t* swords = T != 0.0f ? up_put(w, words, nops) : stick;
+  if (!largs || !stick || !swords) return fail(DEFER_GPU_E_HIP, "batch staging of %zu bytes exceeded", w.up_cap);
+  rc = up_send(w, s);
+  if (rc) return rc;
   k_begin<<<1, 1, 0, s>>>(w.st);
   const uint32_t tag0 = m->samp_next;
   m->samp_next += nops;
-  k_b_sample<<<nops, BLOCK, samp_lds_bytes(m), s>>>(w.largs, w.stick, w.swords, T, tag0, w.sout);
+  k_b_sample<<<nops, BLOCK, samp_lds_bytes(m), s>>>(largs, stick, swords, T, tag0, w.sout);
   HIP_TRY(hipGetLastError());
   if (deferred) return DEFER_GPU_OK;
-  HIP_TRY(hipMemcpyAsync(out, w.sout, nops * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(w.h_out, w.sout, nops * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  HIP_TRY(hipMemcpyAsync(w.h_st, w.st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   HIP_TRY(hipStreamSynchronize(s));
-  DevState h;
-  HIP_TRY(hipMemcpy(&h, w.st, sizeof(h), hipMemcpyDeviceToHost));
-  if (h.abort) return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound");
+  if (w.h_st->abort) return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound");
+  memcpy(out, w.h_out, nops * sizeof(uint32_t));
   return DEFER_GPU_OK;
 }
 
-// Caches after their batch rows: length, generation base and, from logits
-// row li[k] of the workspace, the tagged logits and chunk maxima a following
-// sample reads. One kernel copies every cache's words, one sets the device
-// states, then one synchronisation.
-static int batch_commit_many(defer_gpu_model* m, defer_gpu_cache* const* cs, const uint32_t* li,
-                             const uint32_t* pos, const uint32_t* tick, uint32_t n) {
+// Caches after their batch rows: from logits row li[k] of the workspace, the
+// tagged logits and chunk maxima a following sample reads (one kernel copies
+// every cache's words) ...
+static int queue_commit(defer_gpu_model* m, defer_gpu_cache* const* cs, const uint32_t* li, uint32_t n) {
   const Dims& d = m->d;
   const hipStream_t s = m->stream;
-  const BatchWs& w = *m->bw;
+  BatchWs& w = *m->bw;
   std::vector<StateSet> set(n);
   for (uint32_t k = 0; k < n; ++k) {
     defer_gpu_cache* c = cs[k];
-    set[k].st = c->st;
-    set[k].pos = pos[k];
-    set[k].tick = tick[k];
     set[k].logit = c->args.mb_logit;
     set[k].vmax = c->args.mb_vmax;
     set[k].varg = c->args.mb_varg;
     set[k].li = li[k];
   }
-  HIP_TRY(hipMemcpyAsync(w.sets, set.data(), n * sizeof(StateSet), hipMemcpyHostToDevice, s));
   if (n > 0) {
+    const StateSet* sets = up_put(w, set.data(), n);
+    if (!sets) return fail(DEFER_GPU_E_HIP, "batch staging of %zu bytes exceeded", w.up_cap);
+    const int rc = up_send(w, s);
+    if (rc) return rc;
     const uint32_t words = d.V + 2 * d.nvc;
     k_commit_rows<<<dim3(std::min((words + 1023) / 1024, 64u), n), 256, 0, s>>>(
-        w.sets, w.LOGT, w.VMAX, w.VARG, d.V, d.nvc);
+        sets, w.LOGT, w.VMAX, w.VARG, d.V, d.nvc);
   }
-  k_set_state<<<(n + 63) / 64, 64, 0, s>>>(w.sets, n);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipStreamSynchronize(s));
+  return DEFER_GPU_OK;
+}
+// ... and, once that has run, their length and generation base.
+static void commit_host(defer_gpu_cache* const* cs, const uint32_t* pos, const uint32_t* tick, uint32_t n) {
   for (uint32_t k = 0; k < n; ++k) {
     cs[k]->pos = pos[k];
     cs[k]->tick = tick[k];
     cs[k]->has_logits = true;
   }
-  return DEFER_GPU_OK;
 }
 static int batch_commit(defer_gpu_model* m, defer_gpu_cache* c, uint32_t li, uint32_t pos,
                         uint32_t tick) {
-  return batch_commit_many(m, &c, &li, &pos, &tick, 1);
+  const int rc = queue_commit(m, &c, &li, 1);
+  if (rc) return rc;
+  HIP_TRY(hipStreamSynchronize(m->stream));
+  commit_host(&c, &pos, &tick, 1);
+  return DEFER_GPU_OK;
 }
 
 static BRow make_row(const defer_gpu_cache* c, uint32_t pos, uint32_t tick, uint32_t token) {
@@ -2438,7 +2519,9 @@ static int feed_batched(defer_gpu_model* m, defer_gpu_cache* c, const uint32_t* 
     for (uint32_t j = 0; j < k; ++j) rows[j] = make_row(c, c->pos + j, c->tick + j, tokens[o + j]);
     const bool last = o + k == n;
     const uint32_t sel = k - 1;
-    int e = batch_run(m, rows.data(), rc.data(), k, &sel, last ? 1 : 0);
+    int e = up_reset(m);
+    if (e) return e;
+    e = batch_run(m, rows.data(), rc.data(), k, &sel, last ? 1 : 0);
     if (e) return e;
     if (last) {
       e = batch_commit(m, c, 0, c->pos + k, c->tick + k);
@@ -2447,8 +2530,6 @@ static int feed_batched(defer_gpu_model* m, defer_gpu_cache* c, const uint32_t* 
       c->pos += k;
       c->tick += k;
       c->has_logits = false;
-      e = push_state(c);
-      if (e) return e;
     }
   }
   return DEFER_GPU_OK;
@@ -2495,30 +2576,23 @@ static int forward_batch_impl(defer_gpu_model* m, defer_gpu_cache* const* caches
   int rc = batch_run(m, rows.data(), caches, n, sel.data(), (uint32_t)sel.size(), dtok, deferred);
   if (rc) return rc;
   HIP_TRY(hipEventRecord(m->ev1, m->stream));
-  if (deferred)
-    HIP_TRY(hipMemcpyAsync(tok_out, dtok, n * sizeof(uint32_t), hipMemcpyDeviceToHost, m->stream));
-  HIP_TRY(hipEventSynchronize(m->ev1));
-  float ms = 0.0f;
-  HIP_TRY(hipEventElapsedTime(&ms, m->ev0, m->ev1));
-  m->last_ms = ms;
-  if (deferred) {
-    // A wait that ran out leaves the rows undefined: nothing is committed.
-    DevState h;
-    HIP_TRY(hipMemcpy(&h, m->bw->st, sizeof(h), hipMemcpyDeviceToHost));
-    if (h.abort) {
-      for (uint32_t b = 0; b < n; ++b) caches[b]->has_logits = false;
-      return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound; cache state is undefined");
-    }
-  }
+  BatchWs& w = *m->bw;
+  const hipStream_t s = m->stream;
+  // The rest is queued behind the batch, with one wait for all of it.
+  if (deferred) HIP_TRY(hipMemcpyAsync(w.h_out, dtok, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   if (logits_out) {
-    const BatchWs& w = *m->bw;
-    for (uint32_t b = 0; b < n; ++b) {
-      float* dst = caches[b]->d_logits;  // [V] staging of the untagged row
-      k_untag<<<(d.V + 255) / 256, 256, 0, m->stream>>>(w.LOGT + (size_t)li_of[b] * d.V, dst, d.V);
-      HIP_TRY(hipMemcpyAsync(logits_out + (size_t)b * d.V, dst, (size_t)d.V * sizeof(float),
-                             hipMemcpyDeviceToHost, m->stream));
-      HIP_TRY(hipStreamSynchronize(m->stream));
+    // Every row has logits, in row order: untagged together and copied at
+    // once.
+    const size_t words = (size_t)n * d.V;
+    if (words > w.logf_cap) {
+      (void)hipFree(w.LOGF);
+      w.LOGF = nullptr;
+      w.logf_cap = 0;
+      HIP_TRY(counted_malloc(&w.LOGF, words * sizeof(float)));
+      w.logf_cap = words;
     }
+    k_untag<<<(uint32_t)((words + 255) / 256), 256, 0, s>>>(w.LOGT, w.LOGF, words);
+    HIP_TRY(hipMemcpyAsync(logits_out, w.LOGF, words * sizeof(float), hipMemcpyDeviceToHost, s));
   }
   std::vector<defer_gpu_cache*> cc;
   std::vector<uint32_t> cli, cpos, ctick;
@@ -2529,7 +2603,22 @@ static int forward_batch_impl(defer_gpu_model* m, defer_gpu_cache* const* caches
       cpos.push_back(rows[b].pos + 1);
       ctick.push_back(rows[b].tick + 1);
     }
-  return batch_commit_many(m, cc.data(), cli.data(), cpos.data(), ctick.data(), (uint32_t)cc.size());
+  rc = queue_commit(m, cc.data(), cli.data(), (uint32_t)cc.size());
+  if (rc) return rc;
+  HIP_TRY(hipStreamSynchronize(s));
+  float ms = 0.0f;
+  HIP_TRY(hipEventElapsedTime(&ms, m->ev0, m->ev1));
+  m->last_ms = ms;
+  if (deferred) {
+    // A wait that ran out leaves the rows undefined: no cache advances.
+    if (w.h_st->abort) {
+      for (uint32_t b = 0; b < n; ++b) caches[b]->has_logits = false;
+      return fail(DEFER_GPU_E_TIMEOUT, "a device-side wait exceeded its bound; cache state is undefined");
+    }
+    memcpy(tok_out, w.h_out, n * sizeof(uint32_t));
+  }
+  commit_host(cc.data(), cpos.data(), ctick.data(), (uint32_t)cc.size());
+  return DEFER_GPU_OK;
 }
 
 extern "C" int defer_gpu_forward_batch(const defer_gpu_model* mc, defer_gpu_cache* const* caches,
@@ -2539,6 +2628,8 @@ extern "C" int defer_gpu_forward_batch(const defer_gpu_model* mc, defer_gpu_cach
   if (n == 0) return DEFER_GPU_OK;
   if (!caches || !tokens) return fail(DEFER_GPU_E_INVALID, "null argument");
   if (n > BATCH_MAX_ROWS) return fail(DEFER_GPU_E_INVALID, "at most %u rows per batch", BATCH_MAX_ROWS);
+  const int rc = up_reset(m);
+  if (rc) return rc;
   return forward_batch_impl(m, caches, tokens, nullptr, nullptr, n, logits_out);
 }
 
@@ -2570,6 +2661,8 @@ extern "C" int defer_gpu_step_batch(const defer_gpu_model* mc, defer_gpu_cache* 
   // sized first, so the forward does not reallocate it under them).
   rc = ensure_ws(m, n, n);
   if (rc) return rc;
+  rc = up_reset(m);
+  if (rc) return rc;
   rc = batch_sample(m, caches, nullptr, tick.data(), rng_words, n, temperature, tokens_out, true,
                     true);
   if (rc) return rc;
@@ -2595,7 +2688,9 @@ static int replay_batched(defer_gpu_model* m, defer_gpu_cache* c, const uint32_t
     std::vector<uint32_t> sel;
     for (uint32_t j = 0; j < k; ++j)
       if (o + j + 1 >= plen) sel.push_back(j);
-    int e = batch_run(m, rows.data(), rc.data(), k, sel.data(), (uint32_t)sel.size());
+    int e = up_reset(m);
+    if (e) return e;
+    e = batch_run(m, rows.data(), rc.data(), k, sel.data(), (uint32_t)sel.size());
     if (e) return e;
     // op i = row + 1 samples logits row `row` (the ops inside the history)
     std::vector<uint32_t> lrow, tk, wd, out;
@@ -2626,8 +2721,6 @@ static int replay_batched(defer_gpu_model* m, defer_gpu_cache* c, const uint32_t
     c->pos = (uint32_t)(o + k);
     c->tick = tick0 + (uint32_t)(o + k);
     c->has_logits = false;
-    e = push_state(c);
-    if (e) return e;
   }
   return DEFER_GPU_OK;
 }
