@@ -1240,35 +1240,40 @@ __global__ __launch_bounds__(256) void k_b_chunkmax(const Dims d, const u64* __r
   }
 }
 
-// Chunks per wave and round of k_b_sample's stage A: the one workgroup of an
+// Chunks per wave and round of k_b_sample's stage A: a lone workgroup of an
 // op walks all the row's chunks, so rounds of NWA chunks would each wait a
 // full memory latency. Its LDS holds NWA * SAMP_CPW chunks past the rows
 // layout's scratch start (samp_lds_bytes).
 constexpr uint32_t SAMP_CPW = 8;
 
-// One sampling op per workgroup (the one-token sampler, stages A and B on
-// one workgroup): op j samples logits row lrow[j] for generation base
-// tick[j] with rng word words[j]; the token goes to out[j].
+// Sampling ops, G workgroups each (the one-token sampler, its stages shared
+// among them as among the persistent kernel's workgroups): op j samples
+// logits row lrow[j] for generation base tick[j] with rng word words[j]; the
+// token goes to out[j]. With G > 1 an op's workgroups wait for each other's
+// words, so all of them must be resident (a cooperative launch). An op on one
+// workgroup is bound by that CU's arithmetic (the exp of every logit) and
+// reads: 7 ops of 49,152 logits took 262 us on one workgroup each, 73 on 36.
 __global__ __launch_bounds__(BLOCK) void k_b_sample(const Args* __restrict__ largs,
                                                     const uint32_t* __restrict__ tick,
                                                     const uint32_t* __restrict__ words, float T,
-                                                    uint32_t tag0, uint32_t* __restrict__ out) {
-  const uint32_t j = blockIdx.x;
+                                                    uint32_t tag0, uint32_t G,
+                                                    uint32_t* __restrict__ out) {
+  const uint32_t j = blockIdx.x / G, wg = blockIdx.x - j * G;
   const Args& a = largs[j];
   const Lds s = lds_init_rows(a.d);
   // A row whose wait runs out still leaves a token in range (0), so a
   // following batched embedding never reads outside the table.
-  if (threadIdx.x == 0) out[j] = 0u;
+  if (wg == 0 && threadIdx.x == 0) out[j] = 0u;
   uint32_t tok = 0;
   if (T != 0.0f) {
     float m;
     uint32_t bi;
-    if (!sample_stage_a<SAMP_CPW, 8>(a, tick[j], tag0 + j, T, 0, 1, s, &m, &bi)) return;
-    if (!sample_exact(a, tag0 + j, m, bi, words[j], 0, 1, true, s, &tok)) return;
+    if (!sample_stage_a<SAMP_CPW, 8>(a, tick[j], tag0 + j, T, wg, G, s, &m, &bi)) return;
+    if (!sample_exact(a, tag0 + j, m, bi, words[j], wg, G, true, s, &tok)) return;
   } else if (!sample_greedy(a, tick[j], s, &tok)) {
     return;
   }
-  if (threadIdx.x == 0) out[j] = tok;
+  if (wg == 0 && threadIdx.x == 0) out[j] = tok;
 }
 
 }  // namespace dg

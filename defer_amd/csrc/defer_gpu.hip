@@ -2435,7 +2435,23 @@ static int batch_sample(defer_gpu_model* m, defer_gpu_cache* const* ocache, cons
   k_begin<<<1, 1, 0, s>>>(w.st);
   const uint32_t tag0 = m->samp_next;
   m->samp_next += nops;
-  k_b_sample<<<nops, BLOCK, samp_lds_bytes(m), s>>>(largs, stick, swords, T, tag0, w.sout);
+  // A few ops at T > 0 spread over the CUs, as far as a workgroup still has
+  // several chunks: they fill the chip together, one workgroup per CU, in a
+  // cooperative launch; where that is refused (another process holds it),
+  // and for more ops, one workgroup each.
+  constexpr uint32_t OWN_CHUNKS = 8;  // chunks per workgroup, at least
+  uint32_t G = T != 0.0f ? std::min(m->ncu / nops, (d.nvc + OWN_CHUNKS - 1) / OWN_CHUNKS) : 1;
+  bool launched = false;
+  if (G > 1) {
+    float Tv = T;
+    uint32_t tag = tag0;
+    void* args[] = {&largs, &stick, &swords, &Tv, &tag, &G, &w.sout};
+    launched = hipLaunchCooperativeKernel((const void*)k_b_sample, dim3(nops * G), dim3(BLOCK), args,
+                                          (unsigned)samp_lds_bytes(m), s) == hipSuccess;
+    if (!launched) (void)hipGetLastError();  // refused at launch: nothing ran
+  }
+  if (!launched)
+    k_b_sample<<<nops, BLOCK, samp_lds_bytes(m), s>>>(largs, stick, swords, T, tag0, 1, w.sout);
   HIP_TRY(hipGetLastError());
   if (deferred) return DEFER_GPU_OK;
   HIP_TRY(hipMemcpyAsync(w.h_out, w.sout, nops * sizeof(uint32_t), hipMemcpyDeviceToHost, s));

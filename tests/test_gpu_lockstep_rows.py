@@ -53,3 +53,24 @@ def test_rows_of_distinct_caches_equal_single_steps(shape):
                         assert np.array_equal(bits(x), bits(y)), (i, l)
         for c in A + B:
             c.close()
+
+
+@pytest.mark.parametrize("rows", [1, 2, 5, 7, 40, 130])
+def test_sampled_steps_equal_single_steps(rows):
+    """A step's sampling ops share the CUs (several workgroups per op for few
+    rows, one for many): the tokens are those of stepping each session alone."""
+    cfg = synthetic._cfg(20000, 64, 96, 1, 2, 1, 32, 10000.0, True, max_seq=64)
+    m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 9, std=0.3))
+    rng = np.random.Generator(np.random.PCG64(rows))
+    A, B = [], []
+    for i in range(rows):
+        a = m.new_cache(16)
+        m.prompt(a, synthetic.make_prompt(20000, 1 + i % 3, seed=i))
+        A.append(a)
+        B.append(a.clone())
+    for T in (0.05, 0.7, 1.0, 0.0, 8.0):
+        print(f"rows={rows} T={T}", flush=True)
+        words = rng.integers(0, 1 << 32, size=rows, dtype=np.uint32)
+        words[0] = [0, 0xFFFFFFFF][rows % 2]
+        got = m.step_batch(A, T, words)
+        assert got == [m.step(b, T, int(w)) for b, w in zip(B, words)], T
