@@ -17,6 +17,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -414,6 +415,10 @@ struct defer_gpu_model {
   uint32_t ncu = 0;  // compute units of the device
   uint32_t gemm_ncu = 0;  // compute units the batched path's GEMM launches are shaped for
   uint32_t n_caches = 0;  // live caches (their argument blocks copy the layout)
+  // Pinned slots the caches' runs leave their state in, a slab at a time (an
+  // allocation of its own took 80 us of each cache's creation).
+  std::vector<DevState*> state_slabs, state_free;
+  std::mutex state_mu;
   size_t lds_bytes = 0;
   hipStream_t stream = nullptr;
   float* wbuf = nullptr;
@@ -530,10 +535,14 @@ static const void* attn_rows_kernel(uint32_t hd, uint32_t teams) {
 #undef DG_ROWS
 }
 // Query heads of a group in one task, at most: as many as leave LDS for two
-// workgroups per CU.
+// workgroups per CU, or for three at head_dim 128 and 128-position chunks (a
+// group of four as two tasks of two: 500 rows of the 8B shape 51.4 -> 40.5 us
+// per layer; at head_dim 64 a group of three as 2 + 1 heads takes 250 against
+// 215 us at 256-position chunks, and single heads 218).
 static uint32_t attn_tile_heads(const Dims& d, uint32_t nb) {
+  const size_t most = LDS_BYTES_MAX / (d.hd == 128 && nb == 1 ? 3 : 2);
   uint32_t nj = d.group;
-  while (nj > 1 && attn_tile_lds(d.hd, nb, nj) > LDS_BYTES_MAX / 2) --nj;
+  while (nj > 1 && attn_tile_lds(d.hd, nb, nj) > most) --nj;
   return nj;
 }
 
@@ -908,6 +917,7 @@ extern "C" void defer_gpu_model_destroy(defer_gpu_model* m) {
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   batch_ws_free(m);
   for (hipEvent_t e : m->pev) (void)hipEventDestroy(e);
+  for (DevState* slab : m->state_slabs) (void)hipHostFree(slab);
   (void)hipFree(m->panels);
   (void)hipFree(m->wbuf);
   (void)hipFree(m->d_layers);
@@ -941,6 +951,21 @@ extern "C" int defer_gpu_model_set_grid(defer_gpu_model* m, uint32_t workgroups,
 
 // ------------------------------------------------------------------ caches
 
+static DevState* state_slot(defer_gpu_model* m) {
+  constexpr size_t SLAB = 64;
+  const std::lock_guard<std::mutex> lock(m->state_mu);
+  if (m->state_free.empty()) {
+    DevState* slab = nullptr;
+    if (counted_host_malloc((void**)&slab, SLAB * sizeof(DevState), hipHostMallocDefault) != hipSuccess)
+      return nullptr;
+    m->state_slabs.push_back(slab);
+    for (size_t i = SLAB; i-- > 0;) m->state_free.push_back(slab + i);
+  }
+  DevState* st = m->state_free.back();
+  m->state_free.pop_back();
+  return st;
+}
+
 static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* c) {
   const Dims& d = m->d;
   c->m = m;
@@ -961,7 +986,8 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   HIP_TRY(hipMemset(c->mb, 0, words * sizeof(u64)));
   HIP_TRY(counted_malloc(&c->st, sizeof(DevState)));
   HIP_TRY(hipMemset(c->st, 0, sizeof(DevState)));
-  HIP_TRY(counted_host_malloc((void**)&c->h_st, sizeof(DevState), hipHostMallocDefault));
+  c->h_st = state_slot(const_cast<defer_gpu_model*>(m));
+  if (!c->h_st) return fail(DEFER_GPU_E_HIP, "pinned state allocation failed");
   HIP_TRY(counted_malloc(&c->d_run, sizeof(RunDesc)));
   HIP_TRY(counted_malloc(&c->d_mask, ((cap + 31) / 32) * sizeof(uint32_t)));
   HIP_TRY(counted_malloc(&c->d_logits, (size_t)d.V * sizeof(float)));
@@ -1018,7 +1044,11 @@ static void cache_free(defer_gpu_cache* c) {
   (void)hipFree(c->d_tmp);
   (void)hipFree(c->d_trace);
   (void)hipFree(c->d_norms);
-  if (c->h_st) (void)hipHostFree(c->h_st);
+  if (c->h_st && c->m) {
+    defer_gpu_model* m = const_cast<defer_gpu_model*>(c->m);
+    const std::lock_guard<std::mutex> lock(m->state_mu);
+    m->state_free.push_back(c->h_st);
+  }
   (void)hipFree(c->d_args);
   if (c->h_ring) (void)hipHostFree(c->h_ring);
 }
@@ -2597,18 +2627,21 @@ static int forward_batch_impl(defer_gpu_model* m, defer_gpu_cache* const* caches
   // The rest is queued behind the batch, with one wait for all of it.
   if (deferred) HIP_TRY(hipMemcpyAsync(w.h_out, dtok, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   if (logits_out) {
-    // Every row has logits, in row order: untagged together and copied at
-    // once.
-    const size_t words = (size_t)n * d.V;
-    if (words > w.logf_cap) {
+    // Every row has logits, in row order: untagged and copied 64 rows at a
+    // time (33 MB at a vocabulary of 128,256).
+    const size_t block = std::min(n, 64u) * (size_t)d.V, words = (size_t)n * d.V;
+    if (block > w.logf_cap) {
       (void)hipFree(w.LOGF);
       w.LOGF = nullptr;
       w.logf_cap = 0;
-      HIP_TRY(counted_malloc(&w.LOGF, words * sizeof(float)));
-      w.logf_cap = words;
+      HIP_TRY(counted_malloc(&w.LOGF, block * sizeof(float)));
+      w.logf_cap = block;
     }
-    k_untag<<<(uint32_t)((words + 255) / 256), 256, 0, s>>>(w.LOGT, w.LOGF, words);
-    HIP_TRY(hipMemcpyAsync(logits_out, w.LOGF, words * sizeof(float), hipMemcpyDeviceToHost, s));
+    for (size_t o = 0; o < words; o += block) {
+      const size_t k = std::min(block, words - o);
+      k_untag<<<(uint32_t)((k + 255) / 256), 256, 0, s>>>(w.LOGT + o, w.LOGF, k);
+      HIP_TRY(hipMemcpyAsync(logits_out + o, w.LOGF, k * sizeof(float), hipMemcpyDeviceToHost, s));
+    }
   }
   std::vector<defer_gpu_cache*> cc;
   std::vector<uint32_t> cli, cpos, ctick;
