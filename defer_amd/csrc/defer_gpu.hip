@@ -968,6 +968,10 @@ static DevState* state_slot(defer_gpu_model* m) {
 
 static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* c) {
   const Dims& d = m->d;
+  // A cache's device memory is written on the model's stream only: that
+  // stream does not wait for the null stream, where clears and copies within
+  // the device can return before they are done.
+  const hipStream_t s = m->stream;
   c->m = m;
   ++const_cast<defer_gpu_model*>(m)->n_caches;
   ++g_live_caches;
@@ -983,9 +987,9 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   const size_t words = base_words + MB_REPS * rep_words;
   c->mb_words = words;
   HIP_TRY(counted_malloc(&c->mb, words * sizeof(u64)));
-  HIP_TRY(hipMemset(c->mb, 0, words * sizeof(u64)));
+  HIP_TRY(hipMemsetAsync(c->mb, 0, words * sizeof(u64), s));
   HIP_TRY(counted_malloc(&c->st, sizeof(DevState)));
-  HIP_TRY(hipMemset(c->st, 0, sizeof(DevState)));
+  HIP_TRY(hipMemsetAsync(c->st, 0, sizeof(DevState), s));
   c->h_st = state_slot(const_cast<defer_gpu_model*>(m));
   if (!c->h_st) return fail(DEFER_GPU_E_HIP, "pinned state allocation failed");
   HIP_TRY(counted_malloc(&c->d_run, sizeof(RunDesc)));
@@ -1020,7 +1024,8 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   a.st = c->st;
   a.mask = nullptr;
   HIP_TRY(counted_malloc(&c->d_args, sizeof(Args)));
-  HIP_TRY(hipMemcpy(c->d_args, &a, sizeof(Args), hipMemcpyHostToDevice));
+  HIP_TRY(hipMemcpyAsync(c->d_args, &a, sizeof(Args), hipMemcpyHostToDevice, s));
+  HIP_TRY(hipStreamSynchronize(s));
   return DEFER_GPU_OK;
 }
 
@@ -1101,11 +1106,17 @@ extern "C" int defer_gpu_cache_clone(const defer_gpu_cache* src, defer_gpu_cache
   }
   const Dims& d = src->m->d;
   const size_t kvn = (size_t)d.L * d.nkv * src->cap * d.kvs;
-  hipError_t e = hipMemcpy(c->kc, src->kc, kvn * sizeof(float), hipMemcpyDeviceToDevice);
-  if (e == hipSuccess) e = hipMemcpy(c->vc, src->vc, kvn * sizeof(float), hipMemcpyDeviceToDevice);
-  if (e == hipSuccess)
-    e = hipMemcpy(c->mb, src->mb, src->mb_words * sizeof(u64), hipMemcpyDeviceToDevice);
-  if (e == hipSuccess) e = hipMemcpy(c->st, src->st, sizeof(DevState), hipMemcpyDeviceToDevice);
+  // On the model's stream (cache_alloc says why), and done on return: the
+  // source may be fed or destroyed next.
+  const hipStream_t s = src->m->stream;
+  auto copy = [&](void* to, const void* from, size_t n) {
+    return hipMemcpyAsync(to, from, n, hipMemcpyDeviceToDevice, s);
+  };
+  hipError_t e = copy(c->kc, src->kc, kvn * sizeof(float));
+  if (e == hipSuccess) e = copy(c->vc, src->vc, kvn * sizeof(float));
+  if (e == hipSuccess) e = copy(c->mb, src->mb, src->mb_words * sizeof(u64));
+  if (e == hipSuccess) e = copy(c->st, src->st, sizeof(DevState));
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     cache_free(c);
     delete c;
