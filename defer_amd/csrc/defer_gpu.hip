@@ -1280,11 +1280,18 @@ static int run_begin(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
   return DEFER_GPU_OK;
 }
 
-// Queues n_ops ops described by `r` (host copy, device pointers filled in)
-// on the model's stream, then the copy of the state they leave; run_finish
-// waits for them. in.no_graph: the phase kernels one by one where the mode is
-// a graph.
-static int run_launch(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
+// A run of n_ops ops that failed with part of it queued: waited for, so that
+// nothing writes the caller's memory after the call, and its generations are
+// not used again (the mailboxes may hold words tagged with them). The cache
+// keeps its length; its logit words may be overwritten.
+static int run_abandon(defer_gpu_cache* c, uint32_t n_ops, int rc) {
+  (void)hipStreamSynchronize(c->m->stream);
+  c->tick += n_ops;
+  c->has_logits = false;
+  return rc;
+}
+
+static int run_queue(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
   defer_gpu_model* m = const_cast<defer_gpu_model*>(c->m);
   const hipStream_t s = m->stream;
   const int rb = run_begin(c, r, in);
@@ -1335,6 +1342,14 @@ static int run_launch(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) 
   HIP_TRY(hipEventRecord(m->ev1, s));
   HIP_TRY(hipMemcpyAsync(c->h_st, c->st, sizeof(DevState), hipMemcpyDeviceToHost, s));
   return DEFER_GPU_OK;
+}
+// Queues n_ops ops described by `r` (host copy, device pointers filled in)
+// on the model's stream, then the copy of the state they leave; run_finish
+// waits for them. in.no_graph: the phase kernels one by one where the mode is
+// a graph.
+static int run_launch(defer_gpu_cache* c, const RunDesc& r, const RunInput& in) {
+  const int rc = run_queue(c, r, in);
+  return rc ? run_abandon(c, r.n_ops, rc) : DEFER_GPU_OK;
 }
 
 static int run_finish(defer_gpu_cache* c) {
@@ -1460,16 +1475,16 @@ extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, u
   rc = feed_launch(c, &token, 1, in, tq);
   if (rc) return rc;
   // The results' copies are queued behind the run: one wait for all.
-  if (trace_out) {
-    k_trace<<<dim3(m->d.nh, m->d.L), 256, 0, s>>>(c->d_args, pos0, tq, c->d_trace);
-    HIP_TRY(hipMemcpyAsync(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
-                           hipMemcpyDeviceToHost, s));
-  }
-  if (logits_out) {
-    rc = queue_logits(c, logits_out);
-    if (rc) return rc;
-  }
-  return run_finish(c);
+  auto results = [&]() -> int {
+    if (trace_out) {
+      k_trace<<<dim3(m->d.nh, m->d.L), 256, 0, s>>>(c->d_args, pos0, tq, c->d_trace);
+      HIP_TRY(hipMemcpyAsync(trace_out, c->d_trace, (size_t)m->d.L * m->d.nh * (pos0 + 1) * sizeof(float),
+                             hipMemcpyDeviceToHost, s));
+    }
+    return logits_out ? queue_logits(c, logits_out) : DEFER_GPU_OK;
+  };
+  rc = results();
+  return rc ? run_abandon(c, 1, rc) : run_finish(c);
 }
 
 static bool use_batch(const defer_gpu_model* m, size_t n);
@@ -2629,31 +2644,14 @@ static int forward_batch_impl(defer_gpu_model* m, defer_gpu_cache* const* caches
       li_of[b] = (uint32_t)sel.size();
       sel.push_back(b);
     }
-  HIP_TRY(hipEventRecord(m->ev0, m->stream));
-  int rc = batch_run(m, rows.data(), caches, n, sel.data(), (uint32_t)sel.size(), dtok, deferred);
-  if (rc) return rc;
-  HIP_TRY(hipEventRecord(m->ev1, m->stream));
-  BatchWs& w = *m->bw;
   const hipStream_t s = m->stream;
-  // The rest is queued behind the batch, with one wait for all of it.
-  if (deferred) HIP_TRY(hipMemcpyAsync(w.h_out, dtok, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-  if (logits_out) {
-    // Every row has logits, in row order: untagged and copied 64 rows at a
-    // time (33 MB at a vocabulary of 128,256).
-    const size_t block = std::min(n, 64u) * (size_t)d.V, words = (size_t)n * d.V;
-    if (block > w.logf_cap) {
-      (void)hipFree(w.LOGF);
-      w.LOGF = nullptr;
-      w.logf_cap = 0;
-      HIP_TRY(counted_malloc(&w.LOGF, block * sizeof(float)));
-      w.logf_cap = block;
-    }
-    for (size_t o = 0; o < words; o += block) {
-      const size_t k = std::min(block, words - o);
-      k_untag<<<(uint32_t)((k + 255) / 256), 256, 0, s>>>(w.LOGT + o, w.LOGF, k);
-      HIP_TRY(hipMemcpyAsync(logits_out + o, w.LOGF, k * sizeof(float), hipMemcpyDeviceToHost, s));
-    }
+  HIP_TRY(hipEventRecord(m->ev0, s));
+  int rc = batch_run(m, rows.data(), caches, n, sel.data(), (uint32_t)sel.size(), dtok, deferred);
+  if (rc) {
+    (void)hipStreamSynchronize(s);
+    return rc;
   }
+  BatchWs& w = *m->bw;
   std::vector<defer_gpu_cache*> cc;
   std::vector<uint32_t> cli, cpos, ctick;
   for (uint32_t b = 0; b < n; ++b)
@@ -2663,12 +2661,45 @@ static int forward_batch_impl(defer_gpu_model* m, defer_gpu_cache* const* caches
       cpos.push_back(rows[b].pos + 1);
       ctick.push_back(rows[b].tick + 1);
     }
-  rc = queue_commit(m, cc.data(), cli.data(), (uint32_t)cc.size());
-  if (rc) return rc;
-  HIP_TRY(hipStreamSynchronize(s));
-  float ms = 0.0f;
-  HIP_TRY(hipEventElapsedTime(&ms, m->ev0, m->ev1));
-  m->last_ms = ms;
+  // The rest is queued behind the batch, with one wait for all of it.
+  bool committing = false;
+  auto results = [&]() -> int {
+    HIP_TRY(hipEventRecord(m->ev1, s));
+    if (deferred) HIP_TRY(hipMemcpyAsync(w.h_out, dtok, n * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+    if (logits_out) {
+      // Every row has logits, in row order: untagged and copied 64 rows at a
+      // time (33 MB at a vocabulary of 128,256).
+      const size_t block = std::min(n, 64u) * (size_t)d.V, words = (size_t)n * d.V;
+      if (block > w.logf_cap) {
+        (void)hipFree(w.LOGF);
+        w.LOGF = nullptr;
+        w.logf_cap = 0;
+        HIP_TRY(counted_malloc(&w.LOGF, block * sizeof(float)));
+        w.logf_cap = block;
+      }
+      for (size_t o = 0; o < words; o += block) {
+        const size_t k = std::min(block, words - o);
+        k_untag<<<(uint32_t)((k + 255) / 256), 256, 0, s>>>(w.LOGT + o, w.LOGF, k);
+        HIP_TRY(hipMemcpyAsync(logits_out + o, w.LOGF, k * sizeof(float), hipMemcpyDeviceToHost, s));
+      }
+    }
+    committing = true;
+    const int qrc = queue_commit(m, cc.data(), cli.data(), (uint32_t)cc.size());
+    if (qrc) return qrc;
+    HIP_TRY(hipStreamSynchronize(s));
+    float ms = 0.0f;
+    HIP_TRY(hipEventElapsedTime(&ms, m->ev0, m->ev1));
+    m->last_ms = ms;
+    return DEFER_GPU_OK;
+  };
+  rc = results();
+  if (rc) {
+    // Nothing writes the caller's memory after the call; the caches keep
+    // their lengths, and their logits unless those may be overwritten.
+    (void)hipStreamSynchronize(s);
+    for (uint32_t b = 0; b < n && committing; ++b) caches[b]->has_logits = false;
+    return rc;
+  }
   if (deferred) {
     // A wait that ran out leaves the rows undefined: no cache advances.
     if (w.h_st->abort) {

@@ -68,6 +68,50 @@ def check_clone(hip, G, m, cfg):
     assert not bad, bad
 
 
+def test_a_failed_call_leaves_nothing_running(fake):
+    """A copy that fails ends the call with an error and the stream idle, so
+    that nothing writes the caller's arrays afterwards; the cache keeps its
+    length, and its logits unless they may be overwritten."""
+    child(fake, "failure")
+
+
+def check_failure(hip, G, m, cfg):
+    # per call the copies it makes on the stream, in order: whether the cache
+    # still has its logits when that copy fails
+    calls = {
+        # the run's state, the probabilities, the logits: the run has written its own
+        "forward": ([False, False, False], lambda a, b: m.forward(1, a, trace=True)),
+        # the rows, the run's state, the logits, the list of caches to commit
+        "forward_batch": ([True, True, True, False], lambda a, b: m.forward_batch([a, b], [1, 2], logits=True)),
+    }
+    bad = []
+    for name, (keeps, call) in calls.items():
+        for k, keep in enumerate(keeps):
+            a, b = m.new_cache(64), m.new_cache(64)
+            for c in (a, b):
+                m.prompt(c, list(range(20)))
+            hip.fake_fail_in(k + 1)
+            try:
+                call(a, b)
+                bad.append((name, k, "no error"))
+            except G.DeferGpuError:
+                pass
+            hip.fake_fail_in(0)
+            if hip.fake_pending():
+                bad.append((name, k, "still running"))
+            assert len(a) == 20
+            try:
+                a.last_logits()
+                kept = True
+            except G.DeferGpuError:
+                kept = False
+            if kept != keep:
+                bad.append((name, k, "logits kept" if kept else "logits lost"))
+            a.close()
+            b.close()
+    assert not bad, bad
+
+
 if __name__ == "__main__":
     hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # found before the real runtime
     hip.fake_unordered.restype = ctypes.c_long
@@ -76,5 +120,5 @@ if __name__ == "__main__":
 
     cfg = synthetic.CONFIGS["tiny"]
     model = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 1))
-    {"clone": check_clone}[sys.argv[2]](hip, G, model, cfg)
+    {"clone": check_clone, "failure": check_failure}[sys.argv[2]](hip, G, model, cfg)
     print("ok")
