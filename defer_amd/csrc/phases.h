@@ -1272,9 +1272,12 @@ __device__ __forceinline__ bool phase_o(const Args& a, uint32_t l, uint32_t tick
                         ? gather_vec(rep_of(a, a.mb_xd, wg) + own_item(d, IK_O, wg, G, 0), R, gen_of(d, tick, l - 1, PH_D), xres)
                         : no_gather();
   // Layer 0's residual is the embedding row: its words are loaded before the
-  // wait (pollers, one word per thread).
+  // wait, one per thread; a workgroup with more rows than threads (a small
+  // grid) loads the rest after it.
+  constexpr uint32_t RT = NWA * WAVE;  // the loaders issue no loads of this kind
+  auto emb_word = [&](uint32_t k) { return ldg(a.embed + (size_t)token * d.h + own_item(d, IK_O, wg, G, k)); };
   float emb = 0.0f;
-  if (l == 0 && threadIdx.x < R) emb = ldg(a.embed + (size_t)token * d.h + own_item(d, IK_O, wg, G, threadIdx.x));
+  if (l == 0 && threadIdx.x < min(R, RT)) emb = emb_word(threadIdx.x);
   Preload P;
   const Pub pub = pub_for(sg.on, s);
   // The QKV rows are used: the next layer's are requested -- after the
@@ -1288,7 +1291,11 @@ __device__ __forceinline__ bool phase_o(const Args& a, uint32_t l, uint32_t tick
     if (!(STAGED_ONLY || sg.on) && m0.n == NCW && wave >= NWA) prefetch_first(a, IK_O, l, wg, G, s, wave - NWA, lane);
   }
   if (!poll_gather<4, 1>(ga, gr, NWA, a.st, s.ctl, mv_hook(sg, op, P, IK_O))) return false;
-  if (l == 0 && threadIdx.x < R) lds_st(xres + threadIdx.x, emb);
+  if (l == 0 && threadIdx.x < min(R, RT)) {
+    lds_st(xres + threadIdx.x, emb);
+    if (!STAGED_ONLY)  // its rows fit the LDS, so they are few
+      for (uint32_t k = threadIdx.x + RT; k < R; k += RT) lds_st(xres + k, emb_word(k));
+  }
   if (inl && R > 0)
     for (uint32_t u = threadIdx.x; u < d.q && threadIdx.x < NWA * WAVE; u += NWA * WAVE) {
       const uint32_t hh = u / d.hd, dd = u - hh * d.hd;
