@@ -813,7 +813,10 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
 //    the tree over its PV groups and the sum w = 0..3 in order, from +0.
 // Positions past a query's own (t > pos) carry probability +0, and V rows
 // past the tile's last position are zeros: both leave an accumulator
-// unchanged (a chain started at +0 never holds -0).
+// unchanged (a chain started at +0 never holds -0) as long as the V row is
+// finite, 0 * inf being NaN. So a wave looks at its rows of the tile's own
+// positions, and where one holds an infinity or a NaN it forms its sums
+// again, each query's over the positions it sees alone.
 //
 // K and V rows go from memory (L2: the tiles of a chunk run on one XCD)
 // straight into the registers of the one wave that uses them -- wave w takes
@@ -976,6 +979,23 @@ __global__ __launch_bounds__(256, 2) void k_b_attn_tile(const Dims d, const BRow
   if constexpr (HOLD)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) load_v(nb, vf[nb]);
+  // The wave's V rows at positions that the tile's first query does not see
+  // (t > its own): x * 0 is NaN for an infinity or a NaN, +-0 else. The tile's
+  // positions lie in one 16-aligned block, four of them the wave's: one per lc.
+  const uint32_t p_own = r0.pos - t0;  // past the chunk in all but the tile's last chunk
+  float unseen = 0.0f;
+  if (p_own < CH) {
+    const uint32_t p = p_own / 16 * 16 + PV * wave + lc % PV + GV * (lc / PV);
+    if (p > p_own && p < nk) {
+      const float* r = vb + (size_t)(t0 + p) * HD + 4 * lr;
+#pragma unroll
+      for (int hh = 0; hh < HH; ++hh) {
+        const float4 x = ldg4(r + 64 * hh);
+        unseen += (x.x * 0.0f + x.y * 0.0f) + (x.z * 0.0f + x.w * 0.0f);
+      }
+    }
+  }
+  const bool odd = __any(unseen != unseen);
   __syncthreads();
   // 3. Softmax statistics and probabilities, 16 lanes per (query, head):
   // lane sub holds phase_attn's lane slots L = sub + 16v (v = 0..3); the
@@ -1060,6 +1080,24 @@ __global__ __launch_bounds__(256, 2) void k_b_attn_tile(const Dims d, const BRow
       for (int rr = 0; rr < 4; ++rr)  // query 4*lc + rr, dims 64*hh + 4*lr ..
         *reinterpret_cast<float4*>(Wx + (size_t)(wave * 16 + 4 * lc + rr) * HD + 64 * hh + 4 * lr) =
             make_float4(w[0][rr], w[1][rr], w[2][rr], w[3][rr]);
+    }
+    if (odd) {  // wave-uniform
+#pragma unroll 1
+      for (uint32_t q = 0; q < nq; ++q)
+#pragma unroll 1
+        for (uint32_t dd = lane; dd < HD; dd += WAVE) {
+          float g4[PV];
+#pragma unroll
+          for (int pl = 0; pl < PV; ++pl) {
+            g4[pl] = 0.0f;
+#pragma unroll 1
+            for (uint32_t p = PV * wave + pl; p < nk && p <= p_own + q; p += GV)
+              g4[pl] = fmaf(Ss[(j * 16 + q) * SP + p], vb[(size_t)(t0 + p) * HD + dd], g4[pl]);
+          }
+          float A = g4[0] + g4[1];
+          if constexpr (PV == 4) A = A + (g4[2] + g4[3]);
+          Wx[(size_t)(wave * 16 + q) * HD + dd] = A;
+        }
     }
     __syncthreads();
     const uint32_t hidx = g * d.group + j0 + j;

@@ -46,3 +46,49 @@ def test_windows_equal_token_by_token(shape):
         c.truncate(start + n - 1)
         assert np.array_equal(bits(got), bits(m.forward(int(toks[start + n - 1]), c))), (start, n)
         c.close()
+
+
+# first position, rows, the row with the odd token: in the first and in later
+# tiles, in the tile's first, last and middle row, in chunks of 128 to 512
+ODD = [(0, 40, 7), (0, 16, 15), (120, 30, 8), (120, 30, 16), (1000, 20, 2), (2040, 40, 12), (4090, 40, 10), (6150, 20, 9)]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
+@pytest.mark.parametrize("value", ["nan", "inf"])
+def test_rows_before_an_infinite_or_nan_value_row_are_untouched(shape, value):
+    """A token whose value row holds NaNs, or one infinity beside finite keys:
+    the rows before it in its tile do not see it. Every row's logits must be
+    those of feeding the tokens one at a time (NaN where those are NaN)."""
+    nh, nkv, hd = shape
+    V, h, odd = 200, 128, 199
+    cfg = synthetic._cfg(V, h, 128, 2, nh, nkv, hd, 10000.0, False, max_seq=8192)
+    w = synthetic.make_weights(cfg, 3, std=0.15)
+    embed, wv = w[0], w[4]  # layer 0: norm, q, k, v
+    if value == "nan":
+        embed[odd, 3] = np.nan
+    else:  # element 5 of the hidden row is this token's alone, and reaches one value of each head
+        embed[:, 5] = 0.0
+        embed[odd, 5] = 10.0
+        for t in w[2:4]:
+            t[:, 5] = 0.0
+        wv[:, 5] = 0.0
+        wv[hd - 3::hd, 5] = 3e38
+    m = G.GpuModel(G.Config.from_dict(cfg), w)
+    toks = synthetic.make_prompt(odd, 8192, seed=nh)
+    ref = m.new_cache(8192)
+    m.prompt(ref, toks[:6200])
+    for start, n, at in ODD:
+        print(f"{shape} {value} positions {start}..{start + n - 1}, odd row {at}", flush=True)
+        feed = toks[start:start + n].copy()
+        feed[at] = odd
+        a, b = ref.clone(), ref.clone()
+        a.truncate(start)
+        b.truncate(start)
+        got = m.forward_batch([a] * n, feed, logits=True)
+        for i, t in enumerate(feed):
+            want = m.forward(int(t), b)
+            assert np.all(np.isfinite(want)) == (i < at), (start, i)
+            same = (bits(got[i]) == bits(want)) | (np.isnan(got[i]) & np.isnan(want))
+            assert np.all(same), (start, i)
+        a.close()
+        b.close()
