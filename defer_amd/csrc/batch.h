@@ -562,6 +562,10 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
   phase_attn<true, 0, NCW, 1, 4>(a, l, r.tick, r.pos, x, 0x10000u, s);
 }
 
+// Chunk partials between launches: [row][nh][MAX_ACHUNKS][hd + 4] floats, acc
+// first, then m and l (16-byte aligned rows).
+__host__ __device__ constexpr uint32_t at_part_row(uint32_t hd) { return hd + 4; }
+
 // Attention of rows with distinct caches (a lockstep step), QKV epilogue and
 // chunk combine included: one workgroup per (row, kv head), of TEAMS teams of
 // NCW waves. The first waves form 1/rms of the row and the group's q/k/v from
@@ -578,6 +582,12 @@ __global__ __launch_bounds__(NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 // last of a group (an agent-scope count) polling the others' partials, took
 // 13.7 us per layer for 7 rows of the 135M shape at 150 positions (11.8 now,
 // with the rows' 1/rms inside) and 30 us for 64 of the 1B shape at 256 (27.4).
+// Few rows with long histories leave most CUs idle that way (two rows of the
+// 135M shape at 4,000 positions: 6 workgroups of 16 chunks each). Then a
+// group's chunks are dealt to `splits` workgroups, each with the q/k/v of its
+// own, and the partials go to part_g for k_b_comb to merge (the same values,
+// the same order). A step of two 135M sessions at 4,000 positions takes 1.41 ms
+// so, 2.76 with a workgroup each, at 1,000 positions 1.20 and 1.53.
 // HD: the head size, or 0 to read it from d.
 struct AttnRowsLds {
   uint32_t ml, sc, wp, part, sw, total;  // float offsets: after q, k and v
@@ -593,20 +603,23 @@ __host__ __device__ inline AttnRowsLds attn_rows_lds(uint32_t hd, uint32_t grp, 
   o.total = o.sw + grp * nch + MAX_GROUP;
   return o;
 }
-template <uint32_t HD, uint32_t TEAMS>
+template <uint32_t HD, uint32_t TEAMS, bool SPLIT>
 __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_b_attn_f(
     const Args* __restrict__ ap, const BRow* __restrict__ rows, uint32_t l,
     const float* __restrict__ X, const float* __restrict__ Y, uint32_t ldy, uint32_t max_nch,
-    uint32_t max_ch, float* __restrict__ attp) {
+    uint32_t max_ch, float* __restrict__ attp, uint32_t n_splits, float* __restrict__ part_g) {
   extern __shared__ float lds_raw[];
   // K rows of KU score passes and V rows of VE value steps are requested a
   // chunk ahead, V rows up to VU steps once the scores have freed K's registers.
   constexpr uint32_t KU = HD ? 2 : 1, VE = 4, VU = HD == 64 ? 8 : HD ? 6 : 4, NW = TEAMS * NCW;
   const Args& a = *ap;  // by reference: as kernel arguments its fields took registers (spills, 32 against 27 us at 1B)
   const Dims& d = a.d;
-  const uint32_t b = blockIdx.x / d.nkv, g = blockIdx.x - b * d.nkv;
+  const uint32_t splits = SPLIT ? n_splits : 1, groups = gridDim.x / splits;
+  const uint32_t sp = SPLIT ? blockIdx.x / groups : 0, bg = blockIdx.x - sp * groups;
+  const uint32_t b = bg / d.nkv, g = bg - b * d.nkv;
   const BRow r = rows[b];
   const uint32_t pos = r.pos, nch = attn_nchunks(pos), CH = attn_chunk(pos);
+  if (SPLIT && sp * TEAMS >= nch) return;  // a shorter row: no chunk of its own
   const uint32_t hd = HD ? HD : d.hd, half = hd / 2, grp = d.group, hs = hd + 2;
   const AttnRowsLds o = attn_rows_lds(hd, grp, TEAMS, max_ch, max_nch);
   const uint32_t wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -643,7 +656,7 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
 #pragma unroll
     for (uint32_t u = 0; u < VE; ++u) vr[u] = load_v(min(t0 + vw + u * vstep, t_last));
   };
-  prefetch(team);
+  prefetch(sp * TEAMS + team);
   // q, k and v of the group: one thread per pair of rotated elements.
   const uint32_t pairs = (grp + 2) * half;
   if (wave * WAVE < pairs) {
@@ -657,13 +670,12 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
       float* dst = qs + j * hd;  // k and v follow the queries
       lds_st(dst + i, v.x);
       lds_st(dst + i + half, v.y);
-      if (j >= grp) qkv_epi_cache(d, r, l, hb, i, v);
+      if (j >= grp && sp == 0) qkv_epi_cache(d, r, l, hb, i, v);
     }
   }
   __syncthreads();
-  const uint32_t rounds = (nch + TEAMS - 1) / TEAMS;
-  for (uint32_t rd = 0; rd < rounds; ++rd) {
-    const uint32_t c = rd * TEAMS + team, t0 = c * CH;
+  for (uint32_t c0 = sp * TEAMS; c0 < nch; c0 += TEAMS * splits) {
+    const uint32_t c = c0 + team, t0 = c * CH;
     const uint32_t t1 = c < nch ? min(t0 + CH, pos + 1) : t0;  // an idle team only meets the barriers
     // scores, KU passes per round
     for (uint32_t pb0 = t0; pb0 < t1; pb0 += KU * sstep) {
@@ -741,7 +753,7 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
         }
       }
     }
-    prefetch(c + TEAMS);
+    prefetch(c + TEAMS * splits);
     for (uint32_t x = ge.lv; x < WAVE; x <<= 1) {
 #pragma unroll
       for (uint32_t j = 0; j < MAX_GROUP; ++j) {
@@ -770,6 +782,15 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
         float A = 0.0f;
 #pragma unroll
         for (uint32_t w = 0; w < NCW; ++w) A += lds_ld(wp + (w * grp + j) * hd + dd);
+        if (SPLIT) {  // the tiled attention's layout of the partials
+          float* out = part_g + (((size_t)b * d.nh + g * grp + j) * MAX_ACHUNKS + c) * at_part_row(hd);
+          out[dd] = A;
+          if (dd == 0) {
+            out[hd] = lds_ld(ml + 2 * j);
+            out[hd + 1] = lds_ld(ml + 2 * j + 1);
+          }
+          continue;
+        }
         float* out = part + (j * nch + c) * hs;
         lds_st(out + 2 + dd, A);
         if (dd == 0) {
@@ -778,6 +799,7 @@ __global__ __launch_bounds__(TEAMS * NCW * WAVE) __attribute__((amdgpu_waves_per
         }
       }
   }
+  if (SPLIT) return;
   __syncthreads();
   float* sw = lds_raw + o.sw;         // [grp][nch]
   float* ls = sw + grp * max_nch;     // [grp]
@@ -837,10 +859,6 @@ __host__ __device__ constexpr uint32_t attn_tile_lds(uint32_t hd, uint32_t nb, u
   const uint32_t qo = nj * hd * 16, wx = NCW * 16 * hd;
   return 4 * ((qo > wx ? qo : wx) + nj * 16 * (at_pitch(nb * ACHUNK) + 2));
 }
-// Partials of the tiled path: [row][nh][MAX_ACHUNKS][hd + 4] floats, acc
-// first, then m and l (16-byte aligned rows).
-__host__ __device__ constexpr uint32_t at_part_row(uint32_t hd) { return hd + 4; }
-
 // v[0..3] of lane (lr, lc) = elements 4*lc .. 4*lc+3 of row lr; afterwards
 // v[i] = element 4*i + lc (a 4x4 transpose between components and the wave's
 // four rows of 16 lanes).

@@ -539,10 +539,14 @@ static const void* attn_tile_kernel(uint32_t hd, uint32_t nb) {
   if ((hd != 64 && hd != 128) || nb < 1 || nb > AT_MAX_NB) return nullptr;
   return k[hd == 128][nb - 1];
 }
-// The attention of a lockstep step's rows with `teams` teams per workgroup.
-static const void* attn_rows_kernel(uint32_t hd, uint32_t teams) {
-#define DG_ROWS(HD) \
-  (teams == 4 ? (const void*)k_b_attn_f<HD, 4> : teams == 2 ? (const void*)k_b_attn_f<HD, 2> : (const void*)k_b_attn_f<HD, 1>)
+// The attention of a lockstep step's rows with `teams` teams per workgroup,
+// or (teams = 1) a group's chunks split over several workgroups.
+static const void* attn_rows_kernel(uint32_t hd, uint32_t teams, bool split) {
+#define DG_ROWS(HD)                                   \
+  (split        ? (const void*)k_b_attn_f<HD, 1, true> \
+   : teams == 4 ? (const void*)k_b_attn_f<HD, 4, false> \
+   : teams == 2 ? (const void*)k_b_attn_f<HD, 2, false> \
+                : (const void*)k_b_attn_f<HD, 1, false>)
   return hd == 64 ? DG_ROWS(64) : hd == 128 ? DG_ROWS(128) : DG_ROWS(0);
 #undef DG_ROWS
 }
@@ -712,9 +716,10 @@ static int apply_layout(defer_gpu_model* m, uint32_t G) {
     if (e != hipSuccess)
       return fail(DEFER_GPU_E_HIP, "LDS attribute (%zu bytes): %s", m->lds_attn, hipGetErrorString(e));
   }
-  for (uint32_t teams = 1; teams <= 4; teams *= 2) {
-    const hipError_t e = hipFuncSetAttribute(attn_rows_kernel(d.hd, teams),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES_MAX);
+  for (const void* kf : {attn_rows_kernel(d.hd, 1, false), attn_rows_kernel(d.hd, 2, false),
+                         attn_rows_kernel(d.hd, 4, false), attn_rows_kernel(d.hd, 1, true)}) {
+    const hipError_t e =
+        hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)LDS_BYTES_MAX);
     if (e != hipSuccess)
       return fail(DEFER_GPU_E_HIP, "LDS attribute (rows' attention): %s", hipGetErrorString(e));
   }
@@ -2276,7 +2281,7 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
   // Its teams per workgroup: as many as the longest row has chunks, as long
   // as every workgroup's waves are resident at once (16 per CU), so that a
   // few rows spread over the waves of a CU and many rows over the CUs.
-  uint32_t teams = 1, max_ch = 0, max_nch = 0;
+  uint32_t teams = 1, splits = 1, max_ch = 0, max_nch = 0;
   size_t lds_rows_attn = 0;
   if (fused) {
     for (uint32_t b = 0; b < n; ++b) {
@@ -2287,6 +2292,15 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
     while (teams < 4 && teams < max_nch && n * d.nkv * 2 * teams * NCW <= 16 * m->ncu &&
            lds(2 * teams) <= LDS_BYTES_MAX)
       teams *= 2;
+    // ... or, where its teams take the chunks in more rounds than single
+    // teams spread over the resident waves would, those: a round saved is
+    // 9 us of a layer, the combine's launch about 3 (135M shape, 2 rows).
+    const uint32_t room = 16 * m->ncu / (n * d.nkv * NCW), s1 = std::min(room, max_nch);
+    if (s1 > 1 && (max_nch + s1 - 1) / s1 < (max_nch + teams - 1) / teams) {
+      teams = 1;
+      splits = s1;
+      max_nch = 0;  // no partials in LDS
+    }
     lds_rows_attn = lds(teams);
     fused = lds_rows_attn <= LDS_BYTES_MAX;  // else the chunks as items
   }
@@ -2383,9 +2397,10 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
       ProfSpan ps(m, 1, attn_flop);
       uint32_t li = l, ld = ldy;
       const float *xr = w.X, *yr = w.Y;
-      void* args[] = {&rargs, &drows, &li, &xr, &yr, &ld, &max_nch, &max_ch, &w.XQ};
-      HIP_TRY(hipLaunchKernel(attn_rows_kernel(d.hd, teams), dim3(n * d.nkv), dim3(teams * NCW * WAVE), args,
-                              lds_rows_attn, s));
+      float* pg = reinterpret_cast<float*>(w.PART);
+      void* args[] = {&rargs, &drows, &li, &xr, &yr, &ld, &max_nch, &max_ch, &w.XQ, &splits, &pg};
+      HIP_TRY(hipLaunchKernel(attn_rows_kernel(d.hd, teams, splits > 1), dim3(n * d.nkv * splits), dim3(teams * NCW * WAVE),
+                              args, lds_rows_attn, s));
     } else {
       if (!tiled)
         k_b_qkv_epi<<<dim3((d.qkv_rows / 2 + 255) / 256, n), 256, 0, s>>>(
@@ -2400,12 +2415,12 @@ static int batch_run(defer_gpu_model* m, const BRow* rows, defer_gpu_cache* cons
           k_b_attn_w<<<(uint32_t)items.size(), NCW * WAVE, m->lds_attn, s>>>(rargs, drows, d_items, l);
         }
       }
-      const dim3 comb_grid(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK);
-      if (tiled)
-        k_b_comb<true><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
-      else
-        k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
     }
+    const dim3 comb_grid(n, (d.nh + COMB_HEADS_PER_BLOCK - 1) / COMB_HEADS_PER_BLOCK);
+    if (tiled || (fused && splits > 1))
+      k_b_comb<true><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
+    else if (!fused)
+      k_b_comb<false><<<comb_grid, 256, 0, s>>>(d, drows, w.PART, part_words(d), w.XQ);
     GemmOutArgs x{};  // the residual rows and their panel
     x.Y = w.X;
     x.ldy = d.h;

@@ -55,6 +55,64 @@ def test_rows_of_distinct_caches_equal_single_steps(shape):
             c.close()
 
 
+@pytest.mark.parametrize("shape", SHAPES + [(4, 1, 256, 128, 128)], ids=lambda s: "x".join(map(str, s)))
+def test_few_rows_with_long_histories_equal_single_steps(shape):
+    """Few rows of many chunks: a group's chunks go to several workgroups (as
+    many as the longest row's, fewer for a shorter one), past 8192 positions
+    too; enough rows to fill the CUs without bring one workgroup each back."""
+    nh, nkv, hd, h, ff = shape
+    cfg = synthetic._cfg(200, h, ff, 2, nh, nkv, hd, 10000.0, True, max_seq=10400)
+    m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 8, std=0.12))
+    toks = synthetic.make_prompt(200, 10400, seed=hd)
+    long = m.new_cache(10400)
+    m.prompt(long, toks[:10300])
+    for rows in ([10300, 3], [700, 640], [9000, 0, 10300, 2100, 130], [1000] * 24):
+        print(f"{shape} rows={rows}", flush=True)
+        A, B = [], []
+        for n in rows:
+            for side in (A, B):
+                c = long.clone()
+                c.truncate(n)
+                side.append(c)
+        for step in range(2):
+            feed = toks[step:step + len(rows)]
+            got = m.forward_batch(A, feed, logits=True)
+            for i, (b, t) in enumerate(zip(B, feed)):
+                assert np.array_equal(bits(got[i]), bits(m.forward(int(t), b))), (step, i, rows[i])
+        for x, y in zip(A[0].read(1), B[0].read(1)):
+            assert np.array_equal(bits(x), bits(y))
+        for c in A + B:
+            c.close()
+
+
+def test_few_rows_with_long_histories_use_the_idle_compute_units():
+    """Two rows of 16 chunks: each chunk has CUs of its own, so the attention
+    takes about as long as over one chunk (1.05 times, measured) and not four
+    rounds of it (3.5 times with a workgroup per row and kv head)."""
+    cfg = synthetic._cfg(2000, 576, 1536, 12, 9, 3, 64, 10000.0, True, max_seq=2100)
+    m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 8))
+    toks = synthetic.make_prompt(2000, 2040, seed=1)
+    ms = {}
+    for n in (100, 2030):
+        cs = [m.new_cache(2100), m.new_cache(2100)]
+        for c in cs:
+            m.prompt(c, toks[:n])
+        m.set_profiling(True)
+        best = []
+        for _ in range(8):
+            for c in cs:
+                c.truncate(n)
+            m.batch_stats()
+            m.forward_batch(cs, [1, 2])
+            best.append(m.batch_stats()["attn_ms"])
+        m.set_profiling(False)
+        ms[n] = min(best)
+        for c in cs:
+            c.close()
+    print(ms, ms[2030] / ms[100], flush=True)
+    assert ms[2030] < 2.5 * ms[100], ms
+
+
 @pytest.mark.parametrize("rows", [1, 2, 5, 7, 40, 130])
 def test_sampled_steps_equal_single_steps(rows):
     """A step's sampling ops share the CUs (several workgroups per op for few
