@@ -26,9 +26,10 @@ def bits(a):
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}x{s[2]}")
 def test_windows_equal_token_by_token(shape):
     nh, nkv, hd = shape
-    cfg = synthetic._cfg(64, 128, 128, 2, nh, nkv, hd, 10000.0, False, max_seq=8192)
+    # a vocabulary of four 64-row chunks: the one-token path runs on four workgroups
+    cfg = synthetic._cfg(250, 128, 128, 2, nh, nkv, hd, 10000.0, False, max_seq=8192)
     m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 3, std=0.15))
-    toks = synthetic.make_prompt(64, 8192, seed=nh)
+    toks = synthetic.make_prompt(250, 8192, seed=nh)
     ref = m.new_cache(8192)
     m.set_batching(0)
     m.prompt(ref, toks[:8190])

@@ -55,6 +55,32 @@ def test_traced_and_masked_forwards_equal_the_phase_kernels(shape):
                 assert np.array_equal(x, y), (ctx, mode)
 
 
+@pytest.mark.parametrize("name", ["smollm2-135m", "smollm2-360m", "llama-3.2-1b", "llama-3-8b"])
+def test_traced_and_masked_forwards_at_the_specialised_shapes(name):
+    """The shapes with a persistent kernel of their own, on the whole grid, one
+    chunk and several: as the phase kernels, which are not specialised."""
+    cfg = synthetic.CONFIGS[name]
+    m = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 5, threads=16))
+    toks = synthetic.make_prompt(cfg["vocab_size"], 601, seed=2)
+    c = m.new_cache(610)
+    m.prompt(c, toks[:600])
+    for ctx, mask in ((600, tuple(range(40, 500, 7))), (100, (0, 3, 99))):
+        got = {}
+        for mode in (G.EXEC_PERSISTENT, G.EXEC_EAGER):
+            print(f"{name} ctx={ctx} mode={mode}", flush=True)
+            m.set_exec(mode)
+            out = []
+            for kw in ({"trace": True}, {"trace": True, "masked": mask}, {"masked": mask}):
+                c.truncate(ctx)
+                r = m.forward(int(toks[600]), c, **kw)
+                out += list(r) if isinstance(r, tuple) else [r]
+                out += [x[ctx] for x in c.read(cfg["num_layers"] - 1)]
+            got[mode] = [bits(x) for x in out]
+            assert np.array_equal(got[mode][4], got[mode][8])  # tracing leaves the logits alone
+        for x, y in zip(got[G.EXEC_PERSISTENT], got[G.EXEC_EAGER]):
+            assert np.array_equal(x, y), ctx
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_value_norms_do_not_depend_on_how_many_are_asked_for(shape):
     cfg, m = model(shape)
