@@ -1245,13 +1245,10 @@ __global__ __launch_bounds__(64) void k_b_final(const float* __restrict__ X,
   if (lane == 0) linv[i] = 1.0f / sqrtf(ss / (float)h + eps);
 }
 
-// Chunk (max, argmax) of the tagged logits of each logits row, tagged for
-// the sampler (phase_lm's chunk step; argmax is a total order, so any tree
-// gives its answer). One wave per (chunk, row).
-// Chunk (max, argmax) of every logits row: each wave takes CM_CPW
-// consecutive chunks, one lane per row of a chunk, with all its loads issued
-// before the first reduction (the same reduction per chunk as the lm_head
-// phase's, so the same values).
+// Chunk (max, argmax) of the tagged logits of every logits row, tagged for the
+// sampler: each wave takes CM_CPW consecutive chunks, one lane per row of a
+// chunk, with all its loads issued before the first reduction (phase_lm's
+// reduction; argmax is a total order, so any tree gives its answer).
 constexpr uint32_t CM_CPW = 4;
 __global__ __launch_bounds__(256) void k_b_chunkmax(const Dims d, const u64* __restrict__ logt,
                                                     const uint32_t* __restrict__ gen,

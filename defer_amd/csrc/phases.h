@@ -29,8 +29,6 @@
 // Attention, lm_head and the sampler run on pollers and compute waves.
 #pragma once
 
-#include <type_traits>
-
 #include "device.h"
 #include "exact.h"
 
