@@ -474,15 +474,18 @@ static size_t samp_lds_bytes(const defer_gpu_model* m) {
   return std::max(m->lds_rows, samp_end);
 }
 
-// A persistent kernel compiled for this exact shape, if there is one. The
-// 135M kernel has no streaming path, so it runs only where every kind's rows
-// are staged.
+// A persistent kernel compiled for this exact shape, if there is one and the
+// grid of G workgroups gives none of them more residual rows than threads (the
+// loop over the rest, in every specialised kernel, cost them spilled registers
+// and 0.3 % of the 360M shape's tokens). The 135M kernel has no streaming path,
+// so it runs only where every kind's rows are staged.
 static bool has_shape(const Dims& d, const Dims& f) {
   return d.h == f.h && d.nh == f.nh && d.nkv == f.nkv && d.hd == f.hd && d.ff == f.ff &&
          d.V == f.V && d.L == f.L && d.act == f.act && d.has_bias == f.has_bias && d.tied == f.tied;
 }
 template <bool RANDOM, bool TRACE>
-static const void* persistent_kernel_for(const Dims& d) {
+static const void* persistent_kernel_for(const Dims& d, uint32_t G) {
+  if ((d.h + G - d.o_skip - 1) / (G - d.o_skip) > BLOCK) return (const void*)k_persistent<RANDOM, TRACE>;
   if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_135M)) && d.stg_mask == 0xFu)
     return (const void*)dg135::k_persistent<RANDOM, TRACE>;
   if (has_shape(d, fix_shape(d, DG_SHAPE_ARGS_360M))) return (const void*)dg360::k_persistent<RANDOM, TRACE>;
@@ -686,9 +689,9 @@ static int apply_layout(defer_gpu_model* m, uint32_t G) {
     d.stg_mask = mask;
     d.lds_stg = stg;
   }
-  m->persistent[0] = persistent_kernel_for<false, false>(d);
-  m->persistent[1] = persistent_kernel_for<true, false>(d);
-  m->persistent[2] = persistent_kernel_for<false, true>(d);
+  m->persistent[0] = persistent_kernel_for<false, false>(d, G);
+  m->persistent[1] = persistent_kernel_for<true, false>(d, G);
+  m->persistent[2] = persistent_kernel_for<false, true>(d, G);
   m->lds_bytes = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr + d.lds_stg) * sizeof(float) +
                  (size_t)d.lds_pub * 2 * sizeof(u64) + (d.lds_stg ? 0 : 1024);
   m->lds_rows = (size_t)(4 + 64 + d.lds_vec + d.lds_vec2 + d.lds_scr) * sizeof(float);

@@ -43,6 +43,14 @@ constexpr bool STAGED_ONLY = true;
 constexpr bool STAGED_ONLY = false;
 #endif
 
+// ... nor does one run on a grid so small that a workgroup owns more rows of
+// a phase's output than it has threads.
+#if defined(DG_FIXED_SHAPE)
+constexpr bool SPECIALISED = true;
+#else
+constexpr bool SPECIALISED = false;
+#endif
+
 constexpr uint32_t NPOLL = 2;
 // Words a polling lane owns per round in the per-layer gathers, sized so the
 // specialised shape's vectors (576 and 1536 words) take one round of NWA
@@ -1272,10 +1280,8 @@ __device__ __forceinline__ bool phase_o(const Args& a, uint32_t l, uint32_t tick
   // Layer 0's residual is the embedding row: its words are loaded before the
   // wait, one per thread; a workgroup with more rows than threads (a small
   // grid) loads the rest after it.
-  constexpr uint32_t RT = NWA * WAVE;  // the loaders issue no loads of this kind
-  auto emb_word = [&](uint32_t k) { return ldg(a.embed + (size_t)token * d.h + own_item(d, IK_O, wg, G, k)); };
   float emb = 0.0f;
-  if (l == 0 && threadIdx.x < min(R, RT)) emb = emb_word(threadIdx.x);
+  if (l == 0 && threadIdx.x < R) emb = ldg(a.embed + (size_t)token * d.h + own_item(d, IK_O, wg, G, threadIdx.x));
   Preload P;
   const Pub pub = pub_for(sg.on, s);
   // The QKV rows are used: the next layer's are requested -- after the
@@ -1289,11 +1295,11 @@ __device__ __forceinline__ bool phase_o(const Args& a, uint32_t l, uint32_t tick
     if (!(STAGED_ONLY || sg.on) && m0.n == NCW && wave >= NWA) prefetch_first(a, IK_O, l, wg, G, s, wave - NWA, lane);
   }
   if (!poll_gather<4, 1>(ga, gr, NWA, a.st, s.ctl, mv_hook(sg, op, P, IK_O))) return false;
-  if (l == 0 && threadIdx.x < min(R, RT)) {
-    lds_st(xres + threadIdx.x, emb);
-    if (!STAGED_ONLY)  // its rows fit the LDS, so they are few
-      for (uint32_t k = threadIdx.x + RT; k < R; k += RT) lds_st(xres + k, emb_word(k));
-  }
+  if (l == 0 && threadIdx.x < R) lds_st(xres + threadIdx.x, emb);
+  if (!SPECIALISED && l == 0)
+#pragma unroll 1
+    for (uint32_t k = threadIdx.x + BLOCK; k < R; k += BLOCK)
+      lds_st(xres + k, ldg(a.embed + (size_t)token * d.h + own_item(d, IK_O, wg, G, k)));
   if (inl && R > 0)
     for (uint32_t u = threadIdx.x; u < d.q && threadIdx.x < NWA * WAVE; u += NWA * WAVE) {
       const uint32_t hh = u / d.hd, dd = u - hh * d.hd;
