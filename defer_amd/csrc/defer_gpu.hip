@@ -915,6 +915,9 @@ extern "C" int defer_gpu_model_create(const defer_gpu_config* cfg, const float* 
   }
   if (hipEventCreate(&m->ev0) != hipSuccess || hipEventCreate(&m->ev1) != hipSuccess)
     return cleanup(fail(DEFER_GPU_E_HIP, "event create"));
+  // The uploads went through the null stream, which the model's does not wait for.
+  e = hipStreamSynchronize(nullptr);
+  if (e != hipSuccess) return cleanup(fail(DEFER_GPU_E_HIP, "weight upload: %s", hipGetErrorString(e)));
   *out = m;
   return DEFER_GPU_OK;
 }
@@ -1460,23 +1463,25 @@ extern "C" int defer_gpu_forward(const defer_gpu_model* m, defer_gpu_cache* c, u
   if (token >= m->d.V) return fail(DEFER_GPU_E_TOKEN, "token id %u out of range", token);
   if (c->pos >= c->cap)
     return fail(DEFER_GPU_E_CONTEXT, "context length %u exceeded", m->cfg.max_seq_len);
+  const uint32_t pos0 = c->pos;
+  const hipStream_t s = m->stream;
+  const size_t n_probs = (size_t)m->d.L * m->d.nh * c->cap;
+  rc = ensure_run_buffers(c, 1, 0);
+  if (rc) return rc;
+  if (trace_out && !c->d_trace)
+    HIP_TRY(counted_malloc(&c->d_trace, (n_probs + (size_t)m->d.L * m->d.q) * sizeof(float)));
   bool use_mask = false;
+  std::vector<uint32_t> bits;  // read until the run is waited for
   if (n_masked) {
-    std::vector<uint32_t> bits((c->cap + 31) / 32, 0u);
+    bits.assign((c->cap + 31) / 32, 0u);
     for (size_t i = 0; i < n_masked; ++i)
       if (masked[i] < c->pos) {
         bits[masked[i] >> 5] |= 1u << (masked[i] & 31);
         use_mask = true;
       }
     if (use_mask)
-      HIP_TRY(hipMemcpy(c->d_mask, bits.data(), bits.size() * sizeof(uint32_t),
-                        hipMemcpyHostToDevice));
+      HIP_TRY(hipMemcpyAsync(c->d_mask, bits.data(), bits.size() * sizeof(uint32_t), hipMemcpyHostToDevice, s));
   }
-  const uint32_t pos0 = c->pos;
-  const hipStream_t s = m->stream;
-  const size_t n_probs = (size_t)m->d.L * m->d.nh * c->cap;
-  if (trace_out && !c->d_trace)
-    HIP_TRY(counted_malloc(&c->d_trace, (n_probs + (size_t)m->d.L * m->d.q) * sizeof(float)));
   float* tq = trace_out ? c->d_trace + n_probs : nullptr;
   RunInput in;
   in.mask = use_mask ? c->d_mask : nullptr;
@@ -1580,7 +1585,8 @@ extern "C" int defer_gpu_generate(const defer_gpu_model* m, defer_gpu_cache* c, 
   RunInput in;
   in.words = rng_words;
   in.n_words = temperature != 0.0f ? n : 0;
-  if (n_stop) HIP_TRY(hipMemcpy(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice));
+  if (n_stop)
+    HIP_TRY(hipMemcpyAsync(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream));
   RunDesc r;
   memset(&r, 0, sizeof(r));
   r.n_ops = n;
@@ -1649,7 +1655,8 @@ extern "C" int defer_gpu_generate_cb(const defer_gpu_model* m, defer_gpu_cache* 
   RunInput in;
   in.words = rng_words;
   in.n_words = temperature != 0.0f ? n : 0;
-  if (n_stop) HIP_TRY(hipMemcpy(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice));
+  if (n_stop)
+    HIP_TRY(hipMemcpyAsync(c->d_stop, stop, n_stop * sizeof(uint32_t), hipMemcpyHostToDevice, m->stream));
   const uint32_t pos0 = c->pos;
   RunDesc r;
   memset(&r, 0, sizeof(r));

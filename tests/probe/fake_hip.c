@@ -4,9 +4,9 @@
  * work that nothing has waited for, by HIP's rules for a null stream and
  * streams that do not block on it:
  *
- *  - hipMemcpy within the device and hipMemset go to the null stream and may
- *    return before they are done; hipMemcpy to or from the host waits for the
- *    null stream;
+ *  - hipMemset and hipMemcpy go to the null stream and may return before they
+ *    are done (a copy from pageable memory once that has been read), but for a
+ *    copy to the host, which waits for the null stream;
  *  - anything with a stream argument, and every launch, is queued there;
  *  - synchronising a stream, an event on it or the device waits, and so does
  *    freeing memory.
@@ -48,7 +48,7 @@ hipError_t hipHostGetDevicePointer(void** d, void* h, unsigned f) { (void)f; *d 
 
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind k) {
   queue(NULL);
-  if (k != hipMemcpyDeviceToDevice) pending[0] = 0;
+  if (k == hipMemcpyDeviceToHost) pending[0] = 0;
   memmove(d, s, n);
   return hipSuccess;
 }

@@ -32,10 +32,12 @@ def child(fake, check):
 
 
 def test_a_clone_is_ordered_before_the_next_call(fake):
+    """... and so is what a call itself hands over: a mask, a stop list, a new
+    cache's or model's memory."""
     child(fake, "clone")
 
 
-def check_clone(hip, G, m, cfg):
+def check_clone(hip, G, m, cfg, w):
     c = m.new_cache(64)
     m.prompt(c, list(range(20)))  # batched: the cache's length is the host's
     calls = {
@@ -51,6 +53,7 @@ def check_clone(hip, G, m, cfg):
         "set_logits": lambda x: x.set_logits([0.0] * cfg["vocab_size"]),
         "the source": lambda x: m.forward_batch([c], [1]),
         "a new cache": lambda x: m.forward(1, m.new_cache(8)),
+        "a new model": lambda x: G.GpuModel(m.cfg, w).new_cache(8).clone(),
     }
     bad = []
     for name, call in calls.items():
@@ -75,7 +78,7 @@ def test_a_failed_call_leaves_nothing_running(fake):
     child(fake, "failure")
 
 
-def check_failure(hip, G, m, cfg):
+def check_failure(hip, G, m, cfg, w):
     # per call the copies it makes on the stream, in order: whether the cache
     # still has its logits when that copy fails
     calls = {
@@ -119,6 +122,7 @@ if __name__ == "__main__":
     from defer_amd import synthetic
 
     cfg = synthetic.CONFIGS["tiny"]
-    model = G.GpuModel(G.Config.from_dict(cfg), synthetic.make_weights(cfg, 1))
-    {"clone": check_clone, "failure": check_failure}[sys.argv[2]](hip, G, model, cfg)
+    weights = synthetic.make_weights(cfg, 1)
+    model = G.GpuModel(G.Config.from_dict(cfg), weights)
+    {"clone": check_clone, "failure": check_failure}[sys.argv[2]](hip, G, model, cfg, weights)
     print("ok")
