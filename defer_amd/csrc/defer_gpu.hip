@@ -994,9 +994,11 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
                              5 * (size_t)d.nvc + 64 + 4095) / 4096 * 4096;
   const size_t words = base_words + MB_REPS * rep_words;
   c->mb_words = words;
-  // The mailboxes, and the run state behind them.
+  // The mailboxes, and the run state behind them. A cache's device memory is
+  // written on the model's stream only: that does not wait for the null stream,
+  // where clears and copies can return before they are done.
   HIP_TRY(counted_malloc(&c->mb, words * sizeof(u64) + sizeof(DevState)));
-  HIP_TRY(hipMemset(c->mb, 0, words * sizeof(u64) + sizeof(DevState)));
+  HIP_TRY(hipMemsetAsync(c->mb, 0, words * sizeof(u64) + sizeof(DevState), m->stream));
   c->st = reinterpret_cast<DevState*>(c->mb + words);
   c->h_st = state_slot(const_cast<defer_gpu_model*>(m));
   if (!c->h_st) return fail(DEFER_GPU_E_HIP, "pinned state allocation failed");
@@ -1032,13 +1034,8 @@ static int cache_alloc(const defer_gpu_model* m, uint32_t cap, defer_gpu_cache* 
   a.st = c->st;
   a.mask = nullptr;
   HIP_TRY(counted_malloc(&c->d_args, sizeof(Args)));
-  HIP_TRY(hipMemcpy(c->d_args, &a, sizeof(Args), hipMemcpyHostToDevice));
-  // The clear went to the null stream, which the model's does not wait for: it
-  // is done before the cache is handed out. From here on a cache's device
-  // memory is written on the model's stream only. (Creation and a first
-  // forward of the 135M shape take 551 us so, 563 with the clear and the copy
-  // queued on that stream, 568 with one kernel there.)
-  HIP_TRY(hipStreamSynchronize(nullptr));
+  // Not waited for: c->args stays as it is while the cache lives.
+  HIP_TRY(hipMemcpyAsync(c->d_args, &a, sizeof(Args), hipMemcpyHostToDevice, m->stream));
   return DEFER_GPU_OK;
 }
 
@@ -1118,8 +1115,7 @@ extern "C" int defer_gpu_cache_clone(const defer_gpu_cache* src, defer_gpu_cache
   }
   const Dims& d = src->m->d;
   const size_t kvn = (size_t)d.L * d.nkv * src->cap * d.kvs;
-  // On the model's stream (the null stream's copies within the device can
-  // return before they are done, in no order with it), and done on return: the
+  // On the model's stream (cache_alloc says why), and done on return: the
   // source may be fed or destroyed next.
   const hipStream_t s = src->m->stream;
   auto copy = [&](void* to, const void* from, size_t n) {
