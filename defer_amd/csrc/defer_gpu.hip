@@ -2130,8 +2130,10 @@ static void launch_gemm_tile(hipStream_t s, const float* Wp, uint32_t M, uint32_
 // 4x2, 93, 86 and 76 for 3072 x 576 by 2048 rows). E.g. 576 x 1536: 2048
 // rows 44.2 us at 4x2 (2.25 tasks per CU), 38.4 at 2x2; 301 rows 15.0, 10.0,
 // and 9.2 at 1x1. Every output is computed the same way in every shape.
-// A K that ends inside a chunk takes the smallest tasks; pair products need
-// two row tiles.
+// A K that ends inside a chunk takes the smallest tasks: only those are built
+// with the remainder, which no model shape here has (hidden 1000, a prompt of
+// 2048 tokens through 6 layers: 4.1 ms, 5.4 with the operands shared through
+// LDS in tasks of four tiles). Pair products need two row tiles.
 template <uint32_t OUT>
 static void launch_gemm(hipStream_t s, uint32_t ncu, const float* Wp, uint32_t M, uint32_t K,
                         const float* Xp, uint32_t B, const GemmOutArgs& out) {
